@@ -22,10 +22,14 @@ SOURCES = ["ohpic_particles.hip", "ohpic_particles_mixed.hip", "ohpic_fields.hip
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("OHPIC_ARCH", "gfx950")
 
-# -packed-fp32-ops keeps the compiler from emitting packed FP32 VALU ops.
+# -packed-fp32-ops keeps the compiler from emitting packed FP32 VALU ops.  The
+# atomic optimizer is off: it turns one lane's LDS counter add into a wave-wide
+# reduction that waits for its result at once, while the particle kernels need
+# it only after the charge deposit (they combine lanes themselves).
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17", "-Wall",
     "-Wno-unused-result", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-atomic-optimizer-strategy=None",
     "-I" + os.path.join(ROOT, "include"),
 ]
 

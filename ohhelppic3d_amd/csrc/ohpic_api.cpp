@@ -119,6 +119,9 @@ struct ohpic_ctx {
     WorkItem *d_items = nullptr;
     int nitems = 0;
     int nitems_alloc = 0;
+    CloseItem *d_close = nullptr;  // split tiles (capacity ntiles)
+    int nclose = 0;
+    int slots = 1;               // workgroups of the fused particle kernel resident at once
     int64_t *d_tmp64 = nullptr;  // [ntiles] scratch for repack / store
     int32_t *d_tmp32a = nullptr; // [ntiles]
     int32_t *d_tmp32b = nullptr; // [ntiles]
@@ -251,6 +254,49 @@ int64_t max_work_items(const ohpic_config &c, int64_t ntiles, int num_cus)
     return ntiles + (int64_t)num_cus * 8;
 }
 
+// One tile of one instance as plan_chunks sees it.
+struct TileLoad {
+    int inst, tile;
+    int64_t load;  // bin slots over all species
+};
+
+// A chunk costs about as much as 2K particles (its E tile, charge block and
+// closing), so none is made smaller than this many slots.
+constexpr int64_t kMinChunkLoad = 4096;
+
+// Chunks per tile (nch[i] of tiles[i]) and the order the tiles are dispatched
+// in, for `slots` workgroups resident at once: heaviest first (in steps of an
+// eighth of an octave, tiles of one step in grid order), each tile whole while
+// a share of the work still to come, R / slots, is no smaller than it, else
+// split into that many shares.  A grid with fewer tiles than workgroups is
+// thereby spread over the device, a tile far above the mean (a density hump)
+// does not outlast the others, and the last tiles of a launch end together.
+// At most max_extra items beyond one per tile.  Every further item costs its
+// E tile and charge flush: a group of 32 members of 16^3-64^3, each split as
+// if it ran alone (62936 items), took 3.01 ms per particle launch, planned as
+// one (8008 items) 1.47 ms.
+void plan_chunks(std::vector<TileLoad> &tiles, int64_t slots, int64_t max_extra,
+                 std::vector<int> &nch)
+{
+    auto level = [](int64_t l) { return l <= 0 ? -1 : (int)std::floor(8.0 * std::log2((double)l)); };
+    std::stable_sort(tiles.begin(), tiles.end(), [&](const TileLoad &a, const TileLoad &b) {
+        return level(a.load) > level(b.load);
+    });
+    int64_t rest = 0, made = 0, extra = 0;
+    for (const TileLoad &t : tiles) rest += t.load;
+    nch.assign(tiles.size(), 1);
+    int64_t share = rest / slots;
+    for (size_t i = 0; i < tiles.size(); ++i) {
+        // the first `slots` items start together; later ones as earlier ones end
+        if (made >= slots) share = rest / slots;
+        const int64_t want = tiles[i].load / std::max(share, kMinChunkLoad);
+        nch[i] = (int)std::max<int64_t>(1, std::min<int64_t>({want, 1 + max_extra - extra, 256}));
+        extra += nch[i] - 1;
+        made += nch[i];
+        rest -= tiles[i].load;
+    }
+}
+
 // Device bytes ohpic_create allocates for c (plus the lazily allocated
 // per-cell count buffer), allocation by allocation.
 int64_t estimate_bytes(const ohpic_config &c, int num_cus)
@@ -272,7 +318,9 @@ int64_t estimate_bytes(const ohpic_config &c, int num_cus)
     b += kDiagSlots * 8 + kFlagWords * 8 + kTightListCap * 8 + (int64_t)sizeof(InstDev) + 2 * 4 +
          (int64_t)sizeof(FftJob);
     b += (int64_t)(c.nx + c.ny + c.nz) * (16 + 8);  // twiddles, Green's-function tables
-    b += max_work_items(c, nt, num_cus) * ((int64_t)sizeof(WorkItem) + kKeSlots * 8);
+    b += max_work_items(c, nt, num_cus) *
+         ((int64_t)sizeof(WorkItem) + kKeSlots * 8 + kMaxSpecies * (int64_t)sizeof(int32_t));
+    b += nt * (int64_t)sizeof(CloseItem);
     return b;
 }
 
@@ -328,41 +376,45 @@ void timers_collect(ohpic_ctx *ctx)
     }
 }
 
+// Appends the tiles of an instance with their loads.
+void tile_loads(const ohpic_ctx *ctx, int inst, std::vector<TileLoad> &out)
+{
+    for (int t = 0; t < ctx->ntiles; ++t) {
+        int64_t l = 0;
+        for (int s = 0; s < ctx->cfg.nspecies; ++s)
+            if (!ctx->sp[s].cap.empty()) l += ctx->sp[s].cap[t];
+        out.push_back({inst, t, l});
+    }
+}
+
+// The work items of the planned tiles in dispatch order, and the list of split
+// tiles.  Slots count per instance (next_slot), chunks of a tile in a row.
+void emit_items(const std::vector<TileLoad> &tiles, const std::vector<int> &nch,
+                std::vector<int> &next_slot, std::vector<WorkItem> &items,
+                std::vector<CloseItem> &close)
+{
+    for (size_t i = 0; i < tiles.size(); ++i) {
+        const TileLoad &t = tiles[i];
+        int &slot = next_slot[t.inst];
+        if (nch[i] > 1) close.push_back(CloseItem{t.inst, t.tile, nch[i], slot});
+        for (int c = 0; c < nch[i]; ++c)
+            items.push_back(WorkItem{t.inst, t.tile, (int16_t)c, (int16_t)nch[i], slot++});
+    }
+}
+
 int build_work_items(ohpic_ctx *ctx)
 {
-    const int nt = ctx->ntiles;
-    std::vector<int64_t> load(nt, 0);
-    int64_t maxcap = 0;
-    for (int s = 0; s < ctx->cfg.nspecies; ++s)
-        for (int t = 0; t < nt; ++t) {
-            load[t] += ctx->sp[s].cap.empty() ? 0 : ctx->sp[s].cap[t];
-            if (!ctx->sp[s].cap.empty()) maxcap = std::max<int64_t>(maxcap, ctx->sp[s].cap[t]);
-        }
-    int nch = ctx->cfg.chunks;
-    if (nch <= 0) {
-        const int64_t target = (int64_t)ctx->num_cus * 8;
-        nch = (int)std::max<int64_t>(1, (target + nt - 1) / nt);
-        // keep at least ~512 particles per chunk of the fullest bin
-        const int64_t lim = std::max<int64_t>(1, maxcap / 512);
-        nch = (int)std::min<int64_t>(nch, lim);
-    }
-    std::vector<int> order(nt);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int b) { return load[a] > load[b]; });
+    std::vector<TileLoad> tiles;
+    std::vector<int> nch, next_slot(1, 0);
+    tile_loads(ctx, 0, tiles);
+    plan_chunks(tiles, ctx->slots, ctx->cfg.chunks > 0 ? 0 : (int64_t)ctx->num_cus * 8, nch);
+    if (ctx->cfg.chunks > 0) nch.assign(tiles.size(), ctx->cfg.chunks);
     std::vector<WorkItem> items;
-    items.reserve((size_t)nt * nch);
-    for (int c = 0; c < nch; ++c)
-        for (int i = 0; i < nt; ++i)
-            items.push_back(WorkItem{0, order[i], (int16_t)c, (int16_t)nch, 0});
-    // heavy tiles first within each chunk round: interleave so the first
-    // dispatched items are the heaviest chunks
-    std::stable_sort(items.begin(), items.end(), [&](const WorkItem &a, const WorkItem &b) {
-        return load[a.tile] > load[b.tile];
-    });
-    for (size_t i = 0; i < items.size(); ++i) items[i].slot = (int32_t)i;
+    std::vector<CloseItem> close;
+    emit_items(tiles, nch, next_slot, items, close);
     if ((int)items.size() > ctx->nitems_alloc) {
-        for (void *old : {(void *)ctx->d_items, (void *)ctx->h.ke_partial}) {
+        for (void *old : {(void *)ctx->d_items, (void *)ctx->h.ke_partial,
+                          (void *)ctx->h.chunk_front}) {
             if (!old) continue;
             HIPCHK(ctx, hipStreamSynchronize(ctx->st));
             (void)hipFree(old);
@@ -373,9 +425,13 @@ int build_work_items(ohpic_ctx *ctx)
         }
         ctx->d_items = nullptr;
         ctx->h.ke_partial = nullptr;
+        ctx->h.chunk_front = nullptr;
+        ctx->nitems_alloc = 0;
         int rc = dalloc(ctx, &ctx->d_items, (int64_t)items.size());
         if (rc) return rc;
         rc = dalloc(ctx, &ctx->h.ke_partial, (int64_t)items.size() * kKeSlots);
+        if (rc) return rc;
+        rc = dalloc(ctx, &ctx->h.chunk_front, (int64_t)items.size() * kMaxSpecies);
         if (rc) return rc;
         HIPCHK(ctx, launch_fill_f64(ctx->h.ke_partial, (int64_t)items.size() * kKeSlots, 0.0,
                                     ctx->st));
@@ -383,11 +439,27 @@ int build_work_items(ohpic_ctx *ctx)
     }
     ctx->nitems = (int)items.size();
     ctx->h.nitems = ctx->nitems;
+    ctx->nclose = (int)close.size();
     HIPCHK(ctx, hipMemcpyAsync(ctx->d_items, items.data(), items.size() * sizeof(WorkItem),
                                hipMemcpyHostToDevice, ctx->st));
+    if (!close.empty())
+        HIPCHK(ctx, hipMemcpyAsync(ctx->d_close, close.data(), close.size() * sizeof(CloseItem),
+                                   hipMemcpyHostToDevice, ctx->st));
     ctx->items = std::move(items);
     ctx->items_ver += 1;
     return sync_upload_inst(ctx);
+}
+
+// The particle kernel over this context's work items.
+hipError_t run_particles(ohpic_ctx *ctx, int mode)
+{
+    hipError_t e = launch_particles(mode, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
+                                    ctx->cfg.track_ids != 0, ctx->d_inst, ctx->d_items,
+                                    ctx->nitems, parity_of(ctx), ctx->st);
+    if (e == hipSuccess && (mode == kModeFused || mode == kModeBoundary))
+        e = launch_close_chunks(ctx->cfg.precision, ctx->d_inst, ctx->d_close, ctx->nclose,
+                                ctx->cfg.nspecies, parity_of(ctx), ctx->st);
+    return e;
 }
 
 // Assign capacities/bases from per-bin counts and upload them.
@@ -512,13 +584,6 @@ int bins_to_staging(ohpic_ctx *ctx, int s, int64_t *nlisted)
                                         ctx->d_tmp64, ctx->st));
     HIPCHK(ctx, hipStreamSynchronize(ctx->st));
     *nlisted = tot;
-    return OHPIC_OK;
-}
-
-int zero_next_counts(ohpic_ctx *ctx)
-{
-    for (int s = 0; s < ctx->cfg.nspecies; ++s)
-        HIPCHK(ctx, launch_fill_u64(ctx->h.sp[s].count[ctx->par ^ 1], ctx->ntiles, 0ull, ctx->st));
     return OHPIC_OK;
 }
 
@@ -686,9 +751,8 @@ int rerun_as_list(ohpic_ctx *ctx, int list_mode)
     timer_begin(ctx, 3);
     int rc;
     HIPCHK(ctx, launch_prepare_next_b(ctx->d_inst, parity_of(ctx), 1, ctx->ng, ctx->ntiles,
-                                      nullptr, ctx->st));
-    HIPCHK(ctx, launch_particles(list_mode, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
-                                 ctx->d_inst, ctx->d_items, ctx->nitems, parity_of(ctx), ctx->st));
+                                      ctx->st));
+    HIPCHK(ctx, run_particles(ctx, list_mode));
     if (list_mode == kModeFusedList) HIPCHK(ctx, launch_reduce_ke_b(ctx->d_inst, 1, ctx->st));
     if ((rc = read_flags(ctx))) return rc;
     if (ctx->h_flags[kFlagRange])
@@ -722,8 +786,7 @@ int do_deposit(ohpic_ctx *ctx)
 {
     timer_begin(ctx, 2);
     HIPCHK(ctx, launch_fill_u64(ctx->h.rho_acc[ctx->par], ctx->ng, 0ull, ctx->st));
-    HIPCHK(ctx, launch_particles(kModeDeposit, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
-                                 ctx->d_inst, ctx->d_items, ctx->nitems, parity_of(ctx), ctx->st));
+    HIPCHK(ctx, run_particles(ctx, kModeDeposit));
     timer_end(ctx, 2);
     ctx->rho_valid = true;
     return OHPIC_OK;
@@ -780,8 +843,7 @@ int one_step(ohpic_ctx *ctx)
                                     nullptr, ctx->st));
     if ((rc = do_solve(ctx, false))) return rc;
     timer_begin(ctx, 0);
-    HIPCHK(ctx, launch_particles(kModeFused, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
-                                 ctx->d_inst, ctx->d_items, ctx->nitems, parity_of(ctx), ctx->st));
+    HIPCHK(ctx, run_particles(ctx, kModeFused));
     timer_end(ctx, 0);
     // the parity word is only read here (no out: no flip)
     HIPCHK(ctx, launch_end_step_b(ctx->d_inst, ctx->d_par01 + ctx->par, 1, nullptr, ctx->st));
@@ -971,6 +1033,10 @@ struct ohpic_group {
     WorkItem *d_items = nullptr;
     int64_t cap_items = 0;
     int nitems = 0;
+    CloseItem *d_close = nullptr;      // split tiles
+    int64_t cap_close = 0;
+    int nclose = 0, max_ns = 0;
+    bool ids = false;                  // some member keeps particle ids
     bool dirty = true;
     int64_t max_ng = 0;
     int max_ntiles = 0, max_rows = 0;  // max_rows: largest E-kernel block count
@@ -1035,7 +1101,7 @@ void gfree(T *&p)
     p = nullptr;
 }
 
-int group_reserve(ohpic_group *g, int ninst, int64_t nitems)
+int group_reserve(ohpic_group *g, int ninst, int64_t nitems, int64_t nclose)
 {
     if (ninst > g->cap_insts) {
         const int cap = std::max(ninst, std::max(16, 2 * g->cap_insts));
@@ -1065,7 +1131,45 @@ int group_reserve(ohpic_group *g, int ninst, int64_t nitems)
         GHIP(g, hipMalloc((void **)&g->d_items, cap * sizeof(WorkItem)));
         g->cap_items = cap;
     }
+    if (nclose > g->cap_close) {
+        const int64_t cap = std::max<int64_t>(nclose, std::max<int64_t>(1024, 2 * g->cap_close));
+        GHIP(g, hipStreamSynchronize(g->st));
+        drop_graph(g);
+        gfree(g->d_close);
+        g->cap_close = 0;
+        GHIP(g, hipMalloc((void **)&g->d_close, cap * sizeof(CloseItem)));
+        g->cap_close = cap;
+    }
     return OHPIC_OK;
+}
+
+// The group's work items: the tiles of every member planned together (a tile
+// whole unless the group as a whole is short of work), so that a member's
+// share of the device is not split as if it ran alone.  A member with a given
+// chunk count, or whose planned items would not fit the rows it holds, keeps
+// its own split.  rows[i]: items of member i.
+void group_items(ohpic_group *g, std::vector<WorkItem> &items, std::vector<CloseItem> &close,
+                 std::vector<int> &rows)
+{
+    const int n = (int)g->members.size();
+    std::vector<TileLoad> tiles;
+    for (int i = 0; i < n; ++i) tile_loads(g->members[i], i, tiles);
+    std::vector<int> nch;
+    plan_chunks(tiles, std::max(g->queue_blocks, 1), (int64_t)std::max(g->queue_blocks, 1) * 4, nch);
+    rows.assign(n, 0);
+    for (size_t k = 0; k < tiles.size(); ++k) rows[tiles[k].inst] += nch[k];
+    std::vector<std::vector<int>> own(n);  // a member's own chunks per tile
+    for (int i = 0; i < n; ++i) {
+        const ohpic_ctx *m = g->members[i];
+        if (m->cfg.chunks <= 0 && rows[i] <= m->nitems_alloc) continue;
+        own[i].assign(m->ntiles, 1);
+        for (const WorkItem &w : m->items) own[i][w.tile] = w.nchunks;
+    }
+    for (size_t k = 0; k < tiles.size(); ++k)
+        if (!own[tiles[k].inst].empty()) nch[k] = own[tiles[k].inst][tiles[k].tile];
+    std::vector<int> next(n, 0);
+    emit_items(tiles, nch, next, items, close);
+    rows = next;
 }
 
 // Rebuild the device tables when membership or a member's record / work list
@@ -1078,15 +1182,24 @@ int group_refresh(ohpic_group *g)
         tables = g->members[i]->inst_ver != g->seen_inst[i] ||
                  g->members[i]->items_ver != g->seen_items[i];
     if (tables) {
-        int64_t total = 0;
-        for (ohpic_ctx *m : g->members) total += m->nitems;
-        if (total > INT32_MAX) return gfail(g, OHPIC_EINVAL, "more than 2^31 work items");
-        int rc = group_reserve(g, n, total);
-        if (rc) return rc;
+        g->ids = false;
+        g->max_ns = 0;
+        for (ohpic_ctx *m : g->members) {
+            g->ids = g->ids || m->cfg.track_ids != 0;
+            g->max_ns = std::max(g->max_ns, m->cfg.nspecies);
+        }
+        if (n > 0)
+            g->queue_blocks =
+                particles_queue_blocks(g->precision, g->weight_order, g->T, g->ids, g->device);
         std::vector<InstDev> insts(n);
         std::vector<FftJob> jobs(n);
         std::vector<WorkItem> items;
-        items.reserve((size_t)total);
+        std::vector<CloseItem> close;
+        std::vector<int> rows;
+        group_items(g, items, close, rows);
+        if (items.size() > (size_t)INT32_MAX) return gfail(g, OHPIC_EINVAL, "more than 2^31 work items");
+        int rc = group_reserve(g, n, (int64_t)items.size(), (int64_t)close.size());
+        if (rc) return rc;
         g->max_ng = 0;
         g->max_ntiles = g->max_rows = 0;
         int n256 = 0;
@@ -1097,11 +1210,8 @@ int group_refresh(ohpic_group *g)
         for (int i = 0; i < n; ++i) {
             ohpic_ctx *m = g->members[i];
             insts[i] = m->h;
+            insts[i].nitems = rows[i];
             jobs[i] = m->job;
-            for (WorkItem w : m->items) {
-                w.inst = i;
-                items.push_back(w);
-            }
             g->max_ng = std::max(g->max_ng, m->ng);
             g->max_ntiles = std::max(g->max_ntiles, m->ntiles);
             g->max_rows = std::max(g->max_rows, efield_blocks_of(m->n[0], m->n[1], m->n[2]));
@@ -1114,21 +1224,8 @@ int group_refresh(ohpic_group *g)
             g->seen_items[i] = m->items_ver;
         }
         g->z256 = n256 == 0 ? kZ256None : (n256 == n ? kZ256All : kZ256Some);
-        // heavy items first over the whole table: the dispatcher then fills
-        // the machine with the largest chunks of every instance
-        std::stable_sort(items.begin(), items.end(), [&](const WorkItem &a, const WorkItem &b) {
-            auto load = [&](const WorkItem &w) {
-                const ohpic_ctx *m = g->members[w.inst];
-                int64_t l = 0;
-                for (int s = 0; s < m->cfg.nspecies; ++s)
-                    if (!m->sp[s].cap.empty()) l += m->sp[s].cap[w.tile];
-                return l / w.nchunks;
-            };
-            return load(a) > load(b);
-        });
         g->nitems = (int)items.size();
-        if (n > 0 && g->queue_blocks == 0)
-            g->queue_blocks = particles_queue_blocks(g->precision, g->weight_order, g->T, g->device);
+        g->nclose = (int)close.size();
         if (n > 0) {
             GHIP(g, hipMemcpyAsync(g->d_insts, insts.data(), n * sizeof(InstDev),
                                    hipMemcpyHostToDevice, g->st));
@@ -1137,6 +1234,9 @@ int group_refresh(ohpic_group *g)
         }
         if (!items.empty())
             GHIP(g, hipMemcpyAsync(g->d_items, items.data(), items.size() * sizeof(WorkItem),
+                                   hipMemcpyHostToDevice, g->st));
+        if (!close.empty())
+            GHIP(g, hipMemcpyAsync(g->d_close, close.data(), close.size() * sizeof(CloseItem),
                                    hipMemcpyHostToDevice, g->st));
         GHIP(g, hipStreamSynchronize(g->st));
         drop_graph(g);
@@ -1172,13 +1272,16 @@ hipError_t group_enqueue(ohpic_group *g, int k)
                              g->st);
         if (e == hipSuccess) {
             if (g->persistent)
-                e = launch_particles_queue(g->precision, g->weight_order, g->T, g->d_insts,
+                e = launch_particles_queue(g->precision, g->weight_order, g->T, g->ids, g->d_insts,
                                            g->d_items, g->nitems, g->d_parity, g->d_queue,
                                            g->queue_blocks, g->st);
             else
-                e = launch_particles(kModeFused, g->precision, g->weight_order, g->T, g->d_insts,
-                                     g->d_items, g->nitems, g->d_parity, g->st);
+                e = launch_particles(kModeFused, g->precision, g->weight_order, g->T, g->ids,
+                                     g->d_insts, g->d_items, g->nitems, g->d_parity, g->st);
         }
+        if (e == hipSuccess)
+            e = launch_close_chunks(g->precision, g->d_insts, g->d_close, g->nclose, g->max_ns,
+                                    g->d_parity, g->st);
         if (e == hipSuccess)
             e = launch_end_step_b(g->d_insts, g->d_parity, n,
                                   g->d_flags + (size_t)s * n * kFlagSlots, g->st);
@@ -1593,6 +1696,9 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
                              hipHostMallocDefault));
     CREATE_HIP(hipHostMalloc((void **)&ctx->h_diag, kDiagSlots * sizeof(double),
                              hipHostMallocDefault));
+    CREATE_CHK(dalloc(ctx, &ctx->d_close, nt));
+    ctx->slots = particles_queue_blocks(c.precision, c.weight_order, ctx->T, c.track_ids != 0,
+                                        ctx->device);
     CREATE_CHK(sync_upload_inst(ctx));
     CREATE_CHK(build_work_items(ctx));
     CREATE_HIP(hipStreamSynchronize(ctx->st));
@@ -1938,9 +2044,7 @@ int ohpic_gather_push(ohpic_ctx *ctx)
     if (!ctx->binned)
         return fail(ctx, OHPIC_ESTATE, "gather_push needs binned particles: call boundary");
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    HIPCHK(ctx, launch_particles(kModeGatherPush, ctx->cfg.precision, ctx->cfg.weight_order,
-                                 ctx->T, ctx->d_inst, ctx->d_items, ctx->nitems, parity_of(ctx),
-                                 ctx->st));
+    HIPCHK(ctx, run_particles(ctx, kModeGatherPush));
     HIPCHK(ctx, launch_reduce_ke_b(ctx->d_inst, 1, ctx->st));
     HIPCHK(ctx, hipStreamSynchronize(ctx->st));
     ctx->binned = false;
@@ -1953,12 +2057,10 @@ int ohpic_boundary(ohpic_ctx *ctx)
     GateShared gate;
     if (!ctx) return fail(nullptr, OHPIC_EINVAL, "ctx is NULL");
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    int rc = zero_next_counts(ctx);
+    HIPCHK(ctx, launch_reserve_next_b(ctx->d_inst, parity_of(ctx), 1, ctx->ntiles, ctx->st));
+    HIPCHK(ctx, run_particles(ctx, kModeBoundary));
+    int rc = read_flags(ctx);
     if (rc) return rc;
-    if ((rc = clear_flags(ctx))) return rc;
-    HIPCHK(ctx, launch_particles(kModeBoundary, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
-                                 ctx->d_inst, ctx->d_items, ctx->nitems, parity_of(ctx), ctx->st));
-    if ((rc = read_flags(ctx))) return rc;
     timers_collect(ctx);
     rc = absorb_flags(ctx, ctx->h_flags);
     if (rc < 0) return rc;
@@ -2410,6 +2512,7 @@ int ohpic_group_destroy(ohpic_group *g)
     gfree(g->d_parity);
     gfree(g->d_flags);
     gfree(g->d_items);
+    gfree(g->d_close);
     gfree(g->d_queue);
     if (g->h_flags) (void)hipHostFree(g->h_flags);
     (void)hipStreamDestroy(g->st);
@@ -2440,7 +2543,6 @@ int ohpic_group_attach(ohpic_group *g, ohpic_ctx *ctx)
         g->precision = ctx->cfg.precision;
         g->weight_order = ctx->cfg.weight_order;
         for (int a = 0; a < 3; ++a) g->T[a] = ctx->T[a];
-        g->queue_blocks = 0;
     }
     GHIP(g, hipSetDevice(g->device));
     GHIP(g, hipStreamSynchronize(ctx->st));

@@ -248,11 +248,8 @@ __global__ void k_rho_from_acc_b(const InstDev *__restrict__ insts, const int *_
         rho[i] = (double)(long long)acc[i] * scale;
 }
 
-__global__ void k_prepare_next_b(const InstDev *__restrict__ insts, const int *__restrict__ parity,
-                                 unsigned int *__restrict__ queue)
+__global__ void k_prepare_next_b(const InstDev *__restrict__ insts, const int *__restrict__ parity)
 {
-    // work counter of the queued particle launch that follows
-    if (queue && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *queue = 0u;
     const InstDev *I = insts + blockIdx.y;
     const int nb = parity[blockIdx.y] ^ 1;
     const int64_t n = (int64_t)I->n[0] * I->n[1] * I->n[2];
@@ -267,9 +264,33 @@ __global__ void k_prepare_next_b(const InstDev *__restrict__ insts, const int *_
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
-// Start of a step: rho := the current charge grid * 2^-charge_bits, and the
-// zeroing of k_prepare_next_b (next charge grid and bin words, flags, queue
-// counter) in the same sweep.
+// Reserves each bin's whole current count as the front run of the next buffer:
+// the stayers always fit, and arrivals from neighbours are placed behind them
+// from the start.  (Done here, a tile's workgroup starts without waiting for a
+// reservation of its own, and a tile may be split among several workgroups.)
+__device__ __forceinline__ void reserve_next(const InstDev *I, int par, int64_t t0, int64_t stride)
+{
+    for (int s = 0; s < I->nspecies; ++s) {
+        const SpecDev &S = I->sp[s];
+        for (int64_t t = t0; t < I->ntiles; t += stride) {
+            const unsigned long long c = S.count[par][t];
+            const int cap = S.bin_cap[t], F = min(bin_front(c), cap);
+            S.count[par ^ 1][t] = (unsigned long long)(F + min(bin_back(c), cap - F));
+        }
+    }
+}
+
+__global__ void k_reserve_next_b(const InstDev *__restrict__ insts, const int *__restrict__ parity)
+{
+    const InstDev *I = insts + blockIdx.y;
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    reserve_next(I, parity[blockIdx.y], t0, (int64_t)gridDim.x * blockDim.x);
+    if (t0 < kFlagWords) I->flags[t0] = 0ull;
+}
+
+// Start of a step: rho := the current charge grid * 2^-charge_bits, the next
+// charge grid, the flags and the queue counter zeroed and the next bin words
+// reserved, in the same sweep.
 __global__ void k_begin_step_b(const InstDev *__restrict__ insts, const int *__restrict__ parity,
                                unsigned int *__restrict__ queue)
 {
@@ -287,10 +308,7 @@ __global__ void k_begin_step_b(const InstDev *__restrict__ insts, const int *__r
         rho[i] = (double)(long long)acc[i] * scale;
         next[i] = 0ull;
     }
-    for (int s = 0; s < I->nspecies; ++s) {
-        unsigned long long *__restrict__ w = I->sp[s].count[par ^ 1];
-        for (int64_t t = t0; t < I->ntiles; t += stride) w[t] = 0ull;
-    }
+    reserve_next(I, par, t0, stride);
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
@@ -507,13 +525,21 @@ hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst,
 }
 
 hipError_t launch_prepare_next_b(const InstDev *insts, const int *parity, int ninst,
-                                 int64_t max_ng, int max_ntiles, unsigned int *queue,
-                                 hipStream_t st)
+                                 int64_t max_ng, int max_ntiles, hipStream_t st)
 {
     if (ninst <= 0) return hipSuccess;
     const int64_t n = max_ng > max_ntiles ? max_ng : max_ntiles;
     hipLaunchKernelGGL(k_prepare_next_b, dim3(grid_blocks(n, ninst), ninst), dim3(256), 0, st,
-                       insts, parity, queue);
+                       insts, parity);
+    return hipGetLastError();
+}
+
+hipError_t launch_reserve_next_b(const InstDev *insts, const int *parity, int ninst,
+                                 int max_ntiles, hipStream_t st)
+{
+    if (ninst <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_reserve_next_b, dim3(grid_blocks(max_ntiles, ninst), ninst), dim3(256), 0,
+                       st, insts, parity);
     return hipGetLastError();
 }
 

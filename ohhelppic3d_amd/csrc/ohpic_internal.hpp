@@ -97,6 +97,7 @@ struct InstDev {
     double *ke_partial;           // [kKeSlots][nitems], each row reduced by one block
     double *e_partial;            // [kEfieldMaxBlocks][3] field-energy partial sums
     int nitems;                   // work items of this instance (row length of ke_partial)
+    int32_t *chunk_front;         // [nitems][kMaxSpecies] front-run counts of split tiles' chunks
     unsigned long long *flags;    // kFlagSlots
 };
 
@@ -106,6 +107,11 @@ struct WorkItem {
     int16_t chunk;     // this item's slice of every bin of the tile
     int16_t nchunks;   // slices per bin
     int32_t slot;      // row of the per-item partial-sum table
+};
+// A tile split into several work items (slots slot0 ... slot0 + nchunks - 1):
+// k_close_chunks joins their parts of the new front run.
+struct CloseItem {
+    int32_t inst, tile, nchunks, slot0;
 };
 // largest chunks per tile a configuration may ask for (WorkItem::nchunks)
 constexpr int kMaxChunks = 32767;

@@ -31,9 +31,15 @@ struct Pcg32Dev {
 bool tile_supported(int tx, int ty, int tz);
 
 // parity[item.inst] selects the current buffer of each item's instance.
-hipError_t launch_particles(int mode, int precision, int weight_order, const int T[3],
+// ids: some instance keeps particle ids.
+hipError_t launch_particles(int mode, int precision, int weight_order, const int T[3], bool ids,
                             const InstDev *insts, const WorkItem *items, int nitems,
                             const int *parity, hipStream_t st);
+// After a fused or boundary launch with split tiles: joins the chunks' parts
+// of each listed tile's new front runs (ns: species of the instance that has
+// most).
+hipError_t launch_close_chunks(int precision, const InstDev *insts, const CloseItem *list, int n,
+                               int ns, const int *parity, hipStream_t st);
 // Bin a contiguous list [0, n) of buffer lbuf into the front runs of buffer
 // lbuf^1 (count first, then scatter once capacities are set); wrap != 0
 // applies the periodic wrap twice to each position first.
@@ -54,22 +60,23 @@ hipError_t launch_cell_counts(const InstDev *insts, int inst, int s, int par, in
 
 // The fused step as one resident grid of `blocks` workgroups that claim the
 // nitems work items in list order from *queue (which must be 0 at launch:
-// launch_prepare_next_b zeroes it).  particles_queue_blocks: workgroups of that kernel
+// launch_begin_step_b zeroes it).  particles_queue_blocks: workgroups of that kernel
 // resident on the whole device.
-hipError_t launch_particles_queue(int precision, int weight_order, const int T[3],
+hipError_t launch_particles_queue(int precision, int weight_order, const int T[3], bool ids,
                                   const InstDev *insts, const WorkItem *items, int nitems,
                                   const int *parity, unsigned int *queue, int blocks,
                                   hipStream_t st);
-int particles_queue_blocks(int precision, int weight_order, const int T[3], int device);
+int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int device);
 
 // mixed-precision particles (ohpic_particles_mixed.hip)
-hipError_t launch_particles_mixed(int mode, int weight_order, const int T[3],
+hipError_t launch_particles_mixed(int mode, int weight_order, const int T[3], bool ids,
                                   const InstDev *insts, const WorkItem *items, int nitems,
                                   const int *parity, hipStream_t st);
-hipError_t launch_particles_mixed_queue(int weight_order, const int T[3], const InstDev *insts,
-                                        const WorkItem *items, int nitems, const int *parity,
-                                        unsigned int *queue, int blocks, hipStream_t st);
-int particles_mixed_queue_blocks(int weight_order, const int T[3]);
+hipError_t launch_particles_mixed_queue(int weight_order, const int T[3], bool ids,
+                                        const InstDev *insts, const WorkItem *items, int nitems,
+                                        const int *parity, unsigned int *queue, int blocks,
+                                        hipStream_t st);
+int particles_mixed_queue_blocks(int weight_order, const int T[3], bool ids);
 hipError_t launch_bin_count_mx(const InstDev *insts, int inst, int s, int lbuf, int64_t n,
                                const int T[3], hipStream_t st);
 hipError_t launch_bin_scatter_mx(const InstDev *insts, int inst, int s, int lbuf, int64_t n,
@@ -96,8 +103,9 @@ hipError_t launch_rho_from_acc_b(const InstDev *insts, const int *parity, int ni
 // max_blocks: the largest efield_blocks_of() over the instances
 hipError_t launch_efield_b(const InstDev *insts, int ninst, int max_blocks, bool reduce,
                            hipStream_t st);
-// rho from the current charge grid and the zeroing of launch_prepare_next_b,
-// in one launch at the start of a step
+// rho from the current charge grid, the next charge grid, flags and queue
+// counter zeroed, and the next bin words reserved (launch_reserve_next_b), in
+// one launch at the start of a step
 hipError_t launch_begin_step_b(const InstDev *insts, const int *parity, int ninst,
                                int64_t max_ng, int max_ntiles, unsigned int *queue,
                                hipStream_t st);
@@ -107,11 +115,13 @@ hipError_t launch_begin_step_b(const InstDev *insts, const int *parity, int nins
 // overflowed a bin, in one launch at the end of a step
 hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst,
                              unsigned long long *out, hipStream_t st);
-// zero the next buffer's bin words and charge grid, the flags, and *queue
-// (if not null: the counter of a following launch_particles_queue)
+// zero the next buffer's bin words and charge grid and the flags (list mode)
 hipError_t launch_prepare_next_b(const InstDev *insts, const int *parity, int ninst,
-                                 int64_t max_ng, int max_ntiles, unsigned int *queue,
-                                 hipStream_t st);
+                                 int64_t max_ng, int max_ntiles, hipStream_t st);
+// next bin words := each bin's whole current count as front run (what the
+// particle kernels' stayers fill; arrivals go behind it), flags := 0
+hipError_t launch_reserve_next_b(const InstDev *insts, const int *parity, int ninst,
+                                 int max_ntiles, hipStream_t st);
 // diag[kDiagKeOld..] := sums of ke_partial over the instance's items
 hipError_t launch_reduce_ke_b(const InstDev *insts, int ninst, hipStream_t st);
 

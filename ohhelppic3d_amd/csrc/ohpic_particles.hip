@@ -11,11 +11,21 @@
 //   nodes plus halo (linear_scatter.f90:22-55), and
 //   re-bins it (the replacement of OhHelp's correct_particle/transbound):
 //   a particle that stays in its tile goes to the front run of the tile's
-//   bin in the other buffer (slot from an LDS counter), a particle that left
-//   goes through a per-wave LDS buffer to the back run of its new tile's bin
-//   (batched 64-bit atomics on the bin's front|back word).
+//   bin in the other buffer (64-slot blocks, ohpic_particle_common.hpp), a
+//   particle that left goes through a per-wave LDS buffer to the back run of
+//   its new tile's bin (batched 64-bit atomics on the bin's front|back word).
 // The LDS charge block is flushed with one global 64-bit atomic per node.
 // Integer accumulation makes rho independent of particle order and timing.
+//
+// What bounds it: large grids stream 96 B per particle, at 4.7 TB/s of the 5.2
+// TB/s a bare copy of the same shape reaches; the rest is per tile (E tile,
+// charge flush, the leavers' atomics).  Small grids wait: so every load of an
+// item's start is issued before the first is used, nothing in the particle
+// loop waits for a store, a block's number or the stash, and a species ends
+// with one barrier.  Against slots from an LDS counter at any alignment, a
+// store wait per iteration and the wrap and tile index of every particle:
+// 256^3 x 16 ppc 12.16 -> 11.14 ms, 96^3 x 32 1.35 -> 1.19 ms, 32^3 x 16 51 ->
+// 40 us per launch (HIP events, one box).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -103,50 +113,81 @@ __device__ __forceinline__ void store_bin64(const BinView64 &bv, uint32_t slot, 
     if (ids) gstore(const_cast<int64_t *>(bv.id), (int64_t)slot, q.id);
 }
 
+// The particle's loads have completed from here on.
+__device__ __forceinline__ void arrived(P64 &q, bool ids)
+{
+    asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.vx), "+v"(q.vy), "+v"(q.vz));
+    if (ids) asm volatile("" : "+v"(q.id));
+}
+
 // Append one particle to the back run of bin t (slot from the packed word).
 __device__ __forceinline__ void route_back(const SpecDev &S, int nbuf, int t, const P64 &q,
                                            bool ids, unsigned long long *flags)
 {
+    const int cap = gload(S.bin_cap, t);
+    const int64_t base = gload(S.bin_base, t);
     const unsigned long long old = gatomic_add(&S.count[nbuf][t], 1ull << 32);
     const int f = bin_front(old), b = bin_back(old);
-    const int cap = gload(S.bin_cap, t);
     if (b + f < cap)
-        store_p64(S, nbuf, gload(S.bin_base, t) + (cap - 1 - b), q, ids);
+        store_p64(S, nbuf, base + (cap - 1 - b), q, ids);
     else
         gatomic_add(&flags[kFlagOverflow], 1ull);
 }
 
-struct LeaveBuf {
-    double c[6][kLeaveCap];
-    int64_t id[kLeaveCap];
-    int32_t dest[kLeaveCap];
+template <bool IDS, int CAP>
+struct Buf64 {
+    double c[6][CAP];
+    int64_t id[IDS ? CAP : 1];
+
+    __device__ __forceinline__ void put(int i, const P64 &q, bool ids)
+    {
+        c[0][i] = q.x;
+        c[1][i] = q.y;
+        c[2][i] = q.z;
+        c[3][i] = q.vx;
+        c[4][i] = q.vy;
+        c[5][i] = q.vz;
+        if (IDS && ids) id[i] = q.id;
+    }
+    __device__ __forceinline__ void get(int i, P64 &q, bool ids) const
+    {
+        q.x = c[0][i];
+        q.y = c[1][i];
+        q.z = c[2][i];
+        q.vx = c[3][i];
+        q.vy = c[4][i];
+        q.vz = c[5][i];
+        if (IDS && ids) q.id = id[i];
+    }
 };
 
-// Route the first `cnt` buffered leavers of this wave (lane l takes entry l).
-__device__ __forceinline__ void flush_leavers(LeaveBuf &lb, int cnt, const SpecDev &S, int nbuf,
-                                              bool ids, unsigned long long *flags)
+// The tile of a particle inside the box.
+template <int TX, int TY, int TZ>
+__device__ __forceinline__ int tile_of(const P64 &q, int ntx, int nty)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return (int)q.x / TX + ntx * ((int)q.y / TY + nty * ((int)q.z / TZ));
+}
+
+// Routes the first `cnt` buffered leavers of this wavefront (lane l takes
+// entry l) to the back runs of their new tiles.
+template <int TX, int TY, int TZ, bool IDS>
+__device__ __forceinline__ void flush_leavers(const Buf64<IDS, kLeaveCap> &lb, int cnt,
+                                              const InstDev *__restrict__ I, const SpecDev &S,
+                                              int nbuf, bool ids)
+{
+    wave_sync();
     const int l = lane_id();
     if (l < cnt) {
         P64 q;
-        q.x = lb.c[0][l];
-        q.y = lb.c[1][l];
-        q.z = lb.c[2][l];
-        q.vx = lb.c[3][l];
-        q.vy = lb.c[4][l];
-        q.vz = lb.c[5][l];
-        q.id = lb.id[l];
-        route_back(S, nbuf, lb.dest[l], q, ids, flags);
+        lb.get(l, q, ids);
+        route_back(S, nbuf, tile_of<TX, TY, TZ>(q, I->nt[0], I->nt[1]), q, IDS && ids, I->flags);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
 }
 
-template <int TX, int TY, int TZ, int WO, int MODE_>
+// IDS: instances may keep particle ids (each instance's track_ids says whether
+// it does); without it no register, LDS or branch is spent on them.
+template <int TX, int TY, int TZ, int WO, int MODE_, bool IDS>
 __global__ void __launch_bounds__(kBlock)
     __attribute__((amdgpu_waves_per_eu(OHPIC_PUSH_MIN_WAVES, 8)))
     k_particles_fp64(const InstDev *__restrict__ insts, const WorkItem *__restrict__ items,
@@ -161,23 +202,30 @@ __global__ void __launch_bounds__(kBlock)
     constexpr bool PUSH = (MODE == kModeFused || MODE == kModeGatherPush || MODE == kModeFusedList);
     constexpr bool REBIN = (MODE == kModeFused || MODE == kModeBoundary || LIST);
     constexpr bool DEP = (MODE == kModeFused || MODE == kModeDeposit || MODE == kModeFusedList);
+    constexpr bool BINS = REBIN && !LIST;
     constexpr int EX = TX + 1, EY = TY + 1, EZ = TZ + 1, NE = EX * EY * EZ;
     constexpr int RX = TX + 3, RY = TY + 3, RZ = TZ + 3, NR = RX * RY * RZ;
     __shared__ double sE[PUSH ? 3 * NE : 1];
     __shared__ unsigned long long sR[DEP ? NR : 1];
-    __shared__ LeaveBuf sLeave[(REBIN && !LIST) ? kWaves : 1];
-    __shared__ int sLcnt[kWaves];
-    __shared__ double sRed[kWaves];
-    __shared__ int sFront, sFrontLimit;
-    __shared__ int64_t sListBase;
-
+    __shared__ Buf64<IDS, kLeaveCap> sLeave[BINS ? kWaves : 1];
+    __shared__ Buf64<IDS, kStash> sStash[BINS ? kWaves : 1];
+    __shared__ double sKe[PUSH ? kKeSlots : 1][kWaves];
+    __shared__ SpecMeta sMeta[kMaxSpecies];
+    __shared__ int sBlk[BINS ? kMaxSpecies : 1];          // full blocks written
+    __shared__ int sLeft[BINS ? kMaxSpecies : 1][kWaves];  // stayers left in each stash
     __shared__ int sItem;
+
+    const int lane = lane_id();
+    const int wv = uniform((int)threadIdx.x >> 6);
     for (int iter = 0;; ++iter) {
+        // (opaque: index arithmetic hoisted out of the item loop would hold
+        // registers through the particle loop)
+        const int tid = QUEUE ? opaque((int)threadIdx.x) : (int)threadIdx.x;
         int item;
         if (QUEUE) {
-            if (threadIdx.x == 0) sItem = (int)atomicAdd(queue, 1u);
+            if (tid == 0) sItem = (int)atomicAdd(queue, 1u);
             __syncthreads();
-            item = sItem;
+            item = uniform(sItem);
             if (item >= nitems) break;
         } else {
             if (iter > 0) break;
@@ -191,81 +239,80 @@ __global__ void __launch_bounds__(kBlock)
         const int tile = it.tile;
         const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
         const int lox = tx * TX, loy = ty * TY, loz = tz * TZ;
-        const int tid = threadIdx.x;
-        const int wv = tid >> 6;
-        const bool ids = I->track_ids != 0;
+        const bool ids = IDS && I->track_ids != 0;
         const bool excl = it.nchunks == 1;  // this workgroup alone fills the tile's front runs
-        unsigned long long *__restrict__ flags = I->flags;
+        const int ns = I->nspecies;
+        const int nbuf = par ^ 1;
+        const int acc_buf = (MODE == kModeFused || MODE == kModeFusedList) ? nbuf : par;
 
+        // every load of the E tile and of the species' bin words is issued
+        // before the first one is used
+        constexpr int KE = PUSH ? (NE + kBlock - 1) / kBlock : 1;
+        double ev[3][KE];
         if (PUSH) {
-            const double *__restrict__ ex = I->e[0];
-            const double *__restrict__ ey = I->e[1];
-            const double *__restrict__ ez = I->e[2];
-            for (int l = tid; l < NE; l += kBlock) {
+#pragma unroll
+            for (int k = 0; k < KE; ++k) {
+                const int l = min(tid + k * kBlock, NE - 1);
                 const int lx = l % EX, ly = (l / EX) % EY, lz = l / (EX * EY);
                 const int gx = wrap_near(lox + lx, nx), gy = wrap_near(loy + ly, ny),
                           gz = wrap_near(loz + lz, nz);
                 const int64_t g = gx + (int64_t)nx * (gy + (int64_t)ny * gz);
-                sE[l] = gload(ex, g);
-                sE[NE + l] = gload(ey, g);
-                sE[2 * NE + l] = gload(ez, g);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) ev[a][k] = gload(I->e[a], g);
             }
         }
+        load_meta<LIST>(sMeta, I, it, par, tid, ns);
+        if (BINS && tid < kMaxSpecies) sBlk[tid] = 0;
         if (DEP)
             for (int l = tid; l < NR; l += kBlock) sR[l] = 0ull;
-        if (tid < kWaves) sLcnt[tid] = 0;
+        if (PUSH) {
+#pragma unroll
+            for (int k = 0; k < KE; ++k) {
+                const int l = tid + k * kBlock;
+                if (l < NE) {
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) sE[a * NE + l] = ev[a][k];
+                }
+            }
+        }
         __syncthreads();
 
         const double dt = I->dt;
         const double dt2 = dt * 0.5;
         const double bx = I->b0[0], by = I->b0[1], bz = I->b0[2];
-        const int nbuf = par ^ 1;
-        const unsigned long long lanemask_lt = (1ull << lane_id()) - 1ull;
-        unsigned long long *__restrict__ racc =
-            I->rho_acc[(MODE == kModeFused || MODE == kModeFusedList) ? nbuf : par];
+        // the tile's part of the box
+        const double tlx = uniform((double)lox), tly = uniform((double)loy),
+                     tlz = uniform((double)loz);
+        const double thx = uniform((double)min(lox + TX, nx)), thy = uniform((double)min(loy + TY, ny)),
+                     thz = uniform((double)min(loz + TZ, nz));
+        auto in_tile = [&](const P64 &q) {
+            return q.x >= tlx && q.x < thx && q.y >= tly && q.y < thy && q.z >= tlz && q.z < thz;
+        };
 
-        for (int s = 0; s < I->nspecies; ++s) {
+        for (int s = 0; s < ns; ++s) {
             const SpecDev &S = I->sp[s];
-            const int cap = gload(S.bin_cap, tile);
-            const unsigned long long word = gload(S.count[par], tile);
-            const int F = min(bin_front(word), cap);
-            const int B = min(bin_back(word), cap - F);
+            const int F = uniform(sMeta[s].F), B = uniform(sMeta[s].B);
+            const int cap = uniform(sMeta[s].cap);
             const int cnt = F + B;
-            const int64_t base = gload(S.bin_base, tile);
-            int per = (cnt + it.nchunks - 1) / it.nchunks;
-            per = (per + 63) & ~63;
+            const int64_t base = uniform(sMeta[s].base);
+            const int per = chunk_size(cnt, it.nchunks);
             const int start = it.chunk * per;
             const int end = min(cnt, start + per);
-            if (REBIN) {
-                // the previous species' particles are all stored before its
-                // list base and front counters are replaced
-                __syncthreads();
-                if (tid == 0) {
-                    int lim = cap;
-                    if (LIST && end > start)  // one reservation per item and species
-                        sListBase = (int64_t)gatomic_add(&S.count[nbuf][0],
-                                                         (unsigned long long)(end - start));
-                    if (!LIST && excl && cnt > 0) {
-                        // reserve the whole front run: arrivals from neighbours stay behind it
-                        const unsigned long long old =
-                            gatomic_add(&S.count[nbuf][tile], (unsigned long long)cnt);
-                        lim = cap - bin_back(old);
-                    }
-                    sFront = 0;
-                    sFrontLimit = lim;
-                }
-                __syncthreads();
-            }
+            const int64_t list0 = LIST ? uniform(sMeta[s].list) : 0;
             const double qm = S.qm;
             const double qfix = S.qfix;
             // Boris constants for the uniform B (t = qm B dt/2, s = 2t/(1+|t|^2))
-            const double t0 = qm * bx * dt2, t1 = qm * by * dt2, t2 = qm * bz * dt2;
+            const double t0 = uniform(qm * bx * dt2), t1 = uniform(qm * by * dt2),
+                         t2 = uniform(qm * bz * dt2);
             const double tt = t0 * t0 + t1 * t1 + t2 * t2;
-            const double s0 = 2 * t0 / (1 + tt), s1 = 2 * t1 / (1 + tt), s2 = 2 * t2 / (1 + tt);
+            const double s0 = uniform(2 * t0 / (1 + tt)), s1 = uniform(2 * t1 / (1 + tt)),
+                         s2 = uniform(2 * t2 / (1 + tt));
             double keo = 0.0, ken = 0.0;
+            int lc = 0, sc = 0;  // particles in this wavefront's leaver buffer and stash
 
             const BinView64 cur = bin_view64(S, par, base, ids);
-            const BinView64 nxt = bin_view64(S, nbuf, base, ids);
+            // this chunk's part of the new front run starts at its slot `start`
+            const BinView64 nxt = bin_view64(S, nbuf, base + start, ids);
             P64 nextq{0, 0, 0, 0, 0, 0, 0};
             if (start + tid < end)
                 nextq = load_bin64(cur, (uint32_t)bin_slot(start + tid, F, B, cap), ids);
@@ -286,7 +333,9 @@ __global__ void __launch_bounds__(kBlock)
                     const int lx = min(max(ix - lox, 0), TX - 1);
                     const int ly = min(max(iy - loy, 0), TY - 1);
                     const int lz = min(max(iz - loz, 0), TZ - 1);
-                    const int l0 = lx + EX * (ly + EY * lz);
+                    const unsigned l0 = (unsigned)(lx + EX * (ly + EY * lz));
+                    const lds_ptr<double> ex0 = lds_base(sE, l0), ey0 = lds_base(sE + NE, l0),
+                                          ez0 = lds_base(sE + 2 * NE, l0);
                     double e0 = 0.0, e1 = 0.0, e2 = 0.0;
                     const double wx[2] = {wx0, wx1}, wy[2] = {wy0, wy1}, wz[2] = {wz0, wz1};
 #pragma unroll
@@ -295,11 +344,11 @@ __global__ void __launch_bounds__(kBlock)
                         for (int j = 0; j < 2; ++j)
 #pragma unroll
                             for (int k = 0; k < 2; ++k) {
-                                const int l = l0 + i + EX * (j + EY * k);
+                                const int l = i + EX * (j + EY * k);
                                 const double w = wx[i] * wy[j] * wz[k];
-                                e0 += sE[l] * w;
-                                e1 += sE[NE + l] * w;
-                                e2 += sE[2 * NE + l] * w;
+                                e0 += lds_read(ex0, l) * w;
+                                e1 += lds_read(ey0, l) * w;
+                                e2 += lds_read(ez0, l) * w;
                             }
                     keo += q.vx * q.vx + q.vy * q.vy + q.vz * q.vz;
                     // Boris (particle_mover_boris.f90:42-62)
@@ -324,20 +373,54 @@ __global__ void __launch_bounds__(kBlock)
                     if (active) store_bin64(cur, (uint32_t)bin_slot(p, F, B, cap), q, ids);
                     continue;
                 }
-                int ntile = tile;
-                if (REBIN && active) {
-                    q.x = apply_periodic(apply_periodic(q.x, nx), nx);
-                    q.y = apply_periodic(apply_periodic(q.y, ny), ny);
-                    q.z = apply_periodic(apply_periodic(q.z, nz), nz);
+                // a particle still in its tile needs no wrap and no new tile
+                bool stay = active && in_tile(q);
+                if (REBIN && active && !stay) {
                     if (!(q.x >= 0.0 && q.x < nx && q.y >= 0.0 && q.y < ny && q.z >= 0.0 &&
                           q.z < nz)) {
-                        gatomic_add(&flags[kFlagRange], 1ull);
-                        q.x = fmin(fmax(q.x - floor(q.x / nx) * nx, 0.0), nx - 1e-9);
-                        q.y = fmin(fmax(q.y - floor(q.y / ny) * ny, 0.0), ny - 1e-9);
-                        q.z = fmin(fmax(q.z - floor(q.z / nz) * nz, 0.0), nz - 1e-9);
+                        q.x = apply_periodic(apply_periodic(q.x, nx), nx);
+                        q.y = apply_periodic(apply_periodic(q.y, ny), ny);
+                        q.z = apply_periodic(apply_periodic(q.z, nz), nz);
+                        if (!(q.x >= 0.0 && q.x < nx && q.y >= 0.0 && q.y < ny && q.z >= 0.0 &&
+                              q.z < nz)) {
+                            gatomic_add(&I->flags[kFlagRange], 1ull);
+                            q.x = fmin(fmax(q.x - floor(q.x / nx) * nx, 0.0), nx - 1e-9);
+                            q.y = fmin(fmax(q.y - floor(q.y / ny) * ny, 0.0), ny - 1e-9);
+                            q.z = fmin(fmax(q.z - floor(q.z / nz) * nz, 0.0), nz - 1e-9);
+                        }
+                        stay = in_tile(q);
                     }
-                    const int cxi = (int)q.x, cyi = (int)q.y, czi = (int)q.z;
-                    ntile = cxi / TX + ntx * (cyi / TY + nty * (czi / TZ));
+                }
+                bool block = false;  // this wavefront stores a full block
+                int blk;             // its number (lane 0)
+                int nst = 0;
+                unsigned long long sm = 0ull;
+                if (BINS) {
+                    sm = __ballot(stay);
+                    const unsigned long long lm = __ballot(active && !stay);
+                    if (lm) {
+                        // particles that left: per-wave LDS buffer, routed in batches
+                        const int nl = (int)__popcll(lm);
+                        const bool leave = active && !stay;
+                        if (lc + nl > kLeaveCap) {
+                            flush_leavers<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids);
+                            lc = 0;
+                        }
+                        if (nl <= kLeaveCap) {
+                            if (leave) sLeave[wv].put(lc + lane_rank(lm), q, ids);
+                            lc += nl;
+                        } else if (leave) {
+                            route_back(S, nbuf, tile_of<TX, TY, TZ>(q, ntx, nty), q, ids, I->flags);
+                        }
+                    }
+                    nst = (int)__popcll(sm);
+                    const int holes = 64 - nst;
+                    block = holes <= sc;
+                    if (block) {
+                        // (arrives while the charge is deposited)
+                        if (lane == 0) blk = atomicAdd(&sBlk[s], 1);
+                        sc -= holes;
+                    }
                 }
                 if (DEP && active) {
                     const int ix = (int)q.x, iy = (int)q.y, iz = (int)q.z;
@@ -346,9 +429,12 @@ __global__ void __launch_bounds__(kBlock)
                     cic_w<WO>(q.y - (double)iy, wy0, wy1);
                     cic_w<WO>(q.z - (double)iz, wz0, wz1);
                     const double wx[2] = {wx0, wx1}, wy[2] = {wy0, wy1}, wz[2] = {wz0, wz1};
-                    const int dx = wrap_index(ix - lox + 1, nx);
-                    const int dy = wrap_index(iy - loy + 1, ny);
-                    const int dz = wrap_index(iz - loz + 1, nz);
+                    int dx = ix - lox + 1, dy = iy - loy + 1, dz = iz - loz + 1;
+                    if (!stay) {
+                        dx = wrap_index(dx, nx);
+                        dy = wrap_index(dy, ny);
+                        dz = wrap_index(dz, nz);
+                    }
                     if (dx <= TX + 1 && dy <= TY + 1 && dz <= TZ + 1) {
                         const int l0 = dx + RX * (dy + RY * dz);
 #pragma unroll
@@ -362,7 +448,8 @@ __global__ void __launch_bounds__(kBlock)
                                               (unsigned long long)v);
                                 }
                     } else {
-                        gatomic_add(&flags[kFlagFast], 1ull);
+                        unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
+                        gatomic_add(&I->flags[kFlagFast], 1ull);
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -373,96 +460,62 @@ __global__ void __launch_bounds__(kBlock)
                                               gz = (iz + k) % nz;
                                     const long long v = fix_round(wx[i] * wy[j] * wz[k], qfix);
                                     gatomic_add(&racc[gx + (int64_t)nx * (gy + (int64_t)ny * gz)],
-                                              (unsigned long long)v);
+                                                (unsigned long long)v);
                                 }
                     }
                 }
+                // the particle loaded ahead arrives before the stores are issued:
+                // memory operations complete in order, so a wait for it at the
+                // top of the next iteration would be one for these stores as well
+                if (BINS) arrived(nextq, ids);
                 if (LIST) {
                     // retry path: every particle to the species' contiguous
                     // list, in bin order inside this item's reserved range
-                    if (active) store_p64(S, nbuf, sListBase + (p - start), q, ids);
-                } else if (REBIN) {
-                    // particles that stayed: front run of this tile's bin
-                    const bool stay = active && ntile == tile;
-                    const unsigned long long m = __ballot(stay);
-                    if (m) {
-                        const int leader = __ffsll((unsigned long long)m) - 1;
-                        const int nst = (int)__popcll(m);
-                        int b = 0, lim = 0;
-                        if (excl) {
-                            if (lane_id() == leader) b = atomicAdd(&sFront, nst);
-                            lim = sFrontLimit;
-                        } else if (lane_id() == leader) {
-                            const unsigned long long old =
-                                gatomic_add(&S.count[nbuf][tile], (unsigned long long)nst);
-                            b = bin_front(old);
-                            lim = cap - bin_back(old);
-                        }
-                        b = lane_bcast(b, leader);
-                        lim = lane_bcast(lim, leader);
-                        if (stay) {
-                            const int slot = b + (int)__popcll(m & lanemask_lt);
-                            if (slot < lim)
-                                store_bin64(nxt, (uint32_t)slot, q, ids);
-                            else
-                                gatomic_add(&flags[kFlagOverflow], 1ull);
-                        }
-                    }
-                    // particles that left: per-wave LDS buffer, routed in batches
-                    const bool leave = active && ntile != tile;
-                    const unsigned long long lm = __ballot(leave);
-                    if (lm) {
-                        const int nl = (int)__popcll(lm);
-                        int c = sLcnt[wv];
-                        if (c + nl > kLeaveCap) {
-                            flush_leavers(sLeave[wv], c, S, nbuf, ids, flags);
-                            c = 0;
-                        }
-                        if (nl <= kLeaveCap) {
-                            if (leave) {
-                                const int slot = c + (int)__popcll(lm & lanemask_lt);
-                                LeaveBuf &lb = sLeave[wv];
-                                lb.c[0][slot] = q.x;
-                                lb.c[1][slot] = q.y;
-                                lb.c[2][slot] = q.z;
-                                lb.c[3][slot] = q.vx;
-                                lb.c[4][slot] = q.vy;
-                                lb.c[5][slot] = q.vz;
-                                lb.id[slot] = q.id;
-                                lb.dest[slot] = ntile;
-                            }
-                            c += nl;
-                        } else if (leave) {
-                            route_back(S, nbuf, ntile, q, ids, flags);
-                        }
-                        if (lane_id() == 0) sLcnt[wv] = c;
-                    }
+                    if (active) store_p64(S, nbuf, list0 + (p - start), q, ids);
+                } else if (block) {
+                    wave_sync();
+                    if (!stay) sStash[wv].get(sc + lane_rank(~sm), q, ids);
+                    store_bin64(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                } else if (nst > 0) {
+                    wave_sync();
+                    if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
+                    sc += nst;
                 }
             }
-            if (REBIN && !LIST) {
-                flush_leavers(sLeave[wv], sLcnt[wv], S, nbuf, ids, flags);
+            if (BINS) {
+                flush_leavers<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids);
+                if (lane == 0) sLeft[s][wv] = sc;
                 __syncthreads();
-                if (tid < kWaves) sLcnt[tid] = 0;
-                if (tid == 0 && excl && cnt > sFront) {
-                    // release the reserved but unused part of the front run
-                    gatomic_add(&S.count[nbuf][tile],
-                              (unsigned long long)(-(long long)(cnt - sFront)));
+                // the stayers left in the stashes follow the blocks
+                int o = 64 * sBlk[s], m = o;
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) {
+                    const int r = sLeft[s][w];
+                    if (w < wv) o += r;
+                    m += r;
                 }
-                __syncthreads();
+                if (lane < sc) {
+                    P64 q;
+                    sStash[wv].get(lane, q, ids);
+                    store_bin64(nxt, (uint32_t)(o + lane), q, ids);
+                }
+                wave_sync();
+                if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
             }
             if (PUSH) {
-                const double so = block_sum(keo, sRed);
-                const double sn = block_sum(ken, sRed);
-                if (tid == 0) {
-                    gstore(I->ke_partial, (int64_t)s * I->nitems + it.slot, 0.5 * S.mass * so);
-                    gstore(I->ke_partial, (int64_t)(kMaxSpecies + s) * I->nitems + it.slot,
-                           0.5 * S.mass * sn);
+                keo = wave_total(keo);
+                ken = wave_total(ken);
+                if (lane == 0) {
+                    sKe[s][wv] = keo;
+                    sKe[kMaxSpecies + s][wv] = ken;
                 }
             }
         }
 
+        __syncthreads();
+        if (PUSH) write_ke(I, it, tid, ns, sKe);
         if (DEP) {
-            __syncthreads();
+            unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
             for (int l = tid; l < NR; l += kBlock) {
                 const unsigned long long v = sR[l];
                 if (v == 0ull) continue;
@@ -474,7 +527,7 @@ __global__ void __launch_bounds__(kBlock)
             }
         }
         // the next item reuses the LDS blocks and sItem
-        __syncthreads();
+        if (QUEUE) __syncthreads();
     }
 }
 
@@ -593,23 +646,37 @@ __global__ void k_cell_counts(const InstDev *__restrict__ insts, int inst, int s
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
+// List mode always handles ids (it is the rare retry); a deposit reads none.
 template <int TX, int TY, int TZ, int WO>
-static hipError_t launch_tile(int mode, const InstDev *insts, const WorkItem *items,
+static hipError_t launch_tile(int mode, bool ids, const InstDev *insts, const WorkItem *items,
                               int nitems, const int *parity, hipStream_t st)
 {
     dim3 g(nitems), b(kBlock);
-#define OHPIC_FP_CASE(M)                                                                     \
-    case M:                                                                                  \
-        hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, M>), g, b, 0, st, insts, items, \
-                           parity, nullptr, nitems);                                         \
-        break;
+#define OHPIC_FP_CASE(M, IDS)                                                                     \
+    hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, M, IDS>), g, b, 0, st, insts, items, parity, \
+                       nullptr, nitems)
     switch (mode) {
-        OHPIC_FP_CASE(kModeFused)
-        OHPIC_FP_CASE(kModeDeposit)
-        OHPIC_FP_CASE(kModeGatherPush)
-        OHPIC_FP_CASE(kModeBoundary)
-        OHPIC_FP_CASE(kModeFusedList)
-        OHPIC_FP_CASE(kModeBoundaryList)
+    case kModeFused:
+        if (ids)
+            OHPIC_FP_CASE(kModeFused, true);
+        else
+            OHPIC_FP_CASE(kModeFused, false);
+        break;
+    case kModeGatherPush:
+        if (ids)
+            OHPIC_FP_CASE(kModeGatherPush, true);
+        else
+            OHPIC_FP_CASE(kModeGatherPush, false);
+        break;
+    case kModeBoundary:
+        if (ids)
+            OHPIC_FP_CASE(kModeBoundary, true);
+        else
+            OHPIC_FP_CASE(kModeBoundary, false);
+        break;
+    case kModeDeposit: OHPIC_FP_CASE(kModeDeposit, false); break;
+    case kModeFusedList: OHPIC_FP_CASE(kModeFusedList, true); break;
+    case kModeBoundaryList: OHPIC_FP_CASE(kModeBoundaryList, true); break;
     default:
         return hipErrorInvalidValue;
     }
@@ -618,22 +685,28 @@ static hipError_t launch_tile(int mode, const InstDev *insts, const WorkItem *it
 }
 
 template <int TX, int TY, int TZ, int WO>
-static hipError_t launch_tile_queue(const InstDev *insts, const WorkItem *items, int nitems,
-                                    const int *parity, unsigned int *queue, int blocks,
+static hipError_t launch_tile_queue(bool ids, const InstDev *insts, const WorkItem *items,
+                                    int nitems, const int *parity, unsigned int *queue, int blocks,
                                     hipStream_t st)
 {
-    hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue>), dim3(blocks),
-                       dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+    if (ids)
+        hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, true>), dim3(blocks),
+                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+    else
+        hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, false>), dim3(blocks),
+                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
     return hipGetLastError();
 }
 
 template <int TX, int TY, int TZ, int WO>
-static int queue_blocks_per_cu()
+static int queue_blocks_per_cu(bool ids)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &nb, reinterpret_cast<const void *>(&k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue>),
-            kBlock, 0) != hipSuccess) {
+    const void *f = ids ? reinterpret_cast<const void *>(
+                              &k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, true>)
+                        : reinterpret_cast<const void *>(
+                              &k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, false>);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, kBlock, 0) != hipSuccess) {
         (void)hipGetLastError();
         nb = 1;
     }
@@ -646,19 +719,19 @@ bool tile_supported(int tx, int ty, int tz)
            (tx == 16 && ty == 8 && tz == 4);
 }
 
-hipError_t launch_particles(int mode, int precision, int weight_order, const int T[3],
-                            const InstDev *insts, const WorkItem *items, int nitems, const int *parity,
-                            hipStream_t st)
+hipError_t launch_particles(int mode, int precision, int weight_order, const int T[3], bool ids,
+                            const InstDev *insts, const WorkItem *items, int nitems,
+                            const int *parity, hipStream_t st)
 {
     if (nitems <= 0) return hipSuccess;
     if (precision == 1)
-        return launch_particles_mixed(mode, weight_order, T, insts, items, nitems, parity, st);
+        return launch_particles_mixed(mode, weight_order, T, ids, insts, items, nitems, parity, st);
     if (precision != 0) return hipErrorInvalidValue;
-#define OHPIC_TILE(A, B, C)                                                     \
-    if (T[0] == A && T[1] == B && T[2] == C)                                    \
-        return weight_order == 0                                                \
-                   ? launch_tile<A, B, C, 0>(mode, insts, items, nitems, parity, st) \
-                   : launch_tile<A, B, C, 1>(mode, insts, items, nitems, parity, st);
+#define OHPIC_TILE(A, B, C)                                                               \
+    if (T[0] == A && T[1] == B && T[2] == C)                                              \
+        return weight_order == 0                                                          \
+                   ? launch_tile<A, B, C, 0>(mode, ids, insts, items, nitems, parity, st) \
+                   : launch_tile<A, B, C, 1>(mode, ids, insts, items, nitems, parity, st);
     OHPIC_TILE(4, 4, 4)
     OHPIC_TILE(8, 8, 8)
     OHPIC_TILE(8, 8, 4)
@@ -667,7 +740,7 @@ hipError_t launch_particles(int mode, int precision, int weight_order, const int
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_particles_queue(int precision, int weight_order, const int T[3],
+hipError_t launch_particles_queue(int precision, int weight_order, const int T[3], bool ids,
                                   const InstDev *insts, const WorkItem *items, int nitems,
                                   const int *parity, unsigned int *queue, int blocks,
                                   hipStream_t st)
@@ -676,14 +749,15 @@ hipError_t launch_particles_queue(int precision, int weight_order, const int T[3
     if (blocks > nitems) blocks = nitems;
     if (blocks < 1) blocks = 1;
     if (precision == 1)
-        return launch_particles_mixed_queue(weight_order, T, insts, items, nitems, parity, queue,
-                                            blocks, st);
+        return launch_particles_mixed_queue(weight_order, T, ids, insts, items, nitems, parity,
+                                            queue, blocks, st);
     if (precision != 0) return hipErrorInvalidValue;
-#define OHPIC_TILE(A, B, C)                                                                    \
-    if (T[0] == A && T[1] == B && T[2] == C)                                                   \
-        return weight_order == 0                                                               \
-                   ? launch_tile_queue<A, B, C, 0>(insts, items, nitems, parity, queue, blocks, st) \
-                   : launch_tile_queue<A, B, C, 1>(insts, items, nitems, parity, queue, blocks, st);
+#define OHPIC_TILE(A, B, C)                                                                       \
+    if (T[0] == A && T[1] == B && T[2] == C)                                                      \
+        return weight_order == 0 ? launch_tile_queue<A, B, C, 0>(ids, insts, items, nitems,       \
+                                                                 parity, queue, blocks, st)       \
+                                 : launch_tile_queue<A, B, C, 1>(ids, insts, items, nitems,       \
+                                                                 parity, queue, blocks, st);
     OHPIC_TILE(4, 4, 4)
     OHPIC_TILE(8, 8, 8)
     OHPIC_TILE(8, 8, 4)
@@ -692,7 +766,7 @@ hipError_t launch_particles_queue(int precision, int weight_order, const int T[3
     return hipErrorInvalidValue;
 }
 
-int particles_queue_blocks(int precision, int weight_order, const int T[3], int device)
+int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int device)
 {
     int cus = 256;
     hipDeviceProp_t prop;
@@ -702,18 +776,96 @@ int particles_queue_blocks(int precision, int weight_order, const int T[3], int 
         (void)hipGetLastError();
     int per = 1;
     if (precision == 1) {
-        per = particles_mixed_queue_blocks(weight_order, T);
+        per = particles_mixed_queue_blocks(weight_order, T, ids);
     } else {
-#define OHPIC_TILE(A, B, C)                                                              \
-    if (T[0] == A && T[1] == B && T[2] == C)                                             \
-        per = weight_order == 0 ? queue_blocks_per_cu<A, B, C, 0>() : queue_blocks_per_cu<A, B, C, 1>();
-        OHPIC_TILE(4, 4, 4)
-        OHPIC_TILE(8, 8, 8)
-        OHPIC_TILE(8, 8, 4)
-        OHPIC_TILE(16, 8, 4)
+#define OHPIC_TILE(A, B, C)                                                  \
+    if (T[0] == A && T[1] == B && T[2] == C)                                 \
+        per = weight_order == 0 ? queue_blocks_per_cu<A, B, C, 0>(ids)       \
+                                : queue_blocks_per_cu<A, B, C, 1>(ids);
+    OHPIC_TILE(4, 4, 4)
+    OHPIC_TILE(8, 8, 8)
+    OHPIC_TILE(8, 8, 4)
+    OHPIC_TILE(16, 8, 4)
 #undef OHPIC_TILE
     }
     return per * cus;
+}
+
+// Joins the chunks' parts of a split tile's new front runs (blockIdx.x = list
+// entry, blockIdx.y = species).  Chunk c wrote chunk_front[slot0 + c] particles
+// from slot c * per on; the tile's front run is their sum M, so the gaps below
+// M (as many as the tile's leavers, a few per cent) take the particles at and
+// above M.  A step that overflowed a bin is redone from the other buffer.
+template <typename T, int C0>
+__global__ void __launch_bounds__(256) k_close_chunks(const InstDev *__restrict__ insts,
+                                                      const CloseItem *__restrict__ list,
+                                                      const int *__restrict__ parity)
+{
+    constexpr int kCached = 64;
+    __shared__ int sFront[kCached];
+    __shared__ int sSum;
+    const CloseItem c = list[blockIdx.x];
+    const InstDev *I = insts + c.inst;
+    const int s = blockIdx.y;
+    if (s >= I->nspecies || I->flags[kFlagOverflow] != 0ull) return;
+    const SpecDev &S = I->sp[s];
+    const int par = parity[c.inst], nbuf = par ^ 1;
+    const unsigned long long word = S.count[par][c.tile];
+    const int cap = S.bin_cap[c.tile], F = min(bin_front(word), cap);
+    const int cnt = F + min(bin_back(word), cap - F);
+    const int per = chunk_size(cnt, c.nchunks);
+    const int32_t *fr = I->chunk_front + (int64_t)c.slot0 * kMaxSpecies + s;
+    if (threadIdx.x == 0) sSum = 0;
+    __syncthreads();
+    int sum = 0;
+    for (int k = threadIdx.x; k < c.nchunks; k += blockDim.x) {
+        const int m = fr[(int64_t)k * kMaxSpecies];
+        if (k < kCached) sFront[k] = m;
+        sum += m;
+    }
+    if (sum) atomicAdd(&sSum, sum);
+    __syncthreads();
+    const int M = sSum;
+    auto front = [&](int k) { return k < kCached ? sFront[k] : fr[(int64_t)k * kMaxSpecies]; };
+    const int64_t base = S.bin_base[c.tile];
+    for (int j = threadIdx.x; j < cnt - M; j += blockDim.x) {
+        int hole = -1, from = -1, hj = j, fj = j;
+        for (int k = 0; k < c.nchunks; ++k) {
+            const int lo = k * per, end = lo + front(k);
+            if (hole < 0) {
+                const int h = max(0, min(min(cnt, lo + per), M) - end);
+                if (hj < h) hole = end + hj;
+                hj -= h;
+            }
+            if (from < 0) {
+                const int v = max(0, end - max(lo, M));
+                if (fj < v) from = max(lo, M) + fj;
+                fj -= v;
+            }
+            if (lo + per >= cnt) break;
+        }
+        if (hole < 0 || from < 0) break;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            T *p = (T *)S.buf[nbuf][C0 + k];
+            gstore(p, base + hole, gload(p, base + from));
+        }
+        if (I->track_ids) gstore(S.pid[nbuf], base + hole, gload(S.pid[nbuf], base + from));
+    }
+    if (threadIdx.x == 0)
+        S.count[nbuf][c.tile] = (S.count[nbuf][c.tile] & ~0xffffffffull) | (unsigned long long)M;
+}
+
+hipError_t launch_close_chunks(int precision, const InstDev *insts, const CloseItem *list, int n,
+                               int ns, const int *parity, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    const dim3 g(n, ns);
+    if (precision == 1)
+        hipLaunchKernelGGL((k_close_chunks<uint32_t, 1>), g, dim3(256), 0, st, insts, list, parity);
+    else
+        hipLaunchKernelGGL((k_close_chunks<double, 0>), g, dim3(256), 0, st, insts, list, parity);
+    return hipGetLastError();
 }
 
 hipError_t launch_bin_count(const InstDev *insts, int inst, int s, int lbuf, int64_t n,

@@ -15,6 +15,14 @@
 // and the diagnostics stay FP64.  The periodic boundary is an integer wrap of
 // the cell index.  Work decomposition, LDS staging, deposit blocks and
 // re-binning are those of the FP64 kernel.
+//
+// What bounds it: 48 B per particle, and the instructions (about 220 VALU and
+// 22 LDS per particle) with their latencies.  So the wrap and the new tile are
+// found only for particles that leave, when their buffer is routed; the E
+// gather reads its eight nodes before it uses one; and no iteration waits for
+// its own stores.  With the aligned blocks of the front run: 256^3 x 32 ppc
+// 12.62 -> 11.82 ms, 128^3 x 64 with a density peak 3.93 -> 3.21 ms, 64^3 x 32
+// 313 -> 249 us per launch (HIP events, one box).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -130,6 +138,14 @@ __device__ __forceinline__ void store_bin(const BinView &bv, uint32_t slot, cons
     if (ids) gstore(const_cast<int64_t *>(bv.id), (int64_t)slot, q.id);
 }
 
+// The particle's loads have completed from here on.
+__device__ __forceinline__ void arrived(PMx &q, bool ids)
+{
+#pragma unroll
+    for (int a = 0; a < 3; ++a) asm volatile("" : "+v"(q.w[a]), "+v"(q.v[a]));
+    if (ids) asm volatile("" : "+v"(q.id));
+}
+
 // list form: the binned words plus the tile index in buf[b][0]
 __device__ __forceinline__ void store_list_mx(const SpecDev &S, int b, int64_t o, const PMx &q,
                                               int tile, bool ids)
@@ -165,47 +181,86 @@ __device__ __forceinline__ int wrap_cell(int g, int n)
 __device__ __forceinline__ void route_back_mx(const SpecDev &S, int nbuf, int t, const PMx &q,
                                               bool ids, unsigned long long *flags)
 {
+    const int cap = gload(S.bin_cap, t);
+    const int64_t base = gload(S.bin_base, t);
     const unsigned long long old = gatomic_add(&S.count[nbuf][t], 1ull << 32);
     const int f = bin_front(old), b = bin_back(old);
-    const int cap = gload(S.bin_cap, t);
     if (b + f < cap)
-        store_pmx(S, nbuf, gload(S.bin_base, t) + (cap - 1 - b), q, ids);
+        store_pmx(S, nbuf, base + (cap - 1 - b), q, ids);
     else
         gatomic_add(&flags[kFlagOverflow], 1ull);
 }
 
-struct LeaveBufMx {
-    uint32_t w[3][kLeaveCap];
-    float v[3][kLeaveCap];
-    int64_t id[kLeaveCap];
-    int32_t dest[kLeaveCap];
+template <bool IDS, int CAP>
+struct BufMx {
+    uint32_t w[3][CAP];
+    float v[3][CAP];
+    int64_t id[IDS ? CAP : 1];
+
+    __device__ __forceinline__ void put(int i, const PMx &q, bool ids)
+    {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            w[a][i] = q.w[a];
+            v[a][i] = q.v[a];
+        }
+        if (IDS && ids) id[i] = q.id;
+    }
+    __device__ __forceinline__ void get(int i, PMx &q, bool ids) const
+    {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            q.w[a] = w[a][i];
+            q.v[a] = v[a][i];
+        }
+        if (IDS && ids) q.id = id[i];
+    }
 };
 
-__device__ __forceinline__ void flush_leavers_mx(LeaveBufMx &lb, int cnt, const SpecDev &S,
-                                                 int nbuf, bool ids, unsigned long long *flags)
+// The tile a position word triple relative to tile origin (lox, loy, loz)
+// falls in after the periodic wrap; w becomes relative to that tile.
+template <int TX, int TY, int TZ>
+__device__ __forceinline__ int rebase_words(uint32_t w[3], const InstDev *__restrict__ I, int lox,
+                                            int loy, int loz)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int ntx = I->nt[0], nty = I->nt[1];
+    const int gx = wrap_cell(lox + pos_rel(w[0]), I->n[0]), gy = wrap_cell(loy + pos_rel(w[1]), I->n[1]),
+              gz = wrap_cell(loz + pos_rel(w[2]), I->n[2]);
+    const int tx = (int)((unsigned)gx / TX), ty = (int)((unsigned)gy / TY),
+              tz = (int)((unsigned)gz / TZ);
+    w[0] = pos_word(gx - tx * TX, w[0] & kFracMask);
+    w[1] = pos_word(gy - ty * TY, w[1] & kFracMask);
+    w[2] = pos_word(gz - tz * TZ, w[2] & kFracMask);
+    // tile counts are below 2^24 (axes <= 1024 cells, tiles >= 4)
+    return tx + (int)__umul24((unsigned)ty, (unsigned)ntx) +
+           (int)__umul24((unsigned)tz, (unsigned)(ntx * nty));
+}
+
+// Routes the first `cnt` buffered leavers of this wavefront (lane l takes
+// entry l) to the back runs of their new tiles.  The wrap and the new tile are
+// found here, for up to kLeaveCap particles at once, and not for every
+// particle of the sweep (about 60 of its 254 VALU instructions).
+template <int TX, int TY, int TZ, bool IDS>
+__device__ __forceinline__ void flush_leavers_mx(const BufMx<IDS, kLeaveCap> &lb, int cnt,
+                                                 const InstDev *__restrict__ I, const SpecDev &S,
+                                                 int nbuf, bool ids, int lox, int loy, int loz)
+{
+    wave_sync();
     const int l = lane_id();
     if (l < cnt) {
         PMx q;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            q.w[a] = lb.w[a][l];
-            q.v[a] = lb.v[a][l];
-        }
-        q.id = lb.id[l];
-        route_back_mx(S, nbuf, lb.dest[l], q, ids, flags);
+        lb.get(l, q, ids);
+        const int t = rebase_words<TX, TY, TZ>(q.w, I, lox, loy, loz);
+        route_back_mx(S, nbuf, t, q, IDS && ids, I->flags);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
 }
 
-template <int TX, int TY, int TZ, int WO, int MODE_>
+// IDS: instances may keep particle ids (each instance's track_ids says whether
+// it does); without it no register, LDS or branch is spent on them.
+template <int TX, int TY, int TZ, int WO, int MODE_, bool IDS>
 __global__ void __launch_bounds__(kBlock)
-    __attribute__((amdgpu_waves_per_eu(OHPIC_MX_MIN_WAVES, 8)))
+    __attribute__((amdgpu_waves_per_eu((MODE_ == kModeFusedQueue && IDS) ? 4 : OHPIC_MX_MIN_WAVES, 8)))
     k_particles_mixed(const InstDev *__restrict__ insts, const WorkItem *__restrict__ items,
                       const int *__restrict__ parity, unsigned int *__restrict__ queue,
                       int nitems)
@@ -218,6 +273,7 @@ __global__ void __launch_bounds__(kBlock)
     constexpr bool PUSH = (MODE == kModeFused || MODE == kModeGatherPush || MODE == kModeFusedList);
     constexpr bool REBIN = (MODE == kModeFused || MODE == kModeBoundary || LIST);
     constexpr bool DEP = (MODE == kModeFused || MODE == kModeDeposit || MODE == kModeFusedList);
+    constexpr bool BINS = REBIN && !LIST;
     constexpr int EX = TX + 1, EY = TY + 1, EZ = TZ + 1, NE = EX * EY * EZ;
     constexpr int RX = TX + 3, RY = TY + 3, RZ = TZ + 3, NR = RX * RY * RZ;
     // E tile: (E_x, E_y) of a node side by side and E_z apart, so that the
@@ -228,19 +284,25 @@ __global__ void __launch_bounds__(kBlock)
     __shared__ float2 sExy[PUSH ? NE : 1];
     __shared__ float sEz[PUSH ? NE : 1];
     __shared__ unsigned long long sR[DEP ? NR : 1];
-    __shared__ LeaveBufMx sLeave[(REBIN && !LIST) ? kWaves : 1];
-    __shared__ int sLcnt[kWaves];
-    __shared__ double sRed[kWaves];
-    __shared__ int sFront, sFrontLimit;
-    __shared__ int64_t sListBase;
-
+    __shared__ BufMx<IDS, kLeaveCap> sLeave[BINS ? kWaves : 1];
+    __shared__ BufMx<IDS, kStash> sStash[BINS ? kWaves : 1];
+    __shared__ double sKe[PUSH ? kKeSlots : 1][kWaves];
+    __shared__ SpecMeta sMeta[kMaxSpecies];
+    __shared__ int sBlk[BINS ? kMaxSpecies : 1];          // full blocks written
+    __shared__ int sLeft[BINS ? kMaxSpecies : 1][kWaves];  // stayers left in each stash
     __shared__ int sItem;
+
+    const int lane = lane_id();
+    const int wv = uniform((int)threadIdx.x >> 6);
     for (int iter = 0;; ++iter) {
+        // (opaque: index arithmetic hoisted out of the item loop would hold
+        // registers through the particle loop)
+        const int tid = QUEUE ? opaque((int)threadIdx.x) : (int)threadIdx.x;
         int item;
         if (QUEUE) {
-            if (threadIdx.x == 0) sItem = (int)atomicAdd(queue, 1u);
+            if (tid == 0) sItem = (int)atomicAdd(queue, 1u);
             __syncthreads();
-            item = sItem;
+            item = uniform(sItem);
             if (item >= nitems) break;
         } else {
             if (iter > 0) break;
@@ -254,82 +316,79 @@ __global__ void __launch_bounds__(kBlock)
         const int tile = it.tile;
         const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
         const int lox = tx * TX, loy = ty * TY, loz = tz * TZ;
-        const int tid = threadIdx.x;
-        const int wv = tid >> 6;
-        const bool ids = I->track_ids != 0;
-        const bool excl = it.nchunks == 1;
-        unsigned long long *__restrict__ flags = I->flags;
+        const bool ids = IDS && I->track_ids != 0;
+        const bool excl = it.nchunks == 1;  // this workgroup alone fills the tile's front runs
+        const int ns = I->nspecies;
+        const int nbuf = par ^ 1;
+        const int acc_buf = (MODE == kModeFused || MODE == kModeFusedList) ? nbuf : par;
 
+        // every load of the E tile and of the species' bin words is issued
+        // before the first one is used
+        constexpr int KE = PUSH ? (NE + kBlock - 1) / kBlock : 1;
+        double ev[3][KE];
         if (PUSH) {
-            const double *__restrict__ ex = I->e[0];
-            const double *__restrict__ ey = I->e[1];
-            const double *__restrict__ ez = I->e[2];
-            for (int l = tid; l < NE; l += kBlock) {
+#pragma unroll
+            for (int k = 0; k < KE; ++k) {
+                const int l = min(tid + k * kBlock, NE - 1);
                 const int lx = l % EX, ly = (l / EX) % EY, lz = l / (EX * EY);
                 const int gx = wrap_near(lox + lx, nx), gy = wrap_near(loy + ly, ny),
                           gz = wrap_near(loz + lz, nz);
                 const int64_t g = gx + (int64_t)nx * (gy + (int64_t)ny * gz);
-                sExy[l] = make_float2((float)gload(ex, g), (float)gload(ey, g));
-                sEz[l] = (float)gload(ez, g);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) ev[a][k] = gload(I->e[a], g);
             }
         }
+        load_meta<LIST>(sMeta, I, it, par, tid, ns);
+        if (BINS && tid < kMaxSpecies) sBlk[tid] = 0;
         if (DEP)
             for (int l = tid; l < NR; l += kBlock) sR[l] = 0ull;
-        if (tid < kWaves) sLcnt[tid] = 0;
+        if (PUSH) {
+#pragma unroll
+            for (int k = 0; k < KE; ++k) {
+                const int l = tid + k * kBlock;
+                if (l < NE) {
+                    sExy[l] = make_float2((float)ev[0][k], (float)ev[1][k]);
+                    sEz[l] = (float)ev[2][k];
+                }
+            }
+        }
         __syncthreads();
 
         const float dt = (float)I->dt;
-        const float dt2 = 0.5f * dt;
-        const float dts = dt * kFracScale;  // cells per unit velocity, in 2^-24 units
+        const float dt2 = uniform(0.5f * dt);
+        const float dts = uniform(dt * kFracScale);  // cells per unit velocity, in 2^-24 units
         const float bx = (float)I->b0[0], by = (float)I->b0[1], bz = (float)I->b0[2];
-        const int nbuf = par ^ 1;
-        const unsigned long long lanemask_lt = (1ull << lane_id()) - 1ull;
-        unsigned long long *__restrict__ racc =
-            I->rho_acc[(MODE == kModeFused || MODE == kModeFusedList) ? nbuf : par];
+        // cells of the tile inside the box; an axis of a single tile can wrap
+        // a particle back into its own tile
+        const unsigned limx = (unsigned)min(TX, nx - lox), limy = (unsigned)min(TY, ny - loy),
+                       limz = (unsigned)min(TZ, nz - loz);
+        const bool one_tile = ntx == 1 || nty == 1 || I->nt[2] == 1;
 
-        for (int s = 0; s < I->nspecies; ++s) {
+        for (int s = 0; s < ns; ++s) {
             const SpecDev &S = I->sp[s];
-            const int cap = gload(S.bin_cap, tile);
-            const unsigned long long word = gload(S.count[par], tile);
-            const int F = min(bin_front(word), cap);
-            const int B = min(bin_back(word), cap - F);
+            const int F = uniform(sMeta[s].F), B = uniform(sMeta[s].B);
+            const int cap = uniform(sMeta[s].cap);
             const int cnt = F + B;
-            const int64_t base = gload(S.bin_base, tile);
-            int per = (cnt + it.nchunks - 1) / it.nchunks;
-            per = (per + 63) & ~63;
+            const int64_t base = uniform(sMeta[s].base);
+            const int per = chunk_size(cnt, it.nchunks);
             const int start = it.chunk * per;
             const int end = min(cnt, start + per);
-            if (REBIN) {
-                // the previous species' particles are all stored before its
-                // list base and front counters are replaced
-                __syncthreads();
-                if (tid == 0) {
-                    int lim = cap;
-                    if (LIST && end > start)  // one reservation per item and species
-                        sListBase = (int64_t)gatomic_add(&S.count[nbuf][0],
-                                                         (unsigned long long)(end - start));
-                    if (!LIST && excl && cnt > 0) {
-                        const unsigned long long old =
-                            gatomic_add(&S.count[nbuf][tile], (unsigned long long)cnt);
-                        lim = cap - bin_back(old);
-                    }
-                    sFront = 0;
-                    sFrontLimit = lim;
-                }
-                __syncthreads();
-            }
-            const float qm = (float)S.qm;
+            const int64_t list0 = LIST ? uniform(sMeta[s].list) : 0;
+            const float qm = uniform((float)S.qm);
             const double qfix = S.qfix;
-            const float t0 = qm * bx * dt2, t1 = qm * by * dt2, t2 = qm * bz * dt2;
+            const float t0 = uniform(qm * bx * dt2), t1 = uniform(qm * by * dt2),
+                        t2 = uniform(qm * bz * dt2);
             const float tt = t0 * t0 + t1 * t1 + t2 * t2;
-            const float s0 = 2.0f * t0 / (1.0f + tt), s1 = 2.0f * t1 / (1.0f + tt),
-                        s2 = 2.0f * t2 / (1.0f + tt);
+            const float s0 = uniform(2.0f * t0 / (1.0f + tt)), s1 = uniform(2.0f * t1 / (1.0f + tt)),
+                        s2 = uniform(2.0f * t2 / (1.0f + tt));
             double keo = 0.0, ken = 0.0;
+            int lc = 0, sc = 0;  // particles in this wavefront's leaver buffer and stash
 
             // the next kMxPrefetch particles of this lane are loaded ahead, so each
             // lane keeps that many particle reads in flight
             const BinView cur = bin_view(S, par, base, ids);
-            const BinView nxt = bin_view(S, nbuf, base, ids);
+            // this chunk's part of the new front run starts at its slot `start`
+            const BinView nxt = bin_view(S, nbuf, base + start, ids);
             PMx ahead[kMxPrefetch];
 #pragma unroll
             for (int k = 0; k < kMxPrefetch; ++k) {
@@ -361,8 +420,22 @@ __global__ void __launch_bounds__(kBlock)
                     // base node with 24-bit multiplies (full rate)
                     const unsigned nb =
                         __umul24((unsigned)lz, EX * EY) + __umul24((unsigned)ly, EX) + (unsigned)lx;
-                    const float2 *__restrict__ exy = sExy + nb;
-                    const float *__restrict__ ez0 = sEz + nb;
+                    const lds_ptr<float2> exy = lds_base(sExy, nb);
+                    const lds_ptr<float> ez0 = lds_base(sEz, nb);
+                    // all eight nodes are read before the first is used: one
+                    // LDS latency instead of eight
+                    float2 gxy[2][2][2];
+                    float gz_[2][2][2];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int k = 0; k < 2; ++k)
+#pragma unroll
+                            for (int i = 0; i < 2; ++i) {
+                                gxy[i][j][k] = lds_read(exy, i + EX * (j + EY * k));
+                                gz_[i][j][k] = lds_read(ez0, i + EX * (j + EY * k));
+                            }
+                    __builtin_amdgcn_sched_barrier(0);
                     float e0 = 0.0f, e1 = 0.0f, e2 = 0.0f;
                     const float wx[2] = {wx0, wx1}, wy[2] = {wy0, wy1}, wz[2] = {wz0, wz1};
 #pragma unroll
@@ -371,11 +444,10 @@ __global__ void __launch_bounds__(kBlock)
                         for (int j = 0; j < 2; ++j)
 #pragma unroll
                             for (int k = 0; k < 2; ++k) {
-                                const float2 exy_n = exy[i + EX * (j + EY * k)];
                                 const float w = wx[i] * wy[j] * wz[k];
-                                e0 += exy_n.x * w;
-                                e1 += exy_n.y * w;
-                                e2 += ez0[i + EX * (j + EY * k)] * w;
+                                e0 += gxy[i][j][k].x * w;
+                                e1 += gxy[i][j][k].y * w;
+                                e2 += gz_[i][j][k] * w;
                             }
                     const float vx = q.v[0], vy = q.v[1], vz = q.v[2];
                     keo += (double)(vx * vx + vy * vy + vz * vz);
@@ -399,7 +471,7 @@ __global__ void __launch_bounds__(kBlock)
                     const bool ok =
                         fabsf(sx) < kMaxShift && fabsf(sy) < kMaxShift && fabsf(sz) < kMaxShift;
                     if (!ok) {
-                        gatomic_add(&flags[kFlagRange], 1ull);
+                        gatomic_add(&I->flags[kFlagRange], 1ull);
                     } else {
                         q.w[0] = (uint32_t)((int32_t)q.w[0] + (int32_t)rintf(sx));
                         q.w[1] = (uint32_t)((int32_t)q.w[1] + (int32_t)rintf(sy));
@@ -417,19 +489,53 @@ __global__ void __launch_bounds__(kBlock)
                     }
                 }
                 if (MODE == kModeGatherPush) continue;
-                // global cell, periodic (in [0, n)); new tile and the cell
-                // relative to it
-                const int gx = wrap_cell(lox + rx, nx), gy = wrap_cell(loy + ry, ny),
-                          gz = wrap_cell(loz + rz, nz);
-                const int ctx_t = (int)((unsigned)gx / TX), cty = (int)((unsigned)gy / TY),
-                          ctz = (int)((unsigned)gz / TZ);
-                // tile counts are below 2^24 (axes <= 1024 cells, tiles >= 4)
-                const int ntile = ctx_t + (int)__umul24((unsigned)cty, (unsigned)ntx) +
-                                  (int)__umul24((unsigned)ctz, (unsigned)(ntx * nty));
-                if (REBIN) {
-                    q.w[0] = pos_word(gx - ctx_t * TX, q.w[0] & kFracMask);
-                    q.w[1] = pos_word(gy - cty * TY, q.w[1] & kFracMask);
-                    q.w[2] = pos_word(gz - ctz * TZ, q.w[2] & kFracMask);
+
+                bool block = false;  // this wavefront stores a full block
+                int blk;             // its number (lane 0)
+                bool stay = false;
+                int nst = 0;
+                unsigned long long sm = 0ull;
+                PMx fill;            // what the lanes of leavers store
+                if (BINS) {
+                    stay = active && (unsigned)rx < limx && (unsigned)ry < limy &&
+                           (unsigned)rz < limz;
+                    if (one_tile && active && !stay) {
+                        PMx r = q;
+                        if (rebase_words<TX, TY, TZ>(r.w, I, lox, loy, loz) == tile) {
+                            q = r;
+                            stay = true;
+                        }
+                    }
+                    sm = __ballot(stay);
+                    const unsigned long long lm = __ballot(active && !stay);
+                    if (lm) {
+                        // particles that left: per-wave LDS buffer, routed in batches
+                        const int nl = (int)__popcll(lm);
+                        const bool leave = active && !stay;
+                        if (lc + nl > kLeaveCap) {
+                            flush_leavers_mx<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf,
+                                                              ids, lox, loy, loz);
+                            lc = 0;
+                        }
+                        if (nl <= kLeaveCap) {
+                            if (leave) sLeave[wv].put(lc + lane_rank(lm), q, ids);
+                            lc += nl;
+                        } else if (leave) {
+                            PMx r = q;
+                            const int t = rebase_words<TX, TY, TZ>(r.w, I, lox, loy, loz);
+                            route_back_mx(S, nbuf, t, r, ids, I->flags);
+                        }
+                    }
+                    nst = (int)__popcll(sm);
+                    const int holes = 64 - nst;
+                    block = holes <= sc;
+                    if (block) {
+                        // both arrive while the charge is deposited
+                        if (lane == 0) blk = atomicAdd(&sBlk[s], 1);
+                        sc -= holes;
+                        wave_sync();
+                        if (!stay) sStash[wv].get(sc + lane_rank(~sm), fill, ids);
+                    }
                 }
                 if (DEP && active) {
                     float wx0, wx1, wy0, wy1, wz0, wz1;
@@ -462,7 +568,10 @@ __global__ void __launch_bounds__(kBlock)
                                               (unsigned long long)fix_round(wzd[k], qxy));
                             }
                     } else {
-                        gatomic_add(&flags[kFlagFast], 1ull);
+                        unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
+                        gatomic_add(&I->flags[kFlagFast], 1ull);
+                        const int gx = wrap_cell(lox + rx, nx), gy = wrap_cell(loy + ry, ny),
+                                  gz = wrap_cell(loz + rz, nz);
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -479,87 +588,61 @@ __global__ void __launch_bounds__(kBlock)
                             }
                     }
                 }
+                // the loads ahead arrive before the stores are issued: memory
+                // operations complete in order, so a wait for them at the top
+                // of the next iteration would be one for these stores as well
+#pragma unroll
+                for (int k = 0; BINS && k < kMxPrefetch; ++k) arrived(ahead[k], ids);
                 if (LIST) {
                     // retry path: every particle to the species' contiguous
                     // list, in bin order inside this item's reserved range
-                    if (active) store_list_mx(S, nbuf, sListBase + (p - start), q, ntile, ids);
-                } else if (REBIN) {
-                    const bool stay = active && ntile == tile;
-                    const unsigned long long m = __ballot(stay);
-                    if (m) {
-                        const int leader = __ffsll((unsigned long long)m) - 1;
-                        const int nst = (int)__popcll(m);
-                        int b = 0, lim = 0;
-                        if (excl) {
-                            if (lane_id() == leader) b = atomicAdd(&sFront, nst);
-                            lim = sFrontLimit;
-                        } else if (lane_id() == leader) {
-                            const unsigned long long old =
-                                gatomic_add(&S.count[nbuf][tile], (unsigned long long)nst);
-                            b = bin_front(old);
-                            lim = cap - bin_back(old);
-                        }
-                        b = lane_bcast(b, leader);
-                        lim = lane_bcast(lim, leader);
-                        if (stay) {
-                            const int slot = b + (int)__popcll(m & lanemask_lt);
-                            if (slot < lim)
-                                store_bin(nxt, (uint32_t)slot, q, ids);
-                            else
-                                gatomic_add(&flags[kFlagOverflow], 1ull);
-                        }
+                    if (active) {
+                        const int t = rebase_words<TX, TY, TZ>(q.w, I, lox, loy, loz);
+                        store_list_mx(S, nbuf, list0 + (p - start), q, t, ids);
                     }
-                    const bool leave = active && ntile != tile;
-                    const unsigned long long lm = __ballot(leave);
-                    if (lm) {
-                        const int nl = (int)__popcll(lm);
-                        int c = sLcnt[wv];
-                        if (c + nl > kLeaveCap) {
-                            flush_leavers_mx(sLeave[wv], c, S, nbuf, ids, flags);
-                            c = 0;
-                        }
-                        if (nl <= kLeaveCap) {
-                            if (leave) {
-                                const int slot = c + (int)__popcll(lm & lanemask_lt);
-                                LeaveBufMx &lb = sLeave[wv];
-#pragma unroll
-                                for (int a = 0; a < 3; ++a) {
-                                    lb.w[a][slot] = q.w[a];
-                                    lb.v[a][slot] = q.v[a];
-                                }
-                                lb.id[slot] = q.id;
-                                lb.dest[slot] = ntile;
-                            }
-                            c += nl;
-                        } else if (leave) {
-                            route_back_mx(S, nbuf, ntile, q, ids, flags);
-                        }
-                        if (lane_id() == 0) sLcnt[wv] = c;
-                    }
+                } else if (block) {
+                    if (!stay) q = fill;
+                    store_bin(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                } else if (nst > 0) {
+                    wave_sync();
+                    if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
+                    sc += nst;
                 }
             }
-            if (REBIN && !LIST) {
-                flush_leavers_mx(sLeave[wv], sLcnt[wv], S, nbuf, ids, flags);
+            if (BINS) {
+                flush_leavers_mx<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids, lox, loy, loz);
+                if (lane == 0) sLeft[s][wv] = sc;
                 __syncthreads();
-                if (tid < kWaves) sLcnt[tid] = 0;
-                if (tid == 0 && excl && cnt > sFront)
-                    gatomic_add(&S.count[nbuf][tile],
-                              (unsigned long long)(-(long long)(cnt - sFront)));
-                __syncthreads();
+                // the stayers left in the stashes follow the blocks
+                int o = 64 * sBlk[s], m = o;
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) {
+                    const int r = sLeft[s][w];
+                    if (w < wv) o += r;
+                    m += r;
+                }
+                if (lane < sc) {
+                    PMx q;
+                    sStash[wv].get(lane, q, ids);
+                    store_bin(nxt, (uint32_t)(o + lane), q, ids);
+                }
+                wave_sync();
+                if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
             }
             if (PUSH) {
-                const double so = block_sum(keo, sRed);
-                const double sn = block_sum(ken, sRed);
-                if (tid == 0) {
-                    gstore(I->ke_partial, (int64_t)s * I->nitems + it.slot, 0.5 * S.mass * so);
-                    gstore(I->ke_partial, (int64_t)(kMaxSpecies + s) * I->nitems + it.slot,
-                           0.5 * S.mass * sn);
+                keo = wave_total(keo);
+                ken = wave_total(ken);
+                if (lane == 0) {
+                    sKe[s][wv] = keo;
+                    sKe[kMaxSpecies + s][wv] = ken;
                 }
             }
         }
 
+        __syncthreads();
+        if (PUSH) write_ke(I, it, tid, ns, sKe);
         if (DEP) {
-            __syncthreads();
+            unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
             for (int l = tid; l < NR; l += kBlock) {
                 const unsigned long long v = sR[l];
                 if (v == 0ull) continue;
@@ -571,7 +654,7 @@ __global__ void __launch_bounds__(kBlock)
             }
         }
         // the next item reuses the LDS blocks and sItem
-        __syncthreads();
+        if (QUEUE) __syncthreads();
     }
 }
 
@@ -764,23 +847,37 @@ __global__ void k_load_hump_mx(const InstDev *__restrict__ insts, int inst, int 
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
+// List mode always handles ids (it is the rare retry); a deposit reads none.
 template <int TX, int TY, int TZ, int WO>
-static hipError_t launch_tile_mx(int mode, const InstDev *insts, const WorkItem *items,
-                                 int nitems, const int *parity, hipStream_t st)
+static hipError_t launch_tile_mx(int mode, bool ids, const InstDev *insts, const WorkItem *items,
+                              int nitems, const int *parity, hipStream_t st)
 {
     dim3 g(nitems), b(kBlock);
-#define OHPIC_MX_CASE(M)                                                                 \
-    case M:                                                                              \
-        hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, M>), g, b, 0, st, insts, items, \
-                           parity, nullptr, nitems);                                     \
-        break;
+#define OHPIC_MX_CASE(M, IDS)                                                                     \
+    hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, M, IDS>), g, b, 0, st, insts, items, parity, \
+                       nullptr, nitems)
     switch (mode) {
-        OHPIC_MX_CASE(kModeFused)
-        OHPIC_MX_CASE(kModeDeposit)
-        OHPIC_MX_CASE(kModeGatherPush)
-        OHPIC_MX_CASE(kModeBoundary)
-        OHPIC_MX_CASE(kModeFusedList)
-        OHPIC_MX_CASE(kModeBoundaryList)
+    case kModeFused:
+        if (ids)
+            OHPIC_MX_CASE(kModeFused, true);
+        else
+            OHPIC_MX_CASE(kModeFused, false);
+        break;
+    case kModeGatherPush:
+        if (ids)
+            OHPIC_MX_CASE(kModeGatherPush, true);
+        else
+            OHPIC_MX_CASE(kModeGatherPush, false);
+        break;
+    case kModeBoundary:
+        if (ids)
+            OHPIC_MX_CASE(kModeBoundary, true);
+        else
+            OHPIC_MX_CASE(kModeBoundary, false);
+        break;
+    case kModeDeposit: OHPIC_MX_CASE(kModeDeposit, false); break;
+    case kModeFusedList: OHPIC_MX_CASE(kModeFusedList, true); break;
+    case kModeBoundaryList: OHPIC_MX_CASE(kModeBoundaryList, true); break;
     default:
         return hipErrorInvalidValue;
     }
@@ -788,55 +885,44 @@ static hipError_t launch_tile_mx(int mode, const InstDev *insts, const WorkItem 
     return hipGetLastError();
 }
 
-hipError_t launch_particles_mixed(int mode, int weight_order, const int T[3],
-                                  const InstDev *insts, const WorkItem *items, int nitems,
-                                  const int *parity, hipStream_t st)
-{
-#define OHPIC_TILE(A, B, C)                                                        \
-    if (T[0] == A && T[1] == B && T[2] == C)                                       \
-        return weight_order == 0                                                   \
-                   ? launch_tile_mx<A, B, C, 0>(mode, insts, items, nitems, parity, st) \
-                   : launch_tile_mx<A, B, C, 1>(mode, insts, items, nitems, parity, st);
-    OHPIC_TILE(4, 4, 4)
-    OHPIC_TILE(8, 8, 8)
-    OHPIC_TILE(8, 8, 4)
-    OHPIC_TILE(16, 8, 4)
-#undef OHPIC_TILE
-    return hipErrorInvalidValue;
-}
-
 template <int TX, int TY, int TZ, int WO>
-static hipError_t launch_tile_mx_queue(const InstDev *insts, const WorkItem *items, int nitems,
-                                       const int *parity, unsigned int *queue, int blocks,
-                                       hipStream_t st)
+static hipError_t launch_tile_mx_queue(bool ids, const InstDev *insts, const WorkItem *items,
+                                    int nitems, const int *parity, unsigned int *queue, int blocks,
+                                    hipStream_t st)
 {
-    hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue>), dim3(blocks),
-                       dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+    if (ids)
+        hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, true>), dim3(blocks),
+                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+    else
+        hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, false>), dim3(blocks),
+                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
     return hipGetLastError();
 }
 
 template <int TX, int TY, int TZ, int WO>
-static int queue_blocks_per_cu_mx()
+static int queue_blocks_per_cu_mx(bool ids)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &nb, reinterpret_cast<const void *>(&k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue>),
-            kBlock, 0) != hipSuccess) {
+    const void *f = ids ? reinterpret_cast<const void *>(
+                              &k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, true>)
+                        : reinterpret_cast<const void *>(
+                              &k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, false>);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, kBlock, 0) != hipSuccess) {
         (void)hipGetLastError();
         nb = 1;
     }
     return nb > 0 ? nb : 1;
 }
 
-hipError_t launch_particles_mixed_queue(int weight_order, const int T[3], const InstDev *insts,
-                                        const WorkItem *items, int nitems, const int *parity,
-                                        unsigned int *queue, int blocks, hipStream_t st)
+hipError_t launch_particles_mixed(int mode, int weight_order, const int T[3], bool ids,
+                                  const InstDev *insts, const WorkItem *items, int nitems,
+                                  const int *parity, hipStream_t st)
 {
-#define OHPIC_TILE(A, B, C)                                                                   \
-    if (T[0] == A && T[1] == B && T[2] == C)                                                  \
-        return weight_order == 0                                                              \
-                   ? launch_tile_mx_queue<A, B, C, 0>(insts, items, nitems, parity, queue, blocks, st) \
-                   : launch_tile_mx_queue<A, B, C, 1>(insts, items, nitems, parity, queue, blocks, st);
+#define OHPIC_TILE(A, B, C)                                                                  \
+    if (T[0] == A && T[1] == B && T[2] == C)                                                 \
+        return weight_order == 0                                                             \
+                   ? launch_tile_mx<A, B, C, 0>(mode, ids, insts, items, nitems, parity, st) \
+                   : launch_tile_mx<A, B, C, 1>(mode, ids, insts, items, nitems, parity, st);
     OHPIC_TILE(4, 4, 4)
     OHPIC_TILE(8, 8, 8)
     OHPIC_TILE(8, 8, 4)
@@ -845,12 +931,31 @@ hipError_t launch_particles_mixed_queue(int weight_order, const int T[3], const 
     return hipErrorInvalidValue;
 }
 
-int particles_mixed_queue_blocks(int weight_order, const int T[3])
+hipError_t launch_particles_mixed_queue(int weight_order, const int T[3], bool ids,
+                                        const InstDev *insts, const WorkItem *items, int nitems,
+                                        const int *parity, unsigned int *queue, int blocks,
+                                        hipStream_t st)
 {
-#define OHPIC_TILE(A, B, C)                                                            \
-    if (T[0] == A && T[1] == B && T[2] == C)                                           \
-        return weight_order == 0 ? queue_blocks_per_cu_mx<A, B, C, 0>()                \
-                                 : queue_blocks_per_cu_mx<A, B, C, 1>();
+#define OHPIC_TILE(A, B, C)                                                                       \
+    if (T[0] == A && T[1] == B && T[2] == C)                                                      \
+        return weight_order == 0 ? launch_tile_mx_queue<A, B, C, 0>(ids, insts, items, nitems,    \
+                                                                    parity, queue, blocks, st)    \
+                                 : launch_tile_mx_queue<A, B, C, 1>(ids, insts, items, nitems,    \
+                                                                    parity, queue, blocks, st);
+    OHPIC_TILE(4, 4, 4)
+    OHPIC_TILE(8, 8, 8)
+    OHPIC_TILE(8, 8, 4)
+    OHPIC_TILE(16, 8, 4)
+#undef OHPIC_TILE
+    return hipErrorInvalidValue;
+}
+
+int particles_mixed_queue_blocks(int weight_order, const int T[3], bool ids)
+{
+#define OHPIC_TILE(A, B, C)                                                      \
+    if (T[0] == A && T[1] == B && T[2] == C)                                     \
+        return weight_order == 0 ? queue_blocks_per_cu_mx<A, B, C, 0>(ids)       \
+                                 : queue_blocks_per_cu_mx<A, B, C, 1>(ids);
     OHPIC_TILE(4, 4, 4)
     OHPIC_TILE(8, 8, 8)
     OHPIC_TILE(8, 8, 4)
