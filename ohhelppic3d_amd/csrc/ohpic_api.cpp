@@ -260,21 +260,25 @@ struct TileLoad {
     int64_t load;  // bin slots over all species
 };
 
-// A chunk costs about as much as 2K particles (its E tile, charge block and
-// closing), so none is made smaller than this many slots.
-constexpr int64_t kMinChunkLoad = 4096;
+// No chunk is made smaller than this many slots: it costs an E tile, a charge
+// flush and a part in the closing launch (tiles of 9.4K slots in 2 chunks: 32^3
+// x 64 ppc mixed 124 us per launch, whole 88 us).
+constexpr int64_t kMinChunkLoad = 8192;
 
 // Chunks per tile (nch[i] of tiles[i]) and the order the tiles are dispatched
 // in, for `slots` workgroups resident at once: heaviest first (in steps of an
-// eighth of an octave, tiles of one step in grid order), each tile whole while
-// a share of the work still to come, R / slots, is no smaller than it, else
-// split into that many shares.  A grid with fewer tiles than workgroups is
-// thereby spread over the device, a tile far above the mean (a density hump)
-// does not outlast the others, and the last tiles of a launch end together.
-// At most max_extra items beyond one per tile.  Every further item costs its
-// E tile and charge flush: a group of 32 members of 16^3-64^3, each split as
-// if it ran alone (62936 items), took 3.01 ms per particle launch, planned as
-// one (8008 items) 1.47 ms.
+// eighth of an octave, tiles of one step in grid order).  A tile stays whole
+// unless it would outlast the launch: split are the tiles of a grid with less
+// than a quarter as many tiles as workgroups, so that they fill the device
+// (16^3 x 200 ppc: 169 -> 149 us mixed, 189 -> 158 us FP64; with half as many,
+// 32^3 x 300 ppc mixed, whole tiles are faster, 317 against 363 us), and tiles
+// at least twice as heavy as the mean that hold at least a workgroup's
+// fair share of the work (a density peak).  Splitting further, so that the
+// last tiles of a launch end together, costs more than it gives (80x72x88 x 20
+// ppc mixed: 317 us per launch against 280).  At most max_extra items beyond
+// one per tile.  A group is planned as one: 32 members of 16^3-64^3, each
+// split as if it ran alone (62936 items), took 3.01 ms per particle launch,
+// planned together (5472 items) 1.4 ms.
 void plan_chunks(std::vector<TileLoad> &tiles, int64_t slots, int64_t max_extra,
                  std::vector<int> &nch)
 {
@@ -282,18 +286,17 @@ void plan_chunks(std::vector<TileLoad> &tiles, int64_t slots, int64_t max_extra,
     std::stable_sort(tiles.begin(), tiles.end(), [&](const TileLoad &a, const TileLoad &b) {
         return level(a.load) > level(b.load);
     });
-    int64_t rest = 0, made = 0, extra = 0;
-    for (const TileLoad &t : tiles) rest += t.load;
     nch.assign(tiles.size(), 1);
-    int64_t share = rest / slots;
+    if (tiles.empty()) return;
+    int64_t work = 0, extra = 0;
+    for (const TileLoad &t : tiles) work += t.load;
+    const int64_t share = work / slots, nt = (int64_t)tiles.size();
+    const int64_t unit = std::max(
+        kMinChunkLoad, 4 * nt <= slots ? share : std::max(share / 2, work / nt));
     for (size_t i = 0; i < tiles.size(); ++i) {
-        // the first `slots` items start together; later ones as earlier ones end
-        if (made >= slots) share = rest / slots;
-        const int64_t want = tiles[i].load / std::max(share, kMinChunkLoad);
+        const int64_t want = tiles[i].load / unit;
         nch[i] = (int)std::max<int64_t>(1, std::min<int64_t>({want, 1 + max_extra - extra, 256}));
         extra += nch[i] - 1;
-        made += nch[i];
-        rest -= tiles[i].load;
     }
 }
 

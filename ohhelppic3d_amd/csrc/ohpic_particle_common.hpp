@@ -16,7 +16,6 @@ namespace {
 #define OHPIC_PUSH_MIN_WAVES 1
 #endif
 
-constexpr int kWaves = kBlock / 64;
 constexpr int kLeaveCap = 32;  // per-wave buffer of particles that left the tile
 constexpr int kStash = 64;     // per-wave stash of particles that stayed (below)
 
@@ -129,24 +128,22 @@ __device__ __forceinline__ unsigned long long lane_bcast(unsigned long long v, i
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// Particle state streams through each step once: with OHPIC_NT set, its
-// loads and stores carry the non-temporal hint (measured 3-7% slower on the
-// 256^3 x 64 ppc step, so off by default).
-#ifndef OHPIC_NT
-#define OHPIC_NT 0
-#endif
-
+// Particle state streams through each step once, so its full-line accesses
+// carry the non-temporal hint: 256^3 x 32 ppc mixed 11.82 -> 10.91 ms per
+// launch, 256^3 x 16 FP64 11.14 -> 10.85 ms, and the field kernels of smaller
+// grids find their arrays in the last-level cache (the 32^3 x 16 push loses
+// 1 us, its field solve gains 1.5 us).  Partial lines (leavers, the ends of
+// runs) are stored without it: they are merged in L2.
 template <typename T>
 __device__ __forceinline__ T sload(const T *p, int64_t i)
 {
-    if (OHPIC_NT) return __builtin_nontemporal_load(&as_global(p)[i]);
-    return as_global(p)[i];
+    return __builtin_nontemporal_load(&as_global(p)[i]);
 }
 
-template <typename T>
+template <bool NT, typename T>
 __device__ __forceinline__ void sstore(T *p, int64_t i, T v)
 {
-    if (OHPIC_NT)
+    if (NT)
         __builtin_nontemporal_store(v, &as_global(p)[i]);
     else
         as_global(p)[i] = v;
@@ -241,14 +238,15 @@ __device__ __forceinline__ void publish_front(const InstDev *__restrict__ I, con
         gatomic_add(&S.count[nbuf][tile], (unsigned long long)(-(long long)(cnt - m)));
 }
 
-// The item's kinetic-energy partials, summed over its wavefronts in order.
+// The item's kinetic-energy partials, summed over its W wavefronts in order.
+template <int W>
 __device__ __forceinline__ void write_ke(const InstDev *__restrict__ I, const WorkItem &it, int tid,
-                                         int ns, const double (*ke)[kWaves])
+                                         int ns, const double (*ke)[W])
 {
     if (tid >= 2 * ns) return;
     const int s = tid >> 1, k = (tid & 1) ? kMaxSpecies + s : s;
     double v = 0.0;
-    for (int w = 0; w < kWaves; ++w) v += ke[k][w];
+    for (int w = 0; w < W; ++w) v += ke[k][w];
     gstore(I->ke_partial, (int64_t)k * I->nitems + it.slot, 0.5 * I->sp[s].mass * v);
 }
 

@@ -17,7 +17,7 @@
 // The LDS charge block is flushed with one global 64-bit atomic per node.
 // Integer accumulation makes rho independent of particle order and timing.
 //
-// What bounds it: large grids stream 96 B per particle, at 4.7 TB/s of the 5.2
+// What bounds it: large grids stream 96 B per particle, at 4.75 TB/s of the 5.2
 // TB/s a bare copy of the same shape reaches; the rest is per tile (E tile,
 // charge flush, the leavers' atomics).  Small grids wait: so every load of an
 // item's start is issued before the first is used, nothing in the particle
@@ -46,12 +46,12 @@ struct P64 {
 __device__ __forceinline__ void store_p64(const SpecDev &S, int nbuf, int64_t o, const P64 &p,
                                           bool ids)
 {
-    sstore((double *)S.buf[nbuf][0], o, p.x);
-    sstore((double *)S.buf[nbuf][1], o, p.y);
-    sstore((double *)S.buf[nbuf][2], o, p.z);
-    sstore((double *)S.buf[nbuf][3], o, p.vx);
-    sstore((double *)S.buf[nbuf][4], o, p.vy);
-    sstore((double *)S.buf[nbuf][5], o, p.vz);
+    gstore((double *)S.buf[nbuf][0], o, p.x);
+    gstore((double *)S.buf[nbuf][1], o, p.y);
+    gstore((double *)S.buf[nbuf][2], o, p.z);
+    gstore((double *)S.buf[nbuf][3], o, p.vx);
+    gstore((double *)S.buf[nbuf][4], o, p.vy);
+    gstore((double *)S.buf[nbuf][5], o, p.vz);
     if (ids) gstore(S.pid[nbuf], o, p.id);
 }
 
@@ -100,16 +100,18 @@ __device__ __forceinline__ P64 load_bin64(const BinView64 &bv, uint32_t slot, bo
     return q;
 }
 
+// FULL: the wavefront stores full lines
+template <bool FULL>
 __device__ __forceinline__ void store_bin64(const BinView64 &bv, uint32_t slot, const P64 &q,
                                             bool ids)
 {
     const uint32_t off = slot * 8u;
-    sstore((double *)(bv.c[0] + off), 0, q.x);
-    sstore((double *)(bv.c[1] + off), 0, q.y);
-    sstore((double *)(bv.c[2] + off), 0, q.z);
-    sstore((double *)(bv.c[3] + off), 0, q.vx);
-    sstore((double *)(bv.c[4] + off), 0, q.vy);
-    sstore((double *)(bv.c[5] + off), 0, q.vz);
+    sstore<FULL>((double *)(bv.c[0] + off), 0, q.x);
+    sstore<FULL>((double *)(bv.c[1] + off), 0, q.y);
+    sstore<FULL>((double *)(bv.c[2] + off), 0, q.z);
+    sstore<FULL>((double *)(bv.c[3] + off), 0, q.vx);
+    sstore<FULL>((double *)(bv.c[4] + off), 0, q.vy);
+    sstore<FULL>((double *)(bv.c[5] + off), 0, q.vz);
     if (ids) gstore(const_cast<int64_t *>(bv.id), (int64_t)slot, q.id);
 }
 
@@ -185,10 +187,14 @@ __device__ __forceinline__ void flush_leavers(const Buf64<IDS, kLeaveCap> &lb, i
     wave_sync();
 }
 
+// Threads per workgroup, for every tile shape (kept beside mx_block: 512 for
+// 512-cell tiles measured 1.20 against 1.15 ms at 96^3 x 32 ppc).
+constexpr int fp_block(int) { return kBlock; }
+
 // IDS: instances may keep particle ids (each instance's track_ids says whether
 // it does); without it no register, LDS or branch is spent on them.
 template <int TX, int TY, int TZ, int WO, int MODE_, bool IDS>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(fp_block(TX *TY *TZ))
     __attribute__((amdgpu_waves_per_eu(OHPIC_PUSH_MIN_WAVES, 8)))
     k_particles_fp64(const InstDev *__restrict__ insts, const WorkItem *__restrict__ items,
                      const int *__restrict__ parity, unsigned int *__restrict__ queue,
@@ -205,6 +211,7 @@ __global__ void __launch_bounds__(kBlock)
     constexpr bool BINS = REBIN && !LIST;
     constexpr int EX = TX + 1, EY = TY + 1, EZ = TZ + 1, NE = EX * EY * EZ;
     constexpr int RX = TX + 3, RY = TY + 3, RZ = TZ + 3, NR = RX * RY * RZ;
+    constexpr int kThreads = fp_block(TX * TY * TZ), kWaves = kThreads / 64;
     __shared__ double sE[PUSH ? 3 * NE : 1];
     __shared__ unsigned long long sR[DEP ? NR : 1];
     __shared__ Buf64<IDS, kLeaveCap> sLeave[BINS ? kWaves : 1];
@@ -247,12 +254,12 @@ __global__ void __launch_bounds__(kBlock)
 
         // every load of the E tile and of the species' bin words is issued
         // before the first one is used
-        constexpr int KE = PUSH ? (NE + kBlock - 1) / kBlock : 1;
+        constexpr int KE = PUSH ? (NE + kThreads - 1) / kThreads : 1;
         double ev[3][KE];
         if (PUSH) {
 #pragma unroll
             for (int k = 0; k < KE; ++k) {
-                const int l = min(tid + k * kBlock, NE - 1);
+                const int l = min(tid + k * kThreads, NE - 1);
                 const int lx = l % EX, ly = (l / EX) % EY, lz = l / (EX * EY);
                 const int gx = wrap_near(lox + lx, nx), gy = wrap_near(loy + ly, ny),
                           gz = wrap_near(loz + lz, nz);
@@ -264,11 +271,11 @@ __global__ void __launch_bounds__(kBlock)
         load_meta<LIST>(sMeta, I, it, par, tid, ns);
         if (BINS && tid < kMaxSpecies) sBlk[tid] = 0;
         if (DEP)
-            for (int l = tid; l < NR; l += kBlock) sR[l] = 0ull;
+            for (int l = tid; l < NR; l += kThreads) sR[l] = 0ull;
         if (PUSH) {
 #pragma unroll
             for (int k = 0; k < KE; ++k) {
-                const int l = tid + k * kBlock;
+                const int l = tid + k * kThreads;
                 if (l < NE) {
 #pragma unroll
                     for (int a = 0; a < 3; ++a) sE[a * NE + l] = ev[a][k];
@@ -316,13 +323,13 @@ __global__ void __launch_bounds__(kBlock)
             P64 nextq{0, 0, 0, 0, 0, 0, 0};
             if (start + tid < end)
                 nextq = load_bin64(cur, (uint32_t)bin_slot(start + tid, F, B, cap), ids);
-            for (int p0 = start; p0 < end; p0 += kBlock) {
+            for (int p0 = start; p0 < end; p0 += kThreads) {
                 const int p = p0 + tid;
                 const bool active = p < end;
                 P64 q = nextq;
                 // prefetch the next iteration's particle while this one is processed
-                if (p + kBlock < end)
-                    nextq = load_bin64(cur, (uint32_t)bin_slot(p + kBlock, F, B, cap), ids);
+                if (p + kThreads < end)
+                    nextq = load_bin64(cur, (uint32_t)bin_slot(p + kThreads, F, B, cap), ids);
                 if (PUSH && active) {
                     const int ix = (int)q.x, iy = (int)q.y, iz = (int)q.z;
                     double wx0, wx1, wy0, wy1, wz0, wz1;
@@ -370,7 +377,7 @@ __global__ void __launch_bounds__(kBlock)
                     q.z = q.z + q.vz * dt;
                 }
                 if (MODE == kModeGatherPush) {
-                    if (active) store_bin64(cur, (uint32_t)bin_slot(p, F, B, cap), q, ids);
+                    if (active) store_bin64<true>(cur, (uint32_t)bin_slot(p, F, B, cap), q, ids);
                     continue;
                 }
                 // a particle still in its tile needs no wrap and no new tile
@@ -475,7 +482,7 @@ __global__ void __launch_bounds__(kBlock)
                 } else if (block) {
                     wave_sync();
                     if (!stay) sStash[wv].get(sc + lane_rank(~sm), q, ids);
-                    store_bin64(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                    store_bin64<true>(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
                 } else if (nst > 0) {
                     wave_sync();
                     if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
@@ -497,7 +504,7 @@ __global__ void __launch_bounds__(kBlock)
                 if (lane < sc) {
                     P64 q;
                     sStash[wv].get(lane, q, ids);
-                    store_bin64(nxt, (uint32_t)(o + lane), q, ids);
+                    store_bin64<false>(nxt, (uint32_t)(o + lane), q, ids);
                 }
                 wave_sync();
                 if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
@@ -513,10 +520,10 @@ __global__ void __launch_bounds__(kBlock)
         }
 
         __syncthreads();
-        if (PUSH) write_ke(I, it, tid, ns, sKe);
+        if (PUSH) write_ke<kWaves>(I, it, tid, ns, sKe);
         if (DEP) {
             unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
-            for (int l = tid; l < NR; l += kBlock) {
+            for (int l = tid; l < NR; l += kThreads) {
                 const unsigned long long v = sR[l];
                 if (v == 0ull) continue;
                 const int lx = l % RX, ly = (l / RX) % RY, lz = l / (RX * RY);
@@ -651,7 +658,7 @@ template <int TX, int TY, int TZ, int WO>
 static hipError_t launch_tile(int mode, bool ids, const InstDev *insts, const WorkItem *items,
                               int nitems, const int *parity, hipStream_t st)
 {
-    dim3 g(nitems), b(kBlock);
+    dim3 g(nitems), b(fp_block(TX * TY * TZ));
 #define OHPIC_FP_CASE(M, IDS)                                                                     \
     hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, M, IDS>), g, b, 0, st, insts, items, parity, \
                        nullptr, nitems)
@@ -691,10 +698,10 @@ static hipError_t launch_tile_queue(bool ids, const InstDev *insts, const WorkIt
 {
     if (ids)
         hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, true>), dim3(blocks),
-                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+                           dim3(fp_block(TX * TY * TZ)), 0, st, insts, items, parity, queue, nitems);
     else
         hipLaunchKernelGGL((k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, false>), dim3(blocks),
-                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+                           dim3(fp_block(TX * TY * TZ)), 0, st, insts, items, parity, queue, nitems);
     return hipGetLastError();
 }
 
@@ -706,7 +713,7 @@ static int queue_blocks_per_cu(bool ids)
                               &k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, true>)
                         : reinterpret_cast<const void *>(
                               &k_particles_fp64<TX, TY, TZ, WO, kModeFusedQueue, false>);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, kBlock, 0) != hipSuccess) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, fp_block(TX * TY * TZ), 0) != hipSuccess) {
         (void)hipGetLastError();
         nb = 1;
     }

@@ -127,13 +127,15 @@ __device__ __forceinline__ PMx load_bin(const BinView &bv, uint32_t slot, bool i
     return q;
 }
 
+// FULL: the wavefront stores full lines
+template <bool FULL>
 __device__ __forceinline__ void store_bin(const BinView &bv, uint32_t slot, const PMx &q, bool ids)
 {
     const uint32_t off = slot * 4u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        sstore((uint32_t *)(bv.w[a] + off), 0, q.w[a]);
-        sstore((float *)(bv.v[a] + off), 0, q.v[a]);
+        sstore<FULL>((uint32_t *)(bv.w[a] + off), 0, q.w[a]);
+        sstore<FULL>((float *)(bv.v[a] + off), 0, q.v[a]);
     }
     if (ids) gstore(const_cast<int64_t *>(bv.id), (int64_t)slot, q.id);
 }
@@ -256,10 +258,18 @@ __device__ __forceinline__ void flush_leavers_mx(const BufMx<IDS, kLeaveCap> &lb
     wave_sync();
 }
 
+// Threads per workgroup: 512 for tiles of 512 cells, 256 for smaller ones.  Two
+// large workgroups per CU share their E tile and charge block among twice the
+// wavefronts and end a launch's last tiles sooner (8^3 tiles: 64^3 x 32 ppc
+// 247 -> 223 us per launch, 128^3 x 64 with a density peak 3.10 -> 2.76 ms,
+// 256^3 x 32 10.91 -> 10.78 ms); a small tile has too little work for them
+// (8x8x4 tiles of a group of 32: 12.5 ms per 8 steps with 256, 15.6 with 512).
+constexpr int mx_block(int cells) { return cells >= 512 ? 512 : 256; }
+
 // IDS: instances may keep particle ids (each instance's track_ids says whether
 // it does); without it no register, LDS or branch is spent on them.
 template <int TX, int TY, int TZ, int WO, int MODE_, bool IDS>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(mx_block(TX *TY *TZ))
     __attribute__((amdgpu_waves_per_eu((MODE_ == kModeFusedQueue && IDS) ? 4 : OHPIC_MX_MIN_WAVES, 8)))
     k_particles_mixed(const InstDev *__restrict__ insts, const WorkItem *__restrict__ items,
                       const int *__restrict__ parity, unsigned int *__restrict__ queue,
@@ -281,6 +291,7 @@ __global__ void __launch_bounds__(kBlock)
     // and one 2x32-bit LDS load at constant offsets from the particle's base
     // node (measured 3% faster per step than 16-byte nodes, whose loads share
     // fewer LDS banks, and than three separate arrays)
+    constexpr int kThreads = mx_block(TX * TY * TZ), kWaves = kThreads / 64;
     __shared__ float2 sExy[PUSH ? NE : 1];
     __shared__ float sEz[PUSH ? NE : 1];
     __shared__ unsigned long long sR[DEP ? NR : 1];
@@ -324,12 +335,12 @@ __global__ void __launch_bounds__(kBlock)
 
         // every load of the E tile and of the species' bin words is issued
         // before the first one is used
-        constexpr int KE = PUSH ? (NE + kBlock - 1) / kBlock : 1;
+        constexpr int KE = PUSH ? (NE + kThreads - 1) / kThreads : 1;
         double ev[3][KE];
         if (PUSH) {
 #pragma unroll
             for (int k = 0; k < KE; ++k) {
-                const int l = min(tid + k * kBlock, NE - 1);
+                const int l = min(tid + k * kThreads, NE - 1);
                 const int lx = l % EX, ly = (l / EX) % EY, lz = l / (EX * EY);
                 const int gx = wrap_near(lox + lx, nx), gy = wrap_near(loy + ly, ny),
                           gz = wrap_near(loz + lz, nz);
@@ -341,11 +352,11 @@ __global__ void __launch_bounds__(kBlock)
         load_meta<LIST>(sMeta, I, it, par, tid, ns);
         if (BINS && tid < kMaxSpecies) sBlk[tid] = 0;
         if (DEP)
-            for (int l = tid; l < NR; l += kBlock) sR[l] = 0ull;
+            for (int l = tid; l < NR; l += kThreads) sR[l] = 0ull;
         if (PUSH) {
 #pragma unroll
             for (int k = 0; k < KE; ++k) {
-                const int l = tid + k * kBlock;
+                const int l = tid + k * kThreads;
                 if (l < NE) {
                     sExy[l] = make_float2((float)ev[0][k], (float)ev[1][k]);
                     sEz[l] = (float)ev[2][k];
@@ -393,19 +404,19 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
             for (int k = 0; k < kMxPrefetch; ++k) {
                 ahead[k] = PMx{{0u, 0u, 0u}, {0.0f, 0.0f, 0.0f}, 0};
-                if (start + tid + k * kBlock < end)
-                    ahead[k] = load_bin(cur, (uint32_t)bin_slot(start + tid + k * kBlock, F, B, cap),
+                if (start + tid + k * kThreads < end)
+                    ahead[k] = load_bin(cur, (uint32_t)bin_slot(start + tid + k * kThreads, F, B, cap),
                                         ids);
             }
-            for (int p0 = start; p0 < end; p0 += kBlock) {
+            for (int p0 = start; p0 < end; p0 += kThreads) {
                 const int p = p0 + tid;
                 const bool active = p < end;
                 PMx q = ahead[0];
 #pragma unroll
                 for (int k = 0; k + 1 < kMxPrefetch; ++k) ahead[k] = ahead[k + 1];
-                if (p + kMxPrefetch * kBlock < end)
+                if (p + kMxPrefetch * kThreads < end)
                     ahead[kMxPrefetch - 1] =
-                        load_bin(cur, (uint32_t)bin_slot(p + kMxPrefetch * kBlock, F, B, cap), ids);
+                        load_bin(cur, (uint32_t)bin_slot(p + kMxPrefetch * kThreads, F, B, cap), ids);
                 // cell relative to this tile's origin and in-cell offset per axis
                 int rx = pos_rel(q.w[0]), ry = pos_rel(q.w[1]), rz = pos_rel(q.w[2]);
                 float ox = pos_frac(q.w[0]), oy = pos_frac(q.w[1]), oz = pos_frac(q.w[2]);
@@ -485,7 +496,7 @@ __global__ void __launch_bounds__(kBlock)
                     oz = pos_frac(q.w[2]);
                     if (MODE == kModeGatherPush) {
                         // not re-binned: the cell stays relative to this tile
-                        store_bin(cur, (uint32_t)bin_slot(p, F, B, cap), q, ids);
+                        store_bin<true>(cur, (uint32_t)bin_slot(p, F, B, cap), q, ids);
                     }
                 }
                 if (MODE == kModeGatherPush) continue;
@@ -602,7 +613,7 @@ __global__ void __launch_bounds__(kBlock)
                     }
                 } else if (block) {
                     if (!stay) q = fill;
-                    store_bin(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                    store_bin<true>(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
                 } else if (nst > 0) {
                     wave_sync();
                     if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
@@ -624,7 +635,7 @@ __global__ void __launch_bounds__(kBlock)
                 if (lane < sc) {
                     PMx q;
                     sStash[wv].get(lane, q, ids);
-                    store_bin(nxt, (uint32_t)(o + lane), q, ids);
+                    store_bin<false>(nxt, (uint32_t)(o + lane), q, ids);
                 }
                 wave_sync();
                 if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
@@ -640,10 +651,10 @@ __global__ void __launch_bounds__(kBlock)
         }
 
         __syncthreads();
-        if (PUSH) write_ke(I, it, tid, ns, sKe);
+        if (PUSH) write_ke<kWaves>(I, it, tid, ns, sKe);
         if (DEP) {
             unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
-            for (int l = tid; l < NR; l += kBlock) {
+            for (int l = tid; l < NR; l += kThreads) {
                 const unsigned long long v = sR[l];
                 if (v == 0ull) continue;
                 const int lx = l % RX, ly = (l / RX) % RY, lz = l / (RX * RY);
@@ -852,7 +863,7 @@ template <int TX, int TY, int TZ, int WO>
 static hipError_t launch_tile_mx(int mode, bool ids, const InstDev *insts, const WorkItem *items,
                               int nitems, const int *parity, hipStream_t st)
 {
-    dim3 g(nitems), b(kBlock);
+    dim3 g(nitems), b(mx_block(TX * TY * TZ));
 #define OHPIC_MX_CASE(M, IDS)                                                                     \
     hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, M, IDS>), g, b, 0, st, insts, items, parity, \
                        nullptr, nitems)
@@ -892,10 +903,10 @@ static hipError_t launch_tile_mx_queue(bool ids, const InstDev *insts, const Wor
 {
     if (ids)
         hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, true>), dim3(blocks),
-                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+                           dim3(mx_block(TX * TY * TZ)), 0, st, insts, items, parity, queue, nitems);
     else
         hipLaunchKernelGGL((k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, false>), dim3(blocks),
-                           dim3(kBlock), 0, st, insts, items, parity, queue, nitems);
+                           dim3(mx_block(TX * TY * TZ)), 0, st, insts, items, parity, queue, nitems);
     return hipGetLastError();
 }
 
@@ -907,7 +918,7 @@ static int queue_blocks_per_cu_mx(bool ids)
                               &k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, true>)
                         : reinterpret_cast<const void *>(
                               &k_particles_mixed<TX, TY, TZ, WO, kModeFusedQueue, false>);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, kBlock, 0) != hipSuccess) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, mx_block(TX * TY * TZ), 0) != hipSuccess) {
         (void)hipGetLastError();
         nb = 1;
     }
