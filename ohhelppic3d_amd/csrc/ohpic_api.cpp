@@ -469,13 +469,14 @@ hipError_t run_particles(ohpic_ctx *ctx, int mode)
 int set_bins(ohpic_ctx *ctx, int s, const std::vector<int64_t> &counts)
 {
     SpeciesHost &S = ctx->sp[s];
-    const double slack = config_slack(ctx->cfg);
     const int nt = ctx->ntiles;
+    const std::vector<int64_t> caps =
+        bin_capacities(counts, ctx->nt, config_slack(ctx->cfg), S.alloc);
     S.base.assign(nt, 0);
     S.cap.assign(nt, 0);
     int64_t off = 0;
     for (int t = 0; t < nt; ++t) {
-        const int64_t cap = bin_capacity(counts[t], slack);
+        const int64_t cap = caps[t];
         if (cap >= kBinCapLimit)
             return fail(ctx, OHPIC_ENOMEM, "bin %d needs %lld slots (limit 2^29): use smaller tiles",
                         t, (long long)cap);
@@ -662,7 +663,6 @@ int compact_bins(ohpic_ctx *ctx)
 {
     timer_begin(ctx, 5);
     const int nt = ctx->ntiles, par = ctx->par;
-    const double slack = config_slack(ctx->cfg);
     int rc;
     for (int s = 0; s < ctx->cfg.nspecies; ++s) {
         if ((int)ctx->sp[s].cap.size() != nt) continue;
@@ -670,13 +670,13 @@ int compact_bins(ohpic_ctx *ctx)
         if ((rc = download_words(ctx, ctx->h.sp[s].count[par], F, B))) return rc;
         std::vector<int64_t> used(nt), off(nt);
         std::vector<unsigned long long> words(nt);
-        int64_t o = 0;
         for (int t = 0; t < nt; ++t) {
             used[t] = F[t] + B[t];
             words[t] = (unsigned long long)used[t];  // one front run
-            off[t] = o;
-            o += bin_capacity(used[t], slack);
         }
+        const std::vector<int64_t> caps =
+            bin_capacities(used, ctx->nt, config_slack(ctx->cfg), ctx->sp[s].alloc);
+        for (int64_t t = 0, o = 0; t < nt; o += caps[t++]) off[t] = o;
         HIPCHK(ctx, hipMemcpyAsync(ctx->d_tmp64, off.data(), nt * sizeof(int64_t),
                                    hipMemcpyHostToDevice, ctx->st));
         // the copy reads the current layout; set_bins then uploads the new one
