@@ -133,8 +133,7 @@ struct ohpic_ctx {
     double *d_lam[3]{};
     FftJob job{};                // Poisson transform of rho into phi
     FftJob *d_job = nullptr;
-    int64_t fft_grp[3]{};        // workgroups per axis pass
-    int fft_rs[3]{};             // radix set per axis
+    FftLaunch fft[3];            // launches of each axis' passes
     std::vector<WorkItem> items;  // host copy of d_items
     uint64_t inst_ver = 0;       // bumped whenever h is uploaded
     uint64_t items_ver = 0;      // bumped whenever the work list changes
@@ -798,15 +797,14 @@ int do_deposit(ohpic_ctx *ctx)
 // Poisson solve of the instance table `insts` (n instances, FFT jobs `jobs`)
 // from rho: five axis passes, node E and its energy partials (reduced when
 // reduce_e).
-hipError_t solve_passes(const FftJob *jobs, const InstDev *insts, int n, const int64_t grp[3],
-                        const int rs[3], int z256, int max_eblocks, bool reduce_e,
-                        hipStream_t st)
+hipError_t solve_passes(const FftJob *jobs, const InstDev *insts, int n, const FftLaunch fft[3],
+                        int max_eblocks, bool reduce_e, hipStream_t st)
 {
-    hipError_t e = fft_pass(kPassR2hcXFromSrc, jobs, n, grp[0], rs[0], st);
-    if (e == hipSuccess) e = fft_pass(kPassR2hcY, jobs, n, grp[1], rs[1], st);
-    if (e == hipSuccess) e = fft_poisson_z(jobs, n, grp[2], rs[2], z256, st);
-    if (e == hipSuccess) e = fft_pass(kPassHc2rY, jobs, n, grp[1], rs[1], st);
-    if (e == hipSuccess) e = fft_pass(kPassHc2rXScaled, jobs, n, grp[0], rs[0], st);
+    hipError_t e = fft_pass(kPassR2hcXFromSrc, jobs, n, fft[0], st);
+    if (e == hipSuccess) e = fft_pass(kPassR2hcY, jobs, n, fft[1], st);
+    if (e == hipSuccess) e = fft_pass(kPassPoissonZ, jobs, n, fft[2], st);
+    if (e == hipSuccess) e = fft_pass(kPassHc2rY, jobs, n, fft[1], st);
+    if (e == hipSuccess) e = fft_pass(kPassHc2rXScaled, jobs, n, fft[0], st);
     if (e == hipSuccess) e = launch_efield_b(insts, n, max_eblocks, reduce_e, st);
     return e;
 }
@@ -816,9 +814,8 @@ hipError_t solve_passes(const FftJob *jobs, const InstDev *insts, int n, const i
 int do_solve(ohpic_ctx *ctx, bool reduce_e)
 {
     timer_begin(ctx, 1);
-    HIPCHK(ctx, solve_passes(ctx->d_job, ctx->d_inst, 1, ctx->fft_grp, ctx->fft_rs,
-                             ctx->n[2] == 256 ? kZ256All : kZ256None, efield_blocks_of(ctx->n[0], ctx->n[1], ctx->n[2]), reduce_e,
-                             ctx->st));
+    HIPCHK(ctx, solve_passes(ctx->d_job, ctx->d_inst, 1, ctx->fft,
+                             efield_blocks_of(ctx->n[0], ctx->n[1], ctx->n[2]), reduce_e, ctx->st));
     timer_end(ctx, 1);
     return OHPIC_OK;
 }
@@ -1043,9 +1040,7 @@ struct ohpic_group {
     bool dirty = true;
     int64_t max_ng = 0;
     int max_ntiles = 0, max_rows = 0;  // max_rows: largest E-kernel block count
-    int z256 = kZ256None;              // members whose Poisson z pass has 256-point lines
-    int64_t grp[3]{};
-    int rs[3]{};
+    FftLaunch fft[3];
     int T[3]{};
     int precision = -1, weight_order = -1;
     bool use_graph = true;
@@ -1205,11 +1200,7 @@ int group_refresh(ohpic_group *g)
         if (rc) return rc;
         g->max_ng = 0;
         g->max_ntiles = g->max_rows = 0;
-        int n256 = 0;
-        for (int a = 0; a < 3; ++a) {
-            g->grp[a] = 0;
-            g->rs[a] = 0;
-        }
+        for (FftLaunch &l : g->fft) l = FftLaunch();
         for (int i = 0; i < n; ++i) {
             ohpic_ctx *m = g->members[i];
             insts[i] = m->h;
@@ -1218,15 +1209,10 @@ int group_refresh(ohpic_group *g)
             g->max_ng = std::max(g->max_ng, m->ng);
             g->max_ntiles = std::max(g->max_ntiles, m->ntiles);
             g->max_rows = std::max(g->max_rows, efield_blocks_of(m->n[0], m->n[1], m->n[2]));
-            n256 += m->n[2] == 256;
-            for (int a = 0; a < 3; ++a) {
-                g->grp[a] = std::max(g->grp[a], m->fft_grp[a]);
-                g->rs[a] = std::max(g->rs[a], m->fft_rs[a]);
-            }
+            for (int a = 0; a < 3; ++a) fft_add(g->fft[a], m->ax[a], a, m->n[0], m->n[1], m->n[2]);
             g->seen_inst[i] = m->inst_ver;
             g->seen_items[i] = m->items_ver;
         }
-        g->z256 = n256 == 0 ? kZ256None : (n256 == n ? kZ256All : kZ256Some);
         g->nitems = (int)items.size();
         g->nclose = (int)close.size();
         if (n > 0) {
@@ -1271,8 +1257,7 @@ hipError_t group_enqueue(ohpic_group *g, int k)
         e = launch_begin_step_b(g->d_insts, g->d_parity, n, g->max_ng, g->max_ntiles,
                                 g->persistent ? g->d_queue : nullptr, g->st);
         if (e == hipSuccess)
-            e = solve_passes(g->d_jobs, g->d_insts, n, g->grp, g->rs, g->z256, g->max_rows, false,
-                             g->st);
+            e = solve_passes(g->d_jobs, g->d_insts, n, g->fft, g->max_rows, false, g->st);
         if (e == hipSuccess) {
             if (g->persistent)
                 e = launch_particles_queue(g->precision, g->weight_order, g->T, g->ids, g->d_insts,
@@ -1687,8 +1672,7 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
             J.n[a] = ctx->n[a];
             J.ax[a] = ctx->ax[a];
             J.lam[a] = ctx->d_lam[a];
-            ctx->fft_grp[a] = fft_groups(a, fft_group_lines(ctx->n[a]), c.nx, c.ny, c.nz);
-            ctx->fft_rs[a] = fft_radix_set(ctx->ax[a]);
+            fft_add(ctx->fft[a], ctx->ax[a], a, c.nx, c.ny, c.nz);
         }
         J.inv_n = 1.0 / (double)ctx->ng;
         CREATE_CHK(dalloc(ctx, &ctx->d_job, 1));
@@ -2227,13 +2211,11 @@ int ohpic_fft3d_r2r(int device, int nx, int ny, int nz, int backward, const doub
     FftJob job{};
     job.src = buf;
     job.data = buf;
-    int64_t grp[3];
-    int rs[3];
+    FftLaunch fft[3];
     for (int a = 0; a < 3; ++a) {
         job.n[a] = n[a];
         job.ax[a] = ax[a];
-        grp[a] = fft_groups(a, fft_group_lines(n[a]), nx, ny, nz);
-        rs[a] = fft_radix_set(ax[a]);
+        fft_add(fft[a], ax[a], a, nx, ny, nz);
     }
     job.inv_n = 1.0 / (double)ng;
     FftJob *d_job = nullptr;
@@ -2248,10 +2230,10 @@ int ohpic_fft3d_r2r(int device, int nx, int ny, int nz, int backward, const doub
         e = hipMemcpyAsync(buf, in, ng * sizeof(double), hipMemcpyHostToDevice, st);
     if (!backward) {
         const FftPass p[3] = {kPassR2hcX, kPassR2hcY, kPassR2hcZ};
-        for (int a = 0; a < 3 && e == hipSuccess; ++a) e = fft_pass(p[a], d_job, 1, grp[a], rs[a], st);
+        for (int a = 0; a < 3 && e == hipSuccess; ++a) e = fft_pass(p[a], d_job, 1, fft[a], st);
     } else {
         const FftPass p[3] = {kPassHc2rXScaled, kPassHc2rY, kPassHc2rZ};
-        for (int a = 2; a >= 0 && e == hipSuccess; --a) e = fft_pass(p[a], d_job, 1, grp[a], rs[a], st);
+        for (int a = 2; a >= 0 && e == hipSuccess; --a) e = fft_pass(p[a], d_job, 1, fft[a], st);
     }
     if (e == hipSuccess)
         e = hipMemcpyAsync(out, buf, ng * sizeof(double), hipMemcpyDeviceToHost, st);
@@ -2296,8 +2278,7 @@ int ohpic_fft3d_r2r_noalloc(int device, int nx, int ny, int nz, int backward, co
         return fail(nullptr, OHPIC_EINVAL, "device %d out of range", device);
     const int n[3] = {nx, ny, nz};
     FftJob job{};
-    int64_t grp[3];
-    int rs[3];
+    FftLaunch fft[3];
     for (int a = 0; a < 3; ++a) {
         FftAxisDev &ax = job.ax[a];
         ax.n = n[a];
@@ -2307,8 +2288,7 @@ int ohpic_fft3d_r2r_noalloc(int device, int nx, int ny, int nz, int backward, co
                         kMaxFftLen, kMaxRadix);
         fft_plan_divisors(ax);
         job.n[a] = n[a];
-        grp[a] = fft_groups(a, fft_group_lines(n[a]), nx, ny, nz);
-        rs[a] = fft_radix_set(ax);
+        fft_add(fft[a], ax, a, nx, ny, nz);
     }
     job.inv_n = 1.0 / (double)ng;
 
@@ -2345,10 +2325,10 @@ int ohpic_fft3d_r2r_noalloc(int device, int nx, int ny, int nz, int backward, co
         e = hipMemcpyAsync(d->buf, in, ng * sizeof(double), hipMemcpyHostToDevice, st);
     if (!backward) {
         const FftPass p[3] = {kPassR2hcX, kPassR2hcY, kPassR2hcZ};
-        for (int a = 0; a < 3 && e == hipSuccess; ++a) e = fft_pass(p[a], &d->job, 1, grp[a], rs[a], st);
+        for (int a = 0; a < 3 && e == hipSuccess; ++a) e = fft_pass(p[a], &d->job, 1, fft[a], st);
     } else {
         const FftPass p[3] = {kPassHc2rXScaled, kPassHc2rY, kPassHc2rZ};
-        for (int a = 2; a >= 0 && e == hipSuccess; --a) e = fft_pass(p[a], &d->job, 1, grp[a], rs[a], st);
+        for (int a = 2; a >= 0 && e == hipSuccess; --a) e = fft_pass(p[a], &d->job, 1, fft[a], st);
     }
     if (e == hipSuccess)
         e = hipMemcpyAsync(out, d->buf, ng * sizeof(double), hipMemcpyDeviceToHost, st);

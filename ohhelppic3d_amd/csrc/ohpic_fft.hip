@@ -5,7 +5,9 @@
 // poissonSolver3d_solve (poisson_solver3d.f90:134-207) on one device.
 //
 // Each launch transforms every line of one axis of an nx*ny*nz array (x
-// fastest).  A workgroup loads G real lines of that axis with coalesced
+// fastest).  Lines of n = A B points with A, B <= 16 take k_fft_two_step; for
+// the others (longer lines, and lengths without such factors) a workgroup of
+// k_fft_pass loads G real lines of that axis with coalesced
 // reads (G consecutive rows for x; G consecutive x positions for y and z),
 // packs line pairs into complex lines z = a + i b in LDS, runs a mixed-radix
 // Stockham FFT in LDS (radix 4/2/3/5 and a generic small-prime stage), and
@@ -16,9 +18,10 @@
 // LDS-resident visit of each z line.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
-#include <type_traits>
 
+#include "ohpic_dft.hpp"
 #include "ohpic_fft.hpp"
 #include "ohpic_internal.hpp"
 
@@ -26,19 +29,9 @@ namespace ohpic {
 
 namespace {
 
-
-struct cplx {
-    double re, im;
-};
-
 __device__ __forceinline__ int fastdiv(int t, uint32_t m)
 {
     return m ? (int)__umulhi((uint32_t)t, m) : t;
-}
-
-__device__ __forceinline__ cplx cmul(cplx a, cplx b)
-{
-    return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
 }
 
 // One Stockham radix-P stage, in place over `nlines` complex lines of length
@@ -48,8 +41,8 @@ __device__ __forceinline__ cplx cmul(cplx a, cplx b)
 // synchronises, then the outputs are written back over the same buffer.
 // Twiddle tables live in global memory, or (TL) in the workgroup's LDS copy
 // for lengths up to kTwLds: staged once per workgroup (4 KiB at n = 256, so
-// 8 workgroups still fit a CU), they cut every single-transform pass at 256^3
-// from 60-62 us to 56-59 us.
+// 8 workgroups still fit a CU), they cut a single-transform pass of 256-point
+// lines at 256^3 from 60-62 us to 56-59 us.
 constexpr int kTwLds = 256;
 typedef double d2v __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) d2v lds_d2v;
@@ -65,50 +58,6 @@ __device__ __forceinline__ cplx twiddle(const double2 *__restrict__ tw, int k)
     else
         w = gload(reinterpret_cast<const d2v *>(tw), k);
     return cplx{w.x, SIGN < 0 ? w.y : -w.y};
-}
-
-template <int SIGN, int P, bool TL>
-__device__ __forceinline__ void butterfly(cplx *a, const double2 *__restrict__ tw, int step)
-{
-    if (P == 2) {
-        const cplx t = a[1];
-        a[1] = {a[0].re - t.re, a[0].im - t.im};
-        a[0] = {a[0].re + t.re, a[0].im + t.im};
-    } else if (P == 4) {
-        const cplx t0 = {a[0].re + a[2].re, a[0].im + a[2].im};
-        const cplx t1 = {a[0].re - a[2].re, a[0].im - a[2].im};
-        const cplx t2 = {a[1].re + a[3].re, a[1].im + a[3].im};
-        const cplx t3 = {a[1].re - a[3].re, a[1].im - a[3].im};
-        const cplx wt3 = {-SIGN * t3.im, SIGN * t3.re};  // (SIGN i) * t3
-        a[0] = {t0.re + t2.re, t0.im + t2.im};
-        a[1] = {t1.re + wt3.re, t1.im + wt3.im};
-        a[2] = {t0.re - t2.re, t0.im - t2.im};
-        a[3] = {t1.re - wt3.re, t1.im - wt3.im};
-    } else if (P == 3) {
-        const double sn = SIGN * 0.86602540378443864676372317075294;  // sin(2 pi/3)
-        const cplx ts = {a[1].re + a[2].re, a[1].im + a[2].im};
-        const cplx td = {a[1].re - a[2].re, a[1].im - a[2].im};
-        const cplx m = {a[0].re - 0.5 * ts.re, a[0].im - 0.5 * ts.im};
-        const cplx j = {-sn * td.im, sn * td.re};
-        a[0] = {a[0].re + ts.re, a[0].im + ts.im};
-        a[1] = {m.re + j.re, m.im + j.im};
-        a[2] = {m.re - j.re, m.im - j.im};
-    } else {
-        cplx o[P];
-#pragma unroll
-        for (int u = 0; u < P; ++u) {
-            cplx acc = a[0];
-#pragma unroll
-            for (int q = 1; q < P; ++q) {
-                const cplx v = cmul(a[q], twiddle<SIGN, TL>(tw, ((u * q) % P) * step));
-                acc.re += v.re;
-                acc.im += v.im;
-            }
-            o[u] = acc;
-        }
-#pragma unroll
-        for (int u = 0; u < P; ++u) a[u] = o[u];
-    }
 }
 
 template <int SIGN, int P, bool TL>
@@ -137,7 +86,7 @@ __device__ __forceinline__ void fft_stage(cplx *__restrict__ buf, int n, int nli
                 if (q > 0 && f > 0) v = cmul(v, twiddle<SIGN, TL>(tw, f * q * r));
                 a[k][q] = v;
             }
-            butterfly<SIGN, P, TL>(a[k], tw, n / P);
+            Dft<SIGN, P>::run(a[k]);
         }
     }
     __syncthreads();
@@ -393,7 +342,7 @@ __device__ __forceinline__ void store_complex_pairs(const cplx *buf, gmem_t<doub
 template <int KIND, int AXIS, int RS, bool FROM_SRC, bool SCALE>
 __global__ void __launch_bounds__(kFftBlock)
     __attribute__((amdgpu_waves_per_eu(OHPIC_FFT_MIN_WAVES, 8)))
-    k_fft_pass(const FftJob *__restrict__ jobs, int skip256)
+    k_fft_pass(const FftJob *__restrict__ jobs)
 {
     __shared__ cplx buf[kFftLdsCplx];
     __shared__ double sLamXY[KIND == kFftPoisson ? 64 : 1];
@@ -402,8 +351,7 @@ __global__ void __launch_bounds__(kFftBlock)
     const int nx = J.n[0], ny = J.n[1], nz = J.n[2];
     const FftAxisDev &ax = J.ax[AXIS];
     const int n = ax.n;
-    // a Poisson job with 256-point z lines is k_poisson_z256's
-    if (KIND == kFftPoisson && skip256 && n == 256) return;
+    if (ax.A) return;  // k_fft_two_step's
     const int G = fft_group_lines(n);
     const int64_t ngroups = fft_groups(AXIS, G, nx, ny, nz);
     if ((int64_t)blockIdx.x >= ngroups) return;
@@ -502,198 +450,347 @@ __global__ void __launch_bounds__(kFftBlock)
         store_complex_pairs<AXIS>(buf, dst, lb, n, nlines, ax, out_scale);
 }
 
-// ------------------------------------------------ Poisson z pass, n = 256
-// The fused z pass for z lines of 256 points as a 16 x 16 decomposition with
-// the 16-point DFTs in registers: n = 16 n1 + n2, k = k1 + 16 k2.  A 64-thread
-// workgroup holds four complex lines (8 real z lines at consecutive x, packed
-// in pairs), 16 threads per line, 16 points per thread.  Forward: thread n2
-// loads x[16 n1 + n2] (n1 = 0..15), DFT16 over n1, twiddle W256^{n2 k1},
-// transpose through LDS, DFT16 over n2: thread k1 holds X[k1 + 16 k2].  The
-// Green's-function division pairs X[k] with X[256 - k] (read back from LDS),
-// the inverse runs the same steps backwards, and thread n2 stores x[16 n1 +
-// n2].  Three LDS exchanges per visit against ten for the radix-4 stages of
-// k_fft_pass (67 us against 105 us at 256^3).  Rows of the LDS exchange
-// buffer are padded to 17 entries so that 16 lanes of one line cover all
-// banks.
-constexpr int kZ256Lines = 4;                 // complex lines per workgroup
-constexpr int kZ256Threads = 16 * kZ256Lines;
-constexpr int kZ256Row = 17;                  // padded row of 16 entries
-constexpr int kZ256LineStride = 16 * kZ256Row;
-
-// cos and sin of 2 pi j / 16, j = 0..15
-__device__ __forceinline__ cplx w16(int j, int sign)
-{
-    constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173,
-                     r2 = 0.70710678118654752440;
-    const double C[16] = {1.0, c1, r2, s1, 0.0, -s1, -r2, -c1, -1.0, -c1, -r2, -s1, 0.0, s1, r2, c1};
-    const double S[16] = {0.0, s1, r2, c1, 1.0, c1, r2, s1, 0.0, -s1, -r2, -c1, -1.0, -c1, -r2, -s1};
-    return cplx{C[j & 15], sign < 0 ? -S[j & 15] : S[j & 15]};
-}
-
-// In-place 16-point DFT of a[0..15] with exponent sign SIGN (-1 forward):
-// 4-point DFTs over a[m + 4 j], twiddles w16^{m q}, 4-point DFTs over m;
-// output X[q + 4 r] in a[q + 4 r].
-template <int SIGN>
-__device__ __forceinline__ void dft16(cplx *a)
-{
-    cplx t[4][4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        cplx v[4] = {a[m], a[m + 4], a[m + 8], a[m + 12]};
-        butterfly<SIGN, 4, false>(v, nullptr, 0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) t[m][q] = (m == 0 || q == 0) ? v[q] : cmul(v[q], w16(m * q, SIGN));
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        cplx v[4] = {t[0][q], t[1][q], t[2][q], t[3][q]};
-        butterfly<SIGN, 4, false>(v, nullptr, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) a[q + 4 * r] = v[r];
-    }
-}
+// ------------------------------------------------ axis passes of n = A B points
+// For n = A B with A, B <= 16 (fft_two_step): the transform as two steps of
+// DFTs held in registers.  With positions p = j + B m and modes k = k1 + A k2,
+//   X[k] = sum_j w_n^{j k1} w_B^{j k2} sum_m w_A^{m k1} x[j + B m]:
+// thread j of a line loads its A points, DFT of A points, twiddles, transpose
+// through LDS, and thread k1 takes the DFT of B points and holds X[k1 + A k2].
+// A workgroup is one wavefront of 64 / max(A, B) complex lines (pairs of real
+// lines), so its LDS exchanges need no barrier; every global access of a pass
+// goes straight to or from registers.  A mode and its conjugate partner n - k
+// meet through one more LDS exchange: unpacking R2HC output, packing HC2R
+// input, and the Green's-function division of the fused Poisson z pass, whose
+// inverse runs the same steps backwards.
+//
+// What bounds it: at 256^3 (16 x 16) a pass moves 16 B per node in 44 to 46 us,
+// 5.9 TB/s (52 to 63 us with radix-4 stages in LDS; the fused z pass takes 68,
+// its division included).  The passes of a small grid are one wavefront's
+// chain of a load, two or three exchanges and a store: at 32^3 4.2 to 6.9 us
+// each, where the LDS stages (2 to 5 round trips, twice the barriers) took 6.3
+// to 12.3.  Solves, stages -> two steps: 64^3 59 -> 48 us, 90x126x75 115 -> 82,
+// 128^3 113 -> 105, 169^3 1512 -> 196 (radix 13), 256^3 426 -> 406, and no
+// length of 4 to 256 measured slower.  The step functions are compiled for
+// each number of points and chosen once per step: with loops over 16 guarded
+// points the passes at 32^3 took 5.3 to 9.3 us.
+constexpr int kAbThreads = 64;
 
 // 1/d for 0 < d < 2^1000 (d = 0 gives inf, which the caller discards): the
 // hardware estimate (about 23 correct bits) refined by two Newton steps, so
-// the error is that of the final rounding.  Replacing the 32 correctly
-// rounded divisions per thread (and their branches) took the pass from 82 to
-// 67 us at 256^3.
-__device__ __forceinline__ double z256_recip(double d)
+// the error is that of the final rounding.  Replacing correctly rounded
+// divisions (and their branches) took the 256-point z pass from 82 to 67 us at
+// 256^3.
+__device__ __forceinline__ double fast_recip(double d)
 {
     double r = __builtin_amdgcn_rcp(d);
     r = __fma_rn(__fma_rn(-d, r, 1.0), r, r);
     return __fma_rn(__fma_rn(-d, r, 1.0), r, r);
 }
 
-__global__ void __launch_bounds__(kZ256Threads) k_poisson_z256(const FftJob *__restrict__ jobs)
+__device__ __forceinline__ void wave_exchange()
 {
-    __shared__ cplx xb[kZ256Lines * kZ256LineStride];
-    __shared__ double2 sTw[256];
-    __shared__ double sLam[2 * kZ256Lines];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// f(P) with P as a constant; the same P in every lane.
+template <int FIXED, class F>
+__device__ __forceinline__ void with_points(int P, F &f)
+{
+#define OHPIC_POINTS(N) \
+    case N: f(std::integral_constant<int, N>()); break
+    if (FIXED) {
+        f(std::integral_constant<int, FIXED ? FIXED : 2>());
+        return;
+    }
+    switch (P) {
+        OHPIC_POINTS(2);
+        OHPIC_POINTS(3);
+        OHPIC_POINTS(4);
+        OHPIC_POINTS(5);
+        OHPIC_POINTS(6);
+        OHPIC_POINTS(7);
+        OHPIC_POINTS(8);
+        OHPIC_POINTS(9);
+        OHPIC_POINTS(10);
+        OHPIC_POINTS(11);
+        OHPIC_POINTS(12);
+        OHPIC_POINTS(13);
+        OHPIC_POINTS(14);
+        OHPIC_POINTS(15);
+        OHPIC_POINTS(16);
+    }
+#undef OHPIC_POINTS
+}
+
+// FIXED: A and B when known at compile time (16 x 16), else 0.
+template <int KIND, int AXIS, bool FROM_SRC, bool SCALE, int FIXED>
+__global__ void __launch_bounds__(kAbThreads)
+k_fft_two_step(const FftJob *__restrict__ jobs)
+{
+    extern __shared__ cplx ab_lds[];
     const FftJob &J = jobs[blockIdx.y];
-    if (J.n[2] != 256) return;
-    const int nx = J.n[0], ny = J.n[1];
-    const int64_t nxy = (int64_t)nx * ny;
-    const int ngroups = (int)((nxy + 2 * kZ256Lines - 1) / (2 * kZ256Lines));
-    if ((int)blockIdx.x >= ngroups) return;
-    // neighbouring groups read the two 64-byte halves of the same 128-byte
-    // lines: keep them on one XCD
-    const int grp = xcd_remap((int)blockIdx.x, ngroups);
-    const int64_t l0 = (int64_t)grp * (2 * kZ256Lines);
-    const int nvalid = (int)min<int64_t>(2 * kZ256Lines, nxy - l0);
+    const int nx = J.n[0], ny = J.n[1], nz = J.n[2];
+    const FftAxisDev &ax = J.ax[AXIS];
+    // this launch's jobs: 16 x 16 or any other pair
+    if (ax.A == 0 || (FIXED == 16) != (ax.A == 16 && ax.B == 16)) return;
+    constexpr int R = 16;
+    const int A = FIXED ? FIXED : ax.A, B = FIXED ? FIXED : ax.B, n = A * B;
+    const int L = FIXED ? kAbThreads / FIXED : ax.ab_lines;
+    const int64_t ngroups = fft_groups(AXIS, 2 * L, nx, ny, nz);
+    if ((int64_t)blockIdx.x >= ngroups) return;
+    // neighbouring groups read the parts of the same 128-byte lines (y and z
+    // passes): keep them on one XCD
+    const int grp = xcd_remap((int)blockIdx.x, (int)ngroups);
+    const LineBlock lb = line_block<AXIS>(grp, 2 * L, nx, ny, nz);
     const int tid = threadIdx.x;
-    const int c = tid >> 4, t = tid & 15;
-    gmem_t<double> *__restrict__ data = as_global(J.data);
-    const FftAxisDev &ax = J.ax[2];
-    for (int i = tid; i < 256; i += kZ256Threads) {
-        const d2v w = gload(reinterpret_cast<const d2v *>(ax.tw), i);
-        sTw[i] = make_double2(w.x, w.y);
+    const int M = max(A, B);
+    const int c = FIXED ? tid / FIXED : fastdiv(tid, ax.mg_M), t = tid - c * M;
+    const bool live = c < L;
+    const bool one = live && t < B, two = live && t < A;  // threads of the two steps
+    const int RA = A | 1, RB = B | 1;                     // odd rows of the LDS exchanges
+    cplx *tw = ab_lds;                                    // twiddles, then the exchange buffer
+    cplx *xl = ab_lds + n + (live ? c : 0) * max(B * RA, A * RB);
+    double *lam = reinterpret_cast<double *>(ab_lds + n + L * max(B * RA, A * RB));  // 2 L
+    double *lz = lam + 2 * L;                             // n
+
+    // twiddles and z denominators on their way before the lines
+    constexpr int TQ = 256 / kAbThreads;
+    d2v wq[TQ];
+    double zq[TQ];
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+        const int i = min(tid + q * kAbThreads, n - 1);
+        wq[q] = gload(reinterpret_cast<const d2v *>(ax.tw), i);
+        if (KIND == kFftPoisson) zq[q] = gload(J.lam[2], i);
     }
-    if (tid < 2 * kZ256Lines) {
-        // lam_x + lam_y of real line tid; -1 marks the DC line (ix = iy = 0);
-        // lines past the grid's end get 1 (they hold zeros; no 0/0)
-        double v = 1.0;
-        if (tid < nvalid) {
-            const int64_t l = l0 + tid;
-            const int iy = (int)(l / nx), ix = (int)(l - (int64_t)iy * nx);
-            v = (l == 0) ? -1.0 : gload(J.lam[0], ix) + gload(J.lam[1], iy);
+    auto stage_tables = [&]() __attribute__((always_inline))
+    {
+#pragma unroll
+        for (int q = 0; q < TQ; ++q) {
+            const int i = tid + q * kAbThreads;
+            if (i < n) {
+                tw[i] = cplx{wq[q].x, wq[q].y};
+                if (KIND == kFftPoisson) lz[i] = zq[q];
+            }
         }
-        sLam[tid] = v;
-    }
-    // real lines 2c (re) and 2c + 1 (im): one 16-byte load per point when
-    // both are present and nx*ny is even (l0 is even, so every pair is then
-    // 16-byte aligned), else two 8-byte loads
-    const bool va = 2 * c < nvalid, vb = 2 * c + 1 < nvalid;
-    const bool v16 = vb && (nxy & 1) == 0;
-    const int64_t la = l0 + 2 * c;
+        if (KIND == kFftPoisson && tid < 2 * L) {
+            // lam_x + lam_y of real line tid; -1 marks the DC line (ix = iy = 0);
+            // lines past the grid's end get 1 (they hold zeros; no 0/0)
+            double v = 1.0;
+            if (tid < lb.nvalid) {
+                const int l = (int)lb.base + tid;  // < nx ny <= 2^20
+                const int iy = l / nx, ix = l - iy * nx;
+                v = (l == 0) ? -1.0 : gload(J.lam[0], ix) + gload(J.lam[1], iy);
+            }
+            lam[tid] = v;
+        }
+    };
+
+    // real lines 2c (re) and 2c + 1 (im): y and z lines are adjacent, one
+    // 16-byte access per point when every pair is aligned (an even stride; the
+    // number of lines is then even too)
+    const bool v16 = AXIS != 0 && (lb.estride & 1) == 0;
+    const bool va = live && 2 * c < lb.nvalid, vb = live && 2 * c + 1 < lb.nvalid;
+    const uint32_t g1 = (uint32_t)lb.gstride;
+    const uint32_t lane0 = (uint32_t)(2 * c) * g1 + (uint32_t)t * (uint32_t)lb.estride;
+    // points t, t + step, ... of a thread's lines (the step is uniform)
     cplx a[16];
+    auto load = [&](auto count, int step) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;
+        const gmem_t<double> *s = as_global((FROM_SRC ? J.src : J.data) + lb.base);
+        const int64_t inc = step * lb.estride;
 #pragma unroll
-    for (int n1 = 0; n1 < 16; ++n1) {
-        const int64_t o = la + (int64_t)(16 * n1 + t) * nxy;
-        if (v16) {
-            const d2v v = ((const gmem_t<d2v> *)data)[o >> 1];
-            a[n1] = cplx{v.x, v.y};
+        for (int m = 0; m < P; ++m) a[m] = cplx{0.0, 0.0};
+        if (AXIS != 0 && v16) {
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    const d2v v = ((const gmem_t<d2v> *)(s + m * inc))[lane0 >> 1];
+                    a[m] = cplx{v.x, v.y};
+                }
         } else {
-            a[n1] = cplx{va ? data[o] : 0.0, vb ? data[o + 1] : 0.0};
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) a[m].re = (s + m * inc)[lane0];
+            if (vb)
+#pragma unroll
+                for (int m = 0; m < P; ++m) a[m].im = (s + m * inc)[lane0 + g1];
         }
-    }
-    __syncthreads();  // sTw, sLam
-    const lds_d2v *tw = (const lds_d2v *)sTw;
-    cplx *xl = xb + c * kZ256LineStride;
-
-    // forward: DFT16 over n1 (thread n2 = t), twiddle, transpose
-    dft16<-1>(a);
+    };
+    auto store = [&](auto count, int step) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;
+        gmem_t<double> *d = as_global(J.data + lb.base);
+        const int64_t inc = step * lb.estride;
+        if (AXIS != 0 && v16) {
+            if (va)
 #pragma unroll
-    for (int k1 = 0; k1 < 16; ++k1) {
-        cplx v = a[k1];
-        if (k1 > 0 && t > 0) {
-            const d2v w = tw[t * k1];
-            v = cmul(v, cplx{w.x, w.y});
-        }
-        xl[t * kZ256Row + k1] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int n2 = 0; n2 < 16; ++n2) a[n2] = xl[n2 * kZ256Row + t];
-    // DFT16 over n2 (thread k1 = t): a[k2] = X[t + 16 k2]
-    dft16<-1>(a);
-    __syncthreads();  // transpose reads done before the buffer is reused
-#pragma unroll
-    for (int k2 = 0; k2 < 16; ++k2) xl[k2 * kZ256Row + t] = a[k2];
-    __syncthreads();
-
-    // Green's-function division of the packed spectra (as k_fft_pass):
-    // A_k = (Z_k + conj Z_{n-k}) / 2, B_k = (Z_k - conj Z_{n-k}) / 2i, divided
-    // by their lines' denominators (DC := 0), repacked as A' + i B'
-    const double lam_a = sLam[2 * c], lam_b = sLam[2 * c + 1];
-    const double lxa = lam_a < 0.0 ? 0.0 : lam_a, lxb = lam_b < 0.0 ? 0.0 : lam_b;
-    const gmem_t<double> *__restrict__ lamz = as_global(J.lam[2]);
-#pragma unroll
-    for (int k2 = 0; k2 < 16; ++k2) {
-        const int k = t + 16 * k2;
-        const int m1 = (16 - t) & 15;
-        const int m2 = t == 0 ? ((16 - k2) & 15) : 15 - k2;
-        const cplx zk = a[k2], zm = xl[m2 * kZ256Row + m1];
-        const double lz = lamz[k];
-        const double ra = z256_recip(lxa + lz), rb = z256_recip(lxb + lz);
-        // the DC line's k = 0 mode is set to zero (its denominator is 0)
-        const double sa = (lam_a < 0.0 && k == 0) ? 0.0 : 0.5 * ra;
-        const double sb = (lam_b < 0.0 && k == 0) ? 0.0 : 0.5 * rb;
-        const cplx A = {sa * (zk.re + zm.re), sa * (zk.im - zm.im)};
-        const cplx B = {sb * (zk.im + zm.im), -sb * (zk.re - zm.re)};
-        a[k2] = cplx{A.re - B.im, A.im + B.re};
-    }
-
-    // inverse: DFT16 over k2 (thread k1 = t), twiddle, transpose, DFT16 over k1
-    dft16<+1>(a);
-    __syncthreads();  // pair reads done before the buffer is reused
-#pragma unroll
-    for (int n2 = 0; n2 < 16; ++n2) {
-        cplx v = a[n2];
-        if (n2 > 0 && t > 0) {
-            const d2v w = tw[t * n2];
-            v = cmul(v, cplx{w.x, -w.y});
-        }
-        xl[t * kZ256Row + n2] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k1 = 0; k1 < 16; ++k1) a[k1] = xl[k1 * kZ256Row + t];
-    dft16<+1>(a);
-    // thread n2 = t holds x[16 n1 + n2] in a[n1]
-#pragma unroll
-    for (int n1 = 0; n1 < 16; ++n1) {
-        const int64_t o = la + (int64_t)(16 * n1 + t) * nxy;
-        if (v16) {
-            d2v v;
-            v.x = a[n1].re;
-            v.y = a[n1].im;
-            ((gmem_t<d2v> *)data)[o >> 1] = v;
+                for (int m = 0; m < P; ++m) {
+                    d2v w;
+                    w.x = a[m].re;
+                    w.y = a[m].im;
+                    ((gmem_t<d2v> *)(d + m * inc))[lane0 >> 1] = w;
+                }
         } else {
-            if (va) data[o] = a[n1].re;
-            if (vb) data[o + 1] = a[n1].im;
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) (d + m * inc)[lane0] = a[m].re;
+            if (vb)
+#pragma unroll
+                for (int m = 0; m < P; ++m) (d + m * inc)[lane0 + g1] = a[m].im;
         }
-    }
+    };
+    // a[k] *= exp(SIGN 2 pi i t k / n)
+    auto twiddles = [&](auto sign, auto count) __attribute__((always_inline))
+    {
+#pragma unroll
+        for (int k = 1; k < decltype(count)::value; ++k) {
+            const cplx w = tw[t * k];
+            a[k] = cmul(a[k], cplx{w.re, decltype(sign)::value < 0 ? w.im : -w.im});
+        }
+    };
+    constexpr int SIGN = KIND == kFftHC2R ? +1 : -1;
+    using Sign = std::integral_constant<int, SIGN>;
+    using Back = std::integral_constant<int, +1>;
+
+    // step 1 (thread j = t), twiddles, transpose
+    auto first = [&](auto count) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;  // A
+        constexpr int RP = P | 1;
+        if (one) load(count, B);
+        stage_tables();
+        wave_exchange();
+        if (KIND == kFftHC2R) {
+            // halfcomplex values V_p of both lines -> packed spectrum Z = A + i B
+            if (one) {
+#pragma unroll
+                for (int m = 0; m < P; ++m) xl[m * RB + t] = a[m];
+            }
+            wave_exchange();
+            if (one) {
+                // position n - p: row P - 1 - m, or P - m (mod P) for t = 0
+                const cplx *x = t == 0 ? xl + RB : xl + B - t;
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    const int p = t + B * m;
+                    const cplx v = a[m];
+                    const cplx w = m == 0 && t == 0 ? xl[0] : x[(P - 1 - m) * RB];
+                    const cplx lo = {v.re - w.im, w.re + v.im}, hi = {w.re + v.im, w.im - v.re};
+                    // below n/2 up to m = P/2 - 1, above it from m = P/2 + 1
+                    if (m == 0)
+                        a[m] = t == 0 ? v : lo;
+                    else if (2 * m + 2 <= P)
+                        a[m] = lo;
+                    else if (2 * m > P)
+                        a[m] = hi;
+                    else
+                        a[m] = 2 * p == n ? v : (2 * p < n ? lo : hi);
+                }
+            }
+            wave_exchange();  // reads done before the buffer is reused
+        }
+        if (one) {
+            Dft<SIGN, P>::run(a);
+            twiddles(Sign(), count);
+#pragma unroll
+            for (int k1 = 0; k1 < P; ++k1) xl[t * RP + k1] = a[k1];
+        }
+        wave_exchange();
+    };
+    // step 2 (thread k1 = t): a[k2] = X[t + A k2], and what follows on modes
+    auto second = [&](auto count) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;  // B
+        constexpr int RP = P | 1;
+        if (two) {
+#pragma unroll
+            for (int j = 0; j < P; ++j) a[j] = xl[j * RA + t];
+            Dft<SIGN, P>::run(a);
+        }
+        if (KIND == kFftHC2R) {
+            if (two) {
+                if (SCALE) {
+                    const double scale = J.inv_n;
+#pragma unroll
+                    for (int k2 = 0; k2 < P; ++k2)
+                        a[k2] = cplx{a[k2].re * scale, a[k2].im * scale};
+                }
+                store(count, A);
+            }
+            return;
+        }
+        // each mode meets its partner n - k
+        wave_exchange();  // transpose reads done
+        if (two) {
+#pragma unroll
+            for (int k2 = 0; k2 < P; ++k2) xl[k2 * RA + t] = a[k2];
+        }
+        wave_exchange();
+        if (two) {
+            // mode n - k: row P - 1 - k2, or P - k2 (mod P) for t = 0
+            const cplx *x = t == 0 ? xl + RA : xl + A - t;
+            const double lam_a = KIND == kFftPoisson ? lam[2 * c] : 0.0;
+            const double lam_b = KIND == kFftPoisson ? lam[2 * c + 1] : 0.0;
+            const double lxa = lam_a < 0.0 ? 0.0 : lam_a, lxb = lam_b < 0.0 ? 0.0 : lam_b;
+#pragma unroll
+            for (int k2 = 0; k2 < P; ++k2) {
+                const int k = t + A * k2;
+                const cplx zk = a[k2];
+                const cplx zm = k2 == 0 && t == 0 ? xl[0] : x[(P - 1 - k2) * RA];
+                if (KIND == kFftR2HC) {
+                    // position k of the halfcomplex lines: of A_k = (Z_k +
+                    // conj Z_{n-k}) / 2 and B_k = (Z_k - conj Z_{n-k}) / 2i the
+                    // real parts up to n/2, then the imaginary parts of mode
+                    // n - k
+                    // (k2 from P/2 + 1; up to P/2 - 1 real)
+                    const bool im = 2 * k2 + 2 > P && (2 * k2 > P || 2 * k > n);
+                    a[k2] = im ? cplx{0.5 * (zm.im - zk.im), 0.5 * (zk.re - zm.re)}
+                               : cplx{0.5 * (zk.re + zm.re), 0.5 * (zk.im + zm.im)};
+                } else {
+                    // A_k and B_k divided by their lines' denominators (the DC
+                    // line's k = 0 mode, whose denominator is 0, set to zero),
+                    // repacked as A' + i B'
+                    const double ra = fast_recip(lxa + lz[k]), rb = fast_recip(lxb + lz[k]);
+                    const double sa = (lam_a < 0.0 && k == 0) ? 0.0 : 0.5 * ra;
+                    const double sb = (lam_b < 0.0 && k == 0) ? 0.0 : 0.5 * rb;
+                    const cplx U = {sa * (zk.re + zm.re), sa * (zk.im - zm.im)};
+                    const cplx V = {sb * (zk.im + zm.im), -sb * (zk.re - zm.re)};
+                    a[k2] = cplx{U.re - V.im, U.im + V.re};
+                }
+            }
+        }
+        if (KIND == kFftR2HC) {
+            if (two) store(count, A);
+            return;
+        }
+        // inverse: DFT over k2 (thread k1 = t), twiddles, transpose
+        wave_exchange();  // partner reads done before the buffer is reused
+        if (two) {
+            Dft<+1, P>::run(a);
+            twiddles(Back(), count);
+#pragma unroll
+            for (int j = 0; j < P; ++j) xl[t * RP + j] = a[j];
+        }
+        wave_exchange();
+    };
+    // ... and over k1 (thread j = t)
+    auto third = [&](auto count) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;  // A
+        if (one) {
+#pragma unroll
+            for (int k1 = 0; k1 < P; ++k1) a[k1] = xl[k1 * RB + t];
+            Dft<+1, P>::run(a);
+            store(count, B);
+        }
+    };
+    with_points<FIXED>(A, first);
+    with_points<FIXED>(B, second);
+    if (KIND == kFftPoisson) with_points<FIXED>(A, third);
 }
 
 }  // namespace
@@ -704,12 +801,49 @@ void fft_plan_divisors(FftAxisDev &ax)
     ax.mg_G = fastdiv_magic((uint32_t)fft_group_lines(ax.n));
     ax.mg_half = fastdiv_magic((uint32_t)(ax.n / 2 + 1));
     ax.mg_nl = fastdiv_magic((uint32_t)(fft_group_lines(ax.n) / 2));
+    fft_two_step(ax.n, &ax.A, &ax.B);
+    ax.ab_lines = ax.A ? kAbThreads / (ax.A > ax.B ? ax.A : ax.B) : 0;
+    ax.mg_M = fastdiv_magic((uint32_t)(ax.A > ax.B ? ax.A : ax.B));
     int Ls = 1;
     for (int s = 0; s < kMaxFactors; ++s) {
         const int p = s < ax.nfac ? ax.fac[s] : 1;
         ax.mg_tpl[s] = fastdiv_magic((uint32_t)(ax.n / p));
         ax.mg_Ls[s] = fastdiv_magic((uint32_t)Ls);
         Ls *= p;
+    }
+}
+
+void fft_two_step(int n, int *A, int *B)
+{
+    *A = *B = 0;
+    for (int a = 2; a <= 16 && a * a <= n; ++a)
+        if (n % a == 0 && n / a <= 16) {
+            *A = a;
+            *B = n / a;
+        }
+}
+
+int64_t fft_two_step_lds(int A, int B)
+{
+    const int L = kAbThreads / (A > B ? A : B);
+    const int ra = B * (A | 1), rb = A * (B | 1);
+    return (int64_t)(A * B + L * (ra > rb ? ra : rb)) * (int64_t)sizeof(double2) +
+           (2 * L + A * B) * (int64_t)sizeof(double);
+}
+
+void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz)
+{
+    if (ax.A == 0) {
+        l.groups = std::max(l.groups, fft_groups(axis, fft_group_lines(ax.n), nx, ny, nz));
+        l.rs = std::max(l.rs, fft_radix_set(ax));
+        return;
+    }
+    const int64_t g = fft_groups(axis, 2 * ax.ab_lines, nx, ny, nz);
+    if (ax.A == 16 && ax.B == 16) {
+        l.groups16 = std::max(l.groups16, g);
+    } else {
+        l.groups_ab = std::max(l.groups_ab, g);
+        l.lds_ab = std::max(l.lds_ab, fft_two_step_lds(ax.A, ax.B));
     }
 }
 
@@ -724,48 +858,43 @@ int fft_radix_set(const FftAxisDev &ax)
 }
 
 template <int KIND, int AXIS, bool FROM_SRC, bool SCALE>
-static hipError_t launch_pass(const FftJob *jobs, int njobs, int64_t max_groups, int rs,
-                              hipStream_t st, int skip256 = 0)
+static hipError_t launch_pass(const FftJob *jobs, int njobs, const FftLaunch &l, hipStream_t st)
 {
-    if (njobs <= 0 || max_groups <= 0) return hipSuccess;
-    const dim3 g((unsigned)round_up_xcds(max_groups), (unsigned)njobs), b(kFftBlock);
-    if (rs == 0)
-        hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 0, FROM_SRC, SCALE>), g, b, 0, st, jobs, skip256);
-    else if (rs == 1)
-        hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 1, FROM_SRC, SCALE>), g, b, 0, st, jobs, skip256);
-    else
-        hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 2, FROM_SRC, SCALE>), g, b, 0, st, jobs, skip256);
-    return hipGetLastError();
-}
-
-hipError_t fft_poisson_z(const FftJob *jobs, int njobs, int64_t max_groups, int rs, int z256,
-                         hipStream_t st)
-{
-    if (njobs <= 0 || max_groups <= 0) return hipSuccess;
-    if (z256 != kZ256All) {
-        const hipError_t e = launch_pass<kFftPoisson, 2, false, false>(
-            jobs, njobs, max_groups, rs, st, z256 == kZ256Some ? 1 : 0);
-        if (e != hipSuccess || z256 == kZ256None) return e;
+    if (njobs <= 0) return hipSuccess;
+    if (l.groups > 0) {
+        const dim3 g((unsigned)round_up_xcds(l.groups), (unsigned)njobs), b(kFftBlock);
+        if (l.rs == 0)
+            hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 0, FROM_SRC, SCALE>), g, b, 0, st, jobs);
+        else if (l.rs == 1)
+            hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 1, FROM_SRC, SCALE>), g, b, 0, st, jobs);
+        else
+            hipLaunchKernelGGL((k_fft_pass<KIND, AXIS, 2, FROM_SRC, SCALE>), g, b, 0, st, jobs);
     }
-    // the groups of a 256-point job are those of k_fft_pass (8 real lines each),
-    // so max_groups covers them
-    const dim3 g((unsigned)round_up_xcds(max_groups), (unsigned)njobs), b(kZ256Threads);
-    hipLaunchKernelGGL(k_poisson_z256, g, b, 0, st, jobs);
+    if (l.groups16 > 0) {
+        const dim3 g((unsigned)round_up_xcds(l.groups16), (unsigned)njobs), b(kAbThreads);
+        hipLaunchKernelGGL((k_fft_two_step<KIND, AXIS, FROM_SRC, SCALE, 16>), g, b,
+                           (unsigned)fft_two_step_lds(16, 16), st, jobs);
+    }
+    if (l.groups_ab > 0) {
+        const dim3 g((unsigned)round_up_xcds(l.groups_ab), (unsigned)njobs), b(kAbThreads);
+        hipLaunchKernelGGL((k_fft_two_step<KIND, AXIS, FROM_SRC, SCALE, 0>), g, b,
+                           (unsigned)l.lds_ab, st, jobs);
+    }
     return hipGetLastError();
 }
 
-hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, int64_t max_groups, int rs,
+hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, const FftLaunch &l,
                     hipStream_t st)
 {
     switch (pass) {
-    case kPassR2hcXFromSrc: return launch_pass<kFftR2HC, 0, true, false>(jobs, njobs, max_groups, rs, st);
-    case kPassR2hcX: return launch_pass<kFftR2HC, 0, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassR2hcY: return launch_pass<kFftR2HC, 1, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassR2hcZ: return launch_pass<kFftR2HC, 2, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassPoissonZ: return launch_pass<kFftPoisson, 2, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassHc2rZ: return launch_pass<kFftHC2R, 2, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassHc2rY: return launch_pass<kFftHC2R, 1, false, false>(jobs, njobs, max_groups, rs, st);
-    case kPassHc2rXScaled: return launch_pass<kFftHC2R, 0, false, true>(jobs, njobs, max_groups, rs, st);
+    case kPassR2hcXFromSrc: return launch_pass<kFftR2HC, 0, true, false>(jobs, njobs, l, st);
+    case kPassR2hcX: return launch_pass<kFftR2HC, 0, false, false>(jobs, njobs, l, st);
+    case kPassR2hcY: return launch_pass<kFftR2HC, 1, false, false>(jobs, njobs, l, st);
+    case kPassR2hcZ: return launch_pass<kFftR2HC, 2, false, false>(jobs, njobs, l, st);
+    case kPassPoissonZ: return launch_pass<kFftPoisson, 2, false, false>(jobs, njobs, l, st);
+    case kPassHc2rZ: return launch_pass<kFftHC2R, 2, false, false>(jobs, njobs, l, st);
+    case kPassHc2rY: return launch_pass<kFftHC2R, 1, false, false>(jobs, njobs, l, st);
+    case kPassHc2rXScaled: return launch_pass<kFftHC2R, 0, false, true>(jobs, njobs, l, st);
     }
     return hipErrorInvalidValue;
 }

@@ -47,6 +47,25 @@ struct FftAxisDev {
     uint32_t mg_nl;                // fft_group_lines(n) / 2: line pairs per group
     uint32_t mg_tpl[kMaxFactors];  // n / fac[s]: butterflies per line in stage s
     uint32_t mg_Ls[kMaxFactors];   // fac[0] * ... * fac[s-1]
+    int A, B;                      // n = A B of the two-step form, or 0
+    int ab_lines;                  // its complex lines per workgroup
+    uint32_t mg_M;                 // max(A, B)
+};
+
+// n = A B with 2 <= A <= B <= 16 as close as possible (the two-step register
+// form), or A = B = 0.  Every length up to 256 of a grid that is not a prime
+// and has such factors takes it; the others run the LDS stages.
+void fft_two_step(int n, int *A, int *B);
+int64_t fft_two_step_lds(int A, int B);  // its LDS bytes per workgroup
+
+// Workgroups of one axis pass over a table of jobs: largest counts over the
+// jobs of each form (0: no job of it).
+struct FftLaunch {
+    int64_t groups = 0;     // LDS stages
+    int rs = 0;             // their radix set
+    int64_t groups16 = 0;   // two-step form, 16 x 16
+    int64_t groups_ab = 0;  // two-step form, other A x B
+    int64_t lds_ab = 0;     // its largest LDS bytes
 };
 
 // Factorises n (radix 4 first, then 2, 3, 5, ...); false if a prime factor
@@ -101,17 +120,12 @@ enum FftPass : int {
 
 int fft_radix_set(const FftAxisDev &ax);
 
-// Which jobs of a Poisson z pass have 256-point z lines (run by the 16 x 16
-// register kernel; the others by the radix-4 LDS stages of k_fft_pass).
-enum Z256Jobs : int { kZ256None = 0, kZ256All = 1, kZ256Some = 2 };
+// Adds a job's axis to the launch of that axis' passes.
+void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz);
 
-// The fused Poisson z pass (kPassPoissonZ) for every job of the table.
-hipError_t fft_poisson_z(const FftJob *jobs, int njobs, int64_t max_groups, int rs, int z256,
-                         hipStream_t st);
-
-// One axis pass for every job of the device table `jobs`; max_groups is the
-// largest group count over the jobs, rs the largest radix set.
-hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, int64_t max_groups, int rs,
+// One axis pass for every job of the device table `jobs`.  Each job's form
+// depends on its axis length alone, so it computes the same in every table.
+hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, const FftLaunch &l,
                     hipStream_t st);
 
 }  // namespace ohpic
