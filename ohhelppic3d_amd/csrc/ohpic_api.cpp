@@ -140,6 +140,7 @@ struct ohpic_ctx {
     ohpic_group *group = nullptr;
     bool failed = false;         // a step failed: the state is no longer valid
     unsigned long long *h_flags = nullptr;  // pinned
+    unsigned long long *dh_flags = nullptr; // its device address
     double *h_diag = nullptr;               // pinned
     int par = 0;
     bool rho_valid = false;
@@ -845,9 +846,10 @@ int one_step(ohpic_ctx *ctx)
     timer_begin(ctx, 0);
     HIPCHK(ctx, run_particles(ctx, kModeFused));
     timer_end(ctx, 0);
-    // the parity word is only read here (no out: no flip)
-    HIPCHK(ctx, launch_end_step_b(ctx->d_inst, ctx->d_par01 + ctx->par, 1, nullptr, ctx->st));
-    if ((rc = read_flags(ctx))) return rc;
+    // (a single instance's parity word is only read: no flip)
+    HIPCHK(ctx, launch_end_step_b(ctx->d_inst, ctx->d_par01 + ctx->par, 1, false, ctx->dh_flags,
+                                  ctx->st));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->st));
     timers_collect(ctx);
     rc = absorb_flags(ctx, ctx->h_flags);
     if (rc < 0) return rc;
@@ -1271,7 +1273,7 @@ hipError_t group_enqueue(ohpic_group *g, int k)
             e = launch_close_chunks(g->precision, g->d_insts, g->d_close, g->nclose, g->max_ns,
                                     g->d_parity, g->st);
         if (e == hipSuccess)
-            e = launch_end_step_b(g->d_insts, g->d_parity, n,
+            e = launch_end_step_b(g->d_insts, g->d_parity, n, true,
                                   g->d_flags + (size_t)s * n * kFlagSlots, g->st);
     }
     if (e == hipSuccess)
@@ -1681,6 +1683,7 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
     }
     CREATE_HIP(hipHostMalloc((void **)&ctx->h_flags, kFlagSlots * sizeof(unsigned long long),
                              hipHostMallocDefault));
+    CREATE_HIP(hipHostGetDevicePointer((void **)&ctx->dh_flags, ctx->h_flags, 0));
     CREATE_HIP(hipHostMalloc((void **)&ctx->h_diag, kDiagSlots * sizeof(double),
                              hipHostMallocDefault));
     CREATE_CHK(dalloc(ctx, &ctx->d_close, nt));

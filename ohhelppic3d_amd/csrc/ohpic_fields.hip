@@ -167,13 +167,13 @@ __global__ void __launch_bounds__(256) k_efield_b(const InstDev *__restrict__ in
 // threads of the blocks that reduce per-item and per-block partial sums
 constexpr int kSumBlock = 1024;
 
-// Sum of partial[i*stride + k] over i < count by one block, in an order that
-// depends on count alone.  Each thread keeps kSumLanes running sums (entries
-// i, i + blockDim, ... of one trip go to sums 0, 1, ...), so that many loads
-// are in flight; a single running sum made the reduction over the 32768 work
-// items of a 256^3 step wait for one load at a time.
-__device__ double block_ordered_sum(const double *__restrict__ partial, int count, int stride,
-                                    int k, double *red)
+// This thread's share of the sum of partial[i*stride + k] over i < count by
+// one block (block_total), in an order that depends on count alone.  It keeps
+// kSumLanes running sums (entries i, i + blockDim, ... of one trip go to sums
+// 0, 1, ...), so that many loads are in flight; a single running sum made the
+// reduction over the 32768 work items of a 256^3 step wait for one load at a
+// time.
+__device__ double thread_sum(const double *__restrict__ partial, int count, int stride, int k)
 {
     constexpr int kSumLanes = 8;
     const int nb = (int)blockDim.x;
@@ -192,48 +192,48 @@ __device__ double block_ordered_sum(const double *__restrict__ partial, int coun
     double s = 0.0;
 #pragma unroll
     for (int a = 0; a < kSumLanes; ++a) s += acc[a];
-    red[threadIdx.x] = s;
+    return s;
+}
+
+// Sum of v over a block of kSumBlock threads, in thread 0: each wavefront by
+// shuffles, then their sums in order (a tree over LDS with a barrier per level
+// took 0.7 us more).
+__device__ double block_total(double v, double *red)
+{
+    v = wave_sum(v);
+    if (__lane_id() == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-        __syncthreads();
-    }
-    const double r = red[0];
-    __syncthreads();
+    double r = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < kSumBlock / 64; ++w) r += red[w];
     return r;
 }
 
-// blockIdx.x = instance: diag[kDiagWe + k] := sum of the instance's e_partial rows
-__global__ void __launch_bounds__(kSumBlock) k_reduce_e_b(const InstDev *__restrict__ insts)
+// Energy sum j of an instance, by the threads of block j of kEnergySums:
+// j < kKeSlots: kinetic-energy slot j (j < kMaxSpecies: before the push, else
+// after; species j % kMaxSpecies) over the items: row j of
+// ke_partial[kKeSlots][nitems], contiguous, so that one block streams it
+// (slots of absent species are zero, their rows are not written); the others:
+// column j - kKeSlots of the rows of e_partial.
+constexpr int kEnergySums = kKeSlots + 3;
+__device__ double energy_sum(const InstDev *I, int j)
 {
-    __shared__ double red[kSumBlock];
-    const InstDev *I = insts + blockIdx.x;
-    const int count = efield_blocks_of(I->n[0], I->n[1], I->n[2]);
-    for (int k = 0; k < 3; ++k) {
-        const double v = block_ordered_sum(I->e_partial, count, 3, k, red);
-        if (threadIdx.x == 0) I->diag[kDiagWe + k] = v;
-    }
+    if (j >= kKeSlots)
+        return thread_sum(I->e_partial, efield_blocks_of(I->n[0], I->n[1], I->n[2]), 3,
+                          j - kKeSlots);
+    if (j % kMaxSpecies >= I->nspecies) return 0.0;
+    return thread_sum(I->ke_partial + (int64_t)j * I->nitems, I->nitems, 1, 0);
 }
 
-// Kinetic-energy slot k of an instance (k < kMaxSpecies: before the push, else
-// after; species k % kMaxSpecies) summed over its items: row k of
-// ke_partial[kKeSlots][nitems], contiguous, so that one block streams it.
-// Slots of absent species are zero (their rows are not written).
-__device__ double ke_slot_sum(const InstDev *I, int k, double *red)
+// blockIdx.y = instance, blockIdx.x + first = sum j: its place in diag
+__global__ void __launch_bounds__(kSumBlock) k_energy_sums_b(const InstDev *__restrict__ insts,
+                                                             int first)
 {
-    if (k % kMaxSpecies >= I->nspecies) return 0.0;
-    return block_ordered_sum(I->ke_partial + (int64_t)k * I->nitems, I->nitems, 1, 0, red);
-}
-
-// blockIdx.y = instance, blockIdx.x = slot k: diag[kDiagKeOld + k] := sum
-// over the instance's items of its kinetic-energy slot k
-__global__ void __launch_bounds__(kSumBlock) k_reduce_ke_b(const InstDev *__restrict__ insts)
-{
-    __shared__ double red[kSumBlock];
+    __shared__ double red[kSumBlock / 64];
     const InstDev *I = insts + blockIdx.y;
-    const int k = blockIdx.x;
-    const double v = ke_slot_sum(I, k, red);
-    if (threadIdx.x == 0) I->diag[kDiagKeOld + k] = v;
+    const int j = first + (int)blockIdx.x;
+    const double v = block_total(energy_sum(I, j), red);
+    if (threadIdx.x == 0) I->diag[kDiagKeOld + j] = v;
 }
 
 __global__ void k_rho_from_acc_b(const InstDev *__restrict__ insts, const int *__restrict__ parity)
@@ -312,34 +312,27 @@ __global__ void k_begin_step_b(const InstDev *__restrict__ insts, const int *__r
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
-// End of a step: blocks x < kKeSlots reduce the kinetic-energy slots (as
-// k_reduce_ke_b), block kKeSlots the field-energy partials of k_efield_b (as
-// k_reduce_e_b); unless a bin overflowed, all of them then scan a share of
+// End of a step: block x reduces energy sum x (k_energy_sums_b); unless a bin
+// overflowed, all blocks then scan a share of
 // the step's new bins (buffer parity ^ 1): listed bins go to tight_list (their
 // number to kFlagListed) and a tight one raises kFlagTight (the host then
-// moves them before the next step).  When out is not null the last block to
-// finish completes the instance's step in a group: out[i*kFlagSlots + k] :=
-// flags[k] of instance i, and parity[i] flips unless a bin overflowed (the host
-// then redoes that step in list mode from the unchanged buffer).
+// moves them before the next step).  The last block to finish reports the
+// flags: out[i*kFlagSlots + k] := flags[k] of instance i.  Of a group (flip)
+// it completes the instance's step too: parity[i] flips unless a bin
+// overflowed (the host then redoes that step in list mode from the unchanged
+// buffer).  One instance's out is the host's pinned memory: a copy of the flags
+// after this kernel took 4 us and a gap of 1.3.
 __global__ void __launch_bounds__(kSumBlock) k_end_step_b(const InstDev *__restrict__ insts,
-                                                    int *__restrict__ parity,
+                                                    int *__restrict__ parity, int flip,
                                                     unsigned long long *__restrict__ out)
 {
-    __shared__ double red[kSumBlock];
+    __shared__ double red[kSumBlock / 64];
     const InstDev *I = insts + blockIdx.y;
-    if ((int)blockIdx.x < kKeSlots) {
-        const int k = blockIdx.x;
-        const double v = ke_slot_sum(I, k, red);
-        if (threadIdx.x == 0) I->diag[kDiagKeOld + k] = v;
-    } else {
-        const int count = efield_blocks_of(I->n[0], I->n[1], I->n[2]);
-        for (int k = 0; k < 3; ++k) {
-            const double v = block_ordered_sum(I->e_partial, count, 3, k, red);
-            if (threadIdx.x == 0) I->diag[kDiagWe + k] = v;
-        }
-    }
+    const int j = blockIdx.x;
     unsigned long long *flags = I->flags;
-    if (flags[kFlagOverflow] == 0ull) {
+    const unsigned long long overflow = gload(flags, kFlagOverflow);  // (with the sum's loads)
+    const double sum = energy_sum(I, j);
+    if (overflow == 0ull) {
         const int nb = parity[blockIdx.y] ^ 1;
         const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
         const int stride = gridDim.x * blockDim.x;
@@ -356,7 +349,8 @@ __global__ void __launch_bounds__(kSumBlock) k_end_step_b(const InstDev *__restr
             }
         }
     }
-    if (!out) return;
+    const double total = block_total(sum, red);
+    if (threadIdx.x == 0) I->diag[kDiagKeOld + j] = total;
     // the flags are device-scope atomics (a thread that listed a bin fenced
     // its writes before the barrier), so the counter needs no fence of its
     // own: device-scope fences write back the L2 and cost microseconds per
@@ -373,7 +367,7 @@ __global__ void __launch_bounds__(kSumBlock) k_end_step_b(const InstDev *__restr
             f[k] = __hip_atomic_load(&flags[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             out[i * kFlagSlots + k] = f[k];
         }
-        if (f[kFlagOverflow] == 0ull) parity[i] ^= 1;
+        if (flip && f[kFlagOverflow] == 0ull) parity[i] ^= 1;
     }
 }
 
@@ -500,7 +494,9 @@ hipError_t launch_efield_b(const InstDev *insts, int ninst, int max_blocks, bool
     if (ninst <= 0) return hipSuccess;
     const int blocks = (int)round_up_xcds(max_blocks > 0 ? max_blocks : 1);
     hipLaunchKernelGGL(k_efield_b, dim3(blocks, ninst), dim3(256), 0, st, insts);
-    if (reduce) hipLaunchKernelGGL(k_reduce_e_b, dim3(ninst), dim3(kSumBlock), 0, st, insts);
+    if (reduce)
+        hipLaunchKernelGGL(k_energy_sums_b, dim3(kEnergySums - kKeSlots, ninst), dim3(kSumBlock), 0,
+                           st, insts, kKeSlots);
     return hipGetLastError();
 }
 
@@ -515,12 +511,12 @@ hipError_t launch_begin_step_b(const InstDev *insts, const int *parity, int nins
     return hipGetLastError();
 }
 
-hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst,
+hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst, bool flip,
                              unsigned long long *out, hipStream_t st)
 {
     if (ninst <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_end_step_b, dim3(kKeSlots + 1, ninst), dim3(kSumBlock), 0, st, insts,
-                       parity, out);
+    hipLaunchKernelGGL(k_end_step_b, dim3(kEnergySums, ninst), dim3(kSumBlock), 0, st, insts,
+                       parity, flip ? 1 : 0, out);
     return hipGetLastError();
 }
 
@@ -546,7 +542,7 @@ hipError_t launch_reserve_next_b(const InstDev *insts, const int *parity, int ni
 hipError_t launch_reduce_ke_b(const InstDev *insts, int ninst, hipStream_t st)
 {
     if (ninst <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_ke_b, dim3(kKeSlots, ninst), dim3(kSumBlock), 0, st, insts);
+    hipLaunchKernelGGL(k_energy_sums_b, dim3(kKeSlots, ninst), dim3(kSumBlock), 0, st, insts, 0);
     return hipGetLastError();
 }
 

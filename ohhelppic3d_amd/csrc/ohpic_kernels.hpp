@@ -110,10 +110,10 @@ hipError_t launch_begin_step_b(const InstDev *insts, const int *parity, int nins
                                int64_t max_ng, int max_ntiles, unsigned int *queue,
                                hipStream_t st);
 // launch_reduce_ke_b, the field-energy reduction of launch_efield_b, the
-// tight-bin check of the new buffer (parity ^ 1) and (out not null, group
-// steps) flags to out[i * kFlagSlots + k] with a parity flip unless instance i
+// tight-bin check of the new buffer (parity ^ 1), the flags to out[i *
+// kFlagSlots + k] and (flip, group steps) a parity flip unless instance i
 // overflowed a bin, in one launch at the end of a step
-hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst,
+hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst, bool flip,
                              unsigned long long *out, hipStream_t st);
 // zero the next buffer's bin words and charge grid and the flags (list mode)
 hipError_t launch_prepare_next_b(const InstDev *insts, const int *parity, int ninst,
