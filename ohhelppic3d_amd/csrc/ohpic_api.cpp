@@ -133,7 +133,7 @@ struct ohpic_ctx {
     double *d_lam[3]{};
     FftJob job{};                // Poisson transform of rho into phi
     FftJob *d_job = nullptr;
-    FftLaunch fft[3];            // launches of each axis' passes
+    FftSolve fft;                // launches of the solve
     std::vector<WorkItem> items;  // host copy of d_items
     uint64_t inst_ver = 0;       // bumped whenever h is uploaded
     uint64_t items_ver = 0;      // bumped whenever the work list changes
@@ -796,27 +796,22 @@ int do_deposit(ohpic_ctx *ctx)
 }
 
 // Poisson solve of the instance table `insts` (n instances, FFT jobs `jobs`)
-// from rho: five axis passes, node E and its energy partials (reduced when
-// reduce_e).
-hipError_t solve_passes(const FftJob *jobs, const InstDev *insts, int n, const FftLaunch fft[3],
-                        int max_eblocks, bool reduce_e, hipStream_t st)
+// from rho: axis passes, node E and its energy partials (reduced when
+// reduce_e).  step: the start of a step, of which fft_by_planes takes care.
+hipError_t solve_passes(const FftJob *jobs, const InstDev *insts, int n, const FftSolve &fft,
+                        const FftStep *step, int max_eblocks, bool reduce_e, hipStream_t st)
 {
-    hipError_t e = fft_pass(kPassR2hcXFromSrc, jobs, n, fft[0], st);
-    if (e == hipSuccess) e = fft_pass(kPassR2hcY, jobs, n, fft[1], st);
-    if (e == hipSuccess) e = fft_pass(kPassPoissonZ, jobs, n, fft[2], st);
-    if (e == hipSuccess) e = fft_pass(kPassHc2rY, jobs, n, fft[1], st);
-    if (e == hipSuccess) e = fft_pass(kPassHc2rXScaled, jobs, n, fft[0], st);
-    if (e == hipSuccess) e = launch_efield_b(insts, n, max_eblocks, reduce_e, st);
-    return e;
+    const hipError_t e = fft_poisson(jobs, n, fft, step, st);
+    return e == hipSuccess ? launch_efield_b(insts, n, max_eblocks, reduce_e, st) : e;
 }
 
-// The field solve from rho (FFT passes, E); reduce_e: also the field-energy
-// sums (a step leaves them to its end-of-step reduction).
-int do_solve(ohpic_ctx *ctx, bool reduce_e)
+// The field solve from rho (FFT passes, E); of a step (start) the field-energy
+// sums are left to its end-of-step reduction, otherwise they are reduced.
+int do_solve(ohpic_ctx *ctx, const FftStep *start)
 {
     timer_begin(ctx, 1);
-    HIPCHK(ctx, solve_passes(ctx->d_job, ctx->d_inst, 1, ctx->fft,
-                             efield_blocks_of(ctx->n[0], ctx->n[1], ctx->n[2]), reduce_e, ctx->st));
+    HIPCHK(ctx, solve_passes(ctx->d_job, ctx->d_inst, 1, ctx->fft, start,
+                             efield_blocks_of(ctx->n[0], ctx->n[1], ctx->n[2]), !start, ctx->st));
     timer_end(ctx, 1);
     return OHPIC_OK;
 }
@@ -840,9 +835,11 @@ int one_step(ohpic_ctx *ctx)
     if (!ctx->rho_valid && (rc = do_deposit(ctx))) return rc;
     // rho from the charge grid and the next buffer's zeroing in one sweep,
     // the solve from rho, the step, and all energy sums in one reduction
-    HIPCHK(ctx, launch_begin_step_b(ctx->d_inst, parity_of(ctx), 1, ctx->ng, ctx->ntiles,
-                                    nullptr, ctx->st));
-    if ((rc = do_solve(ctx, false))) return rc;
+    const FftStep start{ctx->d_inst, parity_of(ctx), nullptr};
+    if (!fft_by_planes(ctx->fft))
+        HIPCHK(ctx, launch_begin_step_b(ctx->d_inst, parity_of(ctx), 1, ctx->ng, ctx->ntiles,
+                                        nullptr, ctx->st));
+    if ((rc = do_solve(ctx, &start))) return rc;
     timer_begin(ctx, 0);
     HIPCHK(ctx, run_particles(ctx, kModeFused));
     timer_end(ctx, 0);
@@ -1042,7 +1039,7 @@ struct ohpic_group {
     bool dirty = true;
     int64_t max_ng = 0;
     int max_ntiles = 0, max_rows = 0;  // max_rows: largest E-kernel block count
-    FftLaunch fft[3];
+    FftSolve fft;
     int T[3]{};
     int precision = -1, weight_order = -1;
     bool use_graph = true;
@@ -1202,7 +1199,7 @@ int group_refresh(ohpic_group *g)
         if (rc) return rc;
         g->max_ng = 0;
         g->max_ntiles = g->max_rows = 0;
-        for (FftLaunch &l : g->fft) l = FftLaunch();
+        g->fft = FftSolve();
         for (int i = 0; i < n; ++i) {
             ohpic_ctx *m = g->members[i];
             insts[i] = m->h;
@@ -1211,7 +1208,7 @@ int group_refresh(ohpic_group *g)
             g->max_ng = std::max(g->max_ng, m->ng);
             g->max_ntiles = std::max(g->max_ntiles, m->ntiles);
             g->max_rows = std::max(g->max_rows, efield_blocks_of(m->n[0], m->n[1], m->n[2]));
-            for (int a = 0; a < 3; ++a) fft_add(g->fft[a], m->ax[a], a, m->n[0], m->n[1], m->n[2]);
+            fft_solve_add(g->fft, m->job);
             g->seen_inst[i] = m->inst_ver;
             g->seen_items[i] = m->items_ver;
         }
@@ -1256,10 +1253,12 @@ hipError_t group_enqueue(ohpic_group *g, int k)
     const int n = (int)g->members.size();
     hipError_t e = hipSuccess;
     for (int s = 0; s < k && e == hipSuccess; ++s) {
-        e = launch_begin_step_b(g->d_insts, g->d_parity, n, g->max_ng, g->max_ntiles,
-                                g->persistent ? g->d_queue : nullptr, g->st);
+        const FftStep start{g->d_insts, g->d_parity, g->persistent ? g->d_queue : nullptr};
+        if (!fft_by_planes(g->fft))
+            e = launch_begin_step_b(g->d_insts, g->d_parity, n, g->max_ng, g->max_ntiles,
+                                    start.queue, g->st);
         if (e == hipSuccess)
-            e = solve_passes(g->d_jobs, g->d_insts, n, g->fft, g->max_rows, false, g->st);
+            e = solve_passes(g->d_jobs, g->d_insts, n, g->fft, &start, g->max_rows, false, g->st);
         if (e == hipSuccess) {
             if (g->persistent)
                 e = launch_particles_queue(g->precision, g->weight_order, g->T, g->ids, g->d_insts,
@@ -1674,9 +1673,10 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
             J.n[a] = ctx->n[a];
             J.ax[a] = ctx->ax[a];
             J.lam[a] = ctx->d_lam[a];
-            fft_add(ctx->fft[a], ctx->ax[a], a, c.nx, c.ny, c.nz);
         }
         J.inv_n = 1.0 / (double)ctx->ng;
+        fft_plan_planes(J);
+        fft_solve_add(ctx->fft, J);
         CREATE_CHK(dalloc(ctx, &ctx->d_job, 1));
         CREATE_HIP(hipMemcpyAsync(ctx->d_job, &J, sizeof J, hipMemcpyHostToDevice, ctx->st));
         CREATE_HIP(hipStreamSynchronize(ctx->st));
@@ -2020,7 +2020,7 @@ int ohpic_field_solve(ohpic_ctx *ctx)
     GateShared gate;
     if (!ctx) return fail(nullptr, OHPIC_EINVAL, "ctx is NULL");
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    int rc = do_solve(ctx, true);
+    int rc = do_solve(ctx, nullptr);
     if (rc) return rc;
     HIPCHK(ctx, hipStreamSynchronize(ctx->st));
     timers_collect(ctx);

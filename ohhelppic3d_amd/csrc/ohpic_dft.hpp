@@ -3,6 +3,11 @@
 
 #include <hip/hip_runtime.h>
 
+// Products and sums contract within one statement only, so that the same code
+// rounds the same in every kernel it is part of (an instance's transform may
+// run in either of two kernels, alone or in a group).
+#pragma clang fp contract(on)
+
 namespace ohpic {
 namespace {
 

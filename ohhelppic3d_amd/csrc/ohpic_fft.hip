@@ -474,6 +474,9 @@ __global__ void __launch_bounds__(kFftBlock)
 // each number of points and chosen once per step: with loops over 16 guarded
 // points the passes at 32^3 took 5.3 to 9.3 us.
 constexpr int kAbThreads = 64;
+constexpr int kPlaneWaves = 4;          // most wavefronts of k_fft_planes
+constexpr int64_t kPlaneLds = 64 << 10;  // and its LDS
+constexpr int64_t kMaxPlanes = 512;      // planes of a launch (fft_by_planes)
 
 // 1/d for 0 < d < 2^1000 (d = 0 gives inf, which the caller discards): the
 // hardware estimate (about 23 correct bits) refined by two Newton steps, so
@@ -524,145 +527,77 @@ __device__ __forceinline__ void with_points(int P, F &f)
 #undef OHPIC_POINTS
 }
 
-// FIXED: A and B when known at compile time (16 x 16), else 0.
-template <int KIND, int AXIS, bool FROM_SRC, bool SCALE, int FIXED>
-__global__ void __launch_bounds__(kAbThreads)
-k_fft_two_step(const FftJob *__restrict__ jobs)
+// One thread's place in a wavefront's complex lines of n = A B points: thread t
+// of line c, taking part in step 1 (as j = t) and step 2 (as k1 = t).
+struct TwoStep {
+    int A, B, n, L, c, t;
+    bool live, one, two;
+    int RA, RB;         // odd rows of the LDS exchanges
+    const cplx *tw;     // twiddles (LDS)
+    cplx *xl;           // the line's exchange buffer (LDS)
+    const double *lam;  // Poisson: lam_x + lam_y of the wavefront's real lines,
+    const double *lz;   // and lam_z of the modes (LDS)
+};
+
+__host__ __device__ inline int two_step_row(int A, int B)  // complex values per line
 {
-    extern __shared__ cplx ab_lds[];
-    const FftJob &J = jobs[blockIdx.y];
-    const int nx = J.n[0], ny = J.n[1], nz = J.n[2];
-    const FftAxisDev &ax = J.ax[AXIS];
-    // this launch's jobs: 16 x 16 or any other pair
-    if (ax.A == 0 || (FIXED == 16) != (ax.A == 16 && ax.B == 16)) return;
-    constexpr int R = 16;
-    const int A = FIXED ? FIXED : ax.A, B = FIXED ? FIXED : ax.B, n = A * B;
-    const int L = FIXED ? kAbThreads / FIXED : ax.ab_lines;
-    const int64_t ngroups = fft_groups(AXIS, 2 * L, nx, ny, nz);
-    if ((int64_t)blockIdx.x >= ngroups) return;
-    // neighbouring groups read the parts of the same 128-byte lines (y and z
-    // passes): keep them on one XCD
-    const int grp = xcd_remap((int)blockIdx.x, (int)ngroups);
-    const LineBlock lb = line_block<AXIS>(grp, 2 * L, nx, ny, nz);
-    const int tid = threadIdx.x;
+    const int ra = B * (A | 1), rb = A * (B | 1);
+    return ra > rb ? ra : rb;
+}
+
+__device__ __forceinline__ TwoStep two_step_of(int A, int B, int L, uint32_t mg_M, int lane,
+                                               const cplx *tw, cplx *xbuf)
+{
+    TwoStep w;
+    w.A = A;
+    w.B = B;
+    w.n = A * B;
+    w.L = L;
     const int M = max(A, B);
-    const int c = FIXED ? tid / FIXED : fastdiv(tid, ax.mg_M), t = tid - c * M;
-    const bool live = c < L;
-    const bool one = live && t < B, two = live && t < A;  // threads of the two steps
-    const int RA = A | 1, RB = B | 1;                     // odd rows of the LDS exchanges
-    cplx *tw = ab_lds;                                    // twiddles, then the exchange buffer
-    cplx *xl = ab_lds + n + (live ? c : 0) * max(B * RA, A * RB);
-    double *lam = reinterpret_cast<double *>(ab_lds + n + L * max(B * RA, A * RB));  // 2 L
-    double *lz = lam + 2 * L;                             // n
+    w.c = fastdiv(lane, mg_M);
+    w.t = lane - w.c * M;
+    w.live = w.c < L;
+    w.one = w.live && w.t < B;
+    w.two = w.live && w.t < A;
+    w.RA = A | 1;
+    w.RB = B | 1;
+    w.tw = tw;
+    w.xl = xbuf + (w.live ? w.c : 0) * two_step_row(A, B);
+    return w;
+}
 
-    // twiddles and z denominators on their way before the lines
-    constexpr int TQ = 256 / kAbThreads;
-    d2v wq[TQ];
-    double zq[TQ];
-#pragma unroll
-    for (int q = 0; q < TQ; ++q) {
-        const int i = min(tid + q * kAbThreads, n - 1);
-        wq[q] = gload(reinterpret_cast<const d2v *>(ax.tw), i);
-        if (KIND == kFftPoisson) zq[q] = gload(J.lam[2], i);
-    }
-    auto stage_tables = [&]() __attribute__((always_inline))
-    {
-#pragma unroll
-        for (int q = 0; q < TQ; ++q) {
-            const int i = tid + q * kAbThreads;
-            if (i < n) {
-                tw[i] = cplx{wq[q].x, wq[q].y};
-                if (KIND == kFftPoisson) lz[i] = zq[q];
-            }
-        }
-        if (KIND == kFftPoisson && tid < 2 * L) {
-            // lam_x + lam_y of real line tid; -1 marks the DC line (ix = iy = 0);
-            // lines past the grid's end get 1 (they hold zeros; no 0/0)
-            double v = 1.0;
-            if (tid < lb.nvalid) {
-                const int l = (int)lb.base + tid;  // < nx ny <= 2^20
-                const int iy = l / nx, ix = l - iy * nx;
-                v = (l == 0) ? -1.0 : gload(J.lam[0], ix) + gload(J.lam[1], iy);
-            }
-            lam[tid] = v;
-        }
-    };
+// Transforms the wavefront's lines in `a`.  load(count, step) fills a[m] with
+// point t + step m of the thread's line, m < count; stage() makes the LDS
+// tables ready; store(count, step) takes a[m] as point t + step m.
+template <int KIND, int FIXED, class Load, class Stage, class Store>
+__device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], Load &&load,
+                                               Stage &&stage, Store &&store)
+{
+    constexpr int SIGN = KIND == kFftHC2R ? +1 : -1;
+    using Sign = std::integral_constant<int, SIGN>;
+    using Back = std::integral_constant<int, +1>;
+    const int A = FIXED ? FIXED : W.A, B = FIXED ? FIXED : W.B, n = A * B;
+    const int RA = FIXED ? (FIXED | 1) : W.RA, RB = FIXED ? (FIXED | 1) : W.RB;
+    const int t = W.t;
+    const bool one = W.one, two = W.two;
+    cplx *xl = W.xl;
 
-    // real lines 2c (re) and 2c + 1 (im): y and z lines are adjacent, one
-    // 16-byte access per point when every pair is aligned (an even stride; the
-    // number of lines is then even too)
-    const bool v16 = AXIS != 0 && (lb.estride & 1) == 0;
-    const bool va = live && 2 * c < lb.nvalid, vb = live && 2 * c + 1 < lb.nvalid;
-    const uint32_t g1 = (uint32_t)lb.gstride;
-    const uint32_t lane0 = (uint32_t)(2 * c) * g1 + (uint32_t)t * (uint32_t)lb.estride;
-    // points t, t + step, ... of a thread's lines (the step is uniform)
-    cplx a[16];
-    auto load = [&](auto count, int step) __attribute__((always_inline))
-    {
-        constexpr int P = decltype(count)::value;
-        const gmem_t<double> *s = as_global((FROM_SRC ? J.src : J.data) + lb.base);
-        const int64_t inc = step * lb.estride;
-#pragma unroll
-        for (int m = 0; m < P; ++m) a[m] = cplx{0.0, 0.0};
-        if (AXIS != 0 && v16) {
-            if (va)
-#pragma unroll
-                for (int m = 0; m < P; ++m) {
-                    const d2v v = ((const gmem_t<d2v> *)(s + m * inc))[lane0 >> 1];
-                    a[m] = cplx{v.x, v.y};
-                }
-        } else {
-            if (va)
-#pragma unroll
-                for (int m = 0; m < P; ++m) a[m].re = (s + m * inc)[lane0];
-            if (vb)
-#pragma unroll
-                for (int m = 0; m < P; ++m) a[m].im = (s + m * inc)[lane0 + g1];
-        }
-    };
-    auto store = [&](auto count, int step) __attribute__((always_inline))
-    {
-        constexpr int P = decltype(count)::value;
-        gmem_t<double> *d = as_global(J.data + lb.base);
-        const int64_t inc = step * lb.estride;
-        if (AXIS != 0 && v16) {
-            if (va)
-#pragma unroll
-                for (int m = 0; m < P; ++m) {
-                    d2v w;
-                    w.x = a[m].re;
-                    w.y = a[m].im;
-                    ((gmem_t<d2v> *)(d + m * inc))[lane0 >> 1] = w;
-                }
-        } else {
-            if (va)
-#pragma unroll
-                for (int m = 0; m < P; ++m) (d + m * inc)[lane0] = a[m].re;
-            if (vb)
-#pragma unroll
-                for (int m = 0; m < P; ++m) (d + m * inc)[lane0 + g1] = a[m].im;
-        }
-    };
     // a[k] *= exp(SIGN 2 pi i t k / n)
     auto twiddles = [&](auto sign, auto count) __attribute__((always_inline))
     {
 #pragma unroll
         for (int k = 1; k < decltype(count)::value; ++k) {
-            const cplx w = tw[t * k];
+            const cplx w = W.tw[t * k];
             a[k] = cmul(a[k], cplx{w.re, decltype(sign)::value < 0 ? w.im : -w.im});
         }
     };
-    constexpr int SIGN = KIND == kFftHC2R ? +1 : -1;
-    using Sign = std::integral_constant<int, SIGN>;
-    using Back = std::integral_constant<int, +1>;
-
     // step 1 (thread j = t), twiddles, transpose
     auto first = [&](auto count) __attribute__((always_inline))
     {
         constexpr int P = decltype(count)::value;  // A
         constexpr int RP = P | 1;
         if (one) load(count, B);
-        stage_tables();
+        stage();
         wave_exchange();
         if (KIND == kFftHC2R) {
             // halfcomplex values V_p of both lines -> packed spectrum Z = A + i B
@@ -712,15 +647,7 @@ k_fft_two_step(const FftJob *__restrict__ jobs)
             Dft<SIGN, P>::run(a);
         }
         if (KIND == kFftHC2R) {
-            if (two) {
-                if (SCALE) {
-                    const double scale = J.inv_n;
-#pragma unroll
-                    for (int k2 = 0; k2 < P; ++k2)
-                        a[k2] = cplx{a[k2].re * scale, a[k2].im * scale};
-                }
-                store(count, A);
-            }
+            if (two) store(count, A);
             return;
         }
         // each mode meets its partner n - k
@@ -733,8 +660,8 @@ k_fft_two_step(const FftJob *__restrict__ jobs)
         if (two) {
             // mode n - k: row P - 1 - k2, or P - k2 (mod P) for t = 0
             const cplx *x = t == 0 ? xl + RA : xl + A - t;
-            const double lam_a = KIND == kFftPoisson ? lam[2 * c] : 0.0;
-            const double lam_b = KIND == kFftPoisson ? lam[2 * c + 1] : 0.0;
+            const double lam_a = KIND == kFftPoisson ? W.lam[2 * W.c] : 0.0;
+            const double lam_b = KIND == kFftPoisson ? W.lam[2 * W.c + 1] : 0.0;
             const double lxa = lam_a < 0.0 ? 0.0 : lam_a, lxb = lam_b < 0.0 ? 0.0 : lam_b;
 #pragma unroll
             for (int k2 = 0; k2 < P; ++k2) {
@@ -754,7 +681,7 @@ k_fft_two_step(const FftJob *__restrict__ jobs)
                     // A_k and B_k divided by their lines' denominators (the DC
                     // line's k = 0 mode, whose denominator is 0, set to zero),
                     // repacked as A' + i B'
-                    const double ra = fast_recip(lxa + lz[k]), rb = fast_recip(lxb + lz[k]);
+                    const double ra = fast_recip(lxa + W.lz[k]), rb = fast_recip(lxb + W.lz[k]);
                     const double sa = (lam_a < 0.0 && k == 0) ? 0.0 : 0.5 * ra;
                     const double sb = (lam_b < 0.0 && k == 0) ? 0.0 : 0.5 * rb;
                     const cplx U = {sa * (zk.re + zm.re), sa * (zk.im - zm.im)};
@@ -793,6 +720,333 @@ k_fft_two_step(const FftJob *__restrict__ jobs)
     if (KIND == kFftPoisson) with_points<FIXED>(A, third);
 }
 
+// Line access of a group of 2 L real lines in global memory: complex line c is
+// real lines 2c (re) and 2c + 1 (im).  y and z lines are adjacent: one 16-byte
+// access per point when every pair is aligned (an even stride; the number of
+// lines is then even too).
+template <int AXIS>
+struct LineAccess {
+    int64_t estride;
+    uint32_t g1, lane0;  // offsets of the second line and of the thread's first point
+    bool v16, va, vb;    // pair access; the two lines are there
+    __device__ __forceinline__ LineAccess(const LineBlock &lb, const TwoStep &W)
+    {
+        estride = lb.estride;
+        g1 = (uint32_t)lb.gstride;
+        lane0 = (uint32_t)(2 * W.c) * g1 + (uint32_t)W.t * (uint32_t)lb.estride;
+        v16 = AXIS != 0 && (lb.estride & 1) == 0;
+        va = W.live && 2 * W.c < lb.nvalid;
+        vb = W.live && 2 * W.c + 1 < lb.nvalid;
+    }
+    template <int P>
+    __device__ __forceinline__ void load(cplx (&a)[16], const double *p, int step) const
+    {
+        const gmem_t<double> *s = as_global(p);
+        const int64_t inc = step * estride;
+#pragma unroll
+        for (int m = 0; m < P; ++m) a[m] = cplx{0.0, 0.0};
+        if (AXIS != 0 && v16) {
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    const d2v v = ((const gmem_t<d2v> *)(s + m * inc))[lane0 >> 1];
+                    a[m] = cplx{v.x, v.y};
+                }
+        } else {
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) a[m].re = (s + m * inc)[lane0];
+            if (vb)
+#pragma unroll
+                for (int m = 0; m < P; ++m) a[m].im = (s + m * inc)[lane0 + g1];
+        }
+    }
+    template <int P>
+    __device__ __forceinline__ void store(const cplx (&a)[16], double *p, int step) const
+    {
+        gmem_t<double> *d = as_global(p);
+        const int64_t inc = step * estride;
+        if (AXIS != 0 && v16) {
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    d2v w;
+                    w.x = a[m].re;
+                    w.y = a[m].im;
+                    ((gmem_t<d2v> *)(d + m * inc))[lane0 >> 1] = w;
+                }
+        } else {
+            if (va)
+#pragma unroll
+                for (int m = 0; m < P; ++m) (d + m * inc)[lane0] = a[m].re;
+            if (vb)
+#pragma unroll
+                for (int m = 0; m < P; ++m) (d + m * inc)[lane0 + g1] = a[m].im;
+        }
+    }
+};
+
+// Groups of `lines` real lines of an axis pass; x lines of a job whose planes
+// can go by k_fft_planes (plane != 0) are grouped plane by plane.
+__host__ __device__ inline int64_t two_step_groups(int axis, int lines, int nx, int ny, int nz,
+                                                   int plane)
+{
+    if (axis == 0 && plane) return (int64_t)((ny + lines - 1) / lines) * nz;
+    return fft_groups(axis, lines, nx, ny, nz);
+}
+
+// FIXED: A and B when known at compile time (16 x 16), else 0.
+template <int KIND, int AXIS, bool FROM_SRC, bool SCALE, int FIXED>
+__global__ void __launch_bounds__(kAbThreads) k_fft_two_step(const FftJob *__restrict__ jobs)
+{
+    extern __shared__ cplx ab_lds[];
+    const FftJob &J = jobs[blockIdx.y];
+    const int nx = J.n[0], ny = J.n[1], nz = J.n[2];
+    const FftAxisDev &ax = J.ax[AXIS];
+    // this launch's jobs: 16 x 16 or any other pair
+    if (ax.A == 0 || (FIXED == 16) != (ax.A == 16 && ax.B == 16)) return;
+    const int A = FIXED ? FIXED : ax.A, B = FIXED ? FIXED : ax.B, n = A * B;
+    const int L = FIXED ? kAbThreads / FIXED : ax.ab_lines;
+    const int64_t ngroups = two_step_groups(AXIS, 2 * L, nx, ny, nz, J.plane);
+    if ((int64_t)blockIdx.x >= ngroups) return;
+    // neighbouring groups read the parts of the same 128-byte lines (y and z
+    // passes): keep them on one XCD
+    const int grp = xcd_remap((int)blockIdx.x, (int)ngroups);
+    LineBlock lb;
+    if (AXIS == 0 && J.plane) {
+        // rows pair up within their plane, as in k_fft_planes
+        const int gpp = (int)(ngroups / nz), iz = grp / gpp, row = (grp - iz * gpp) * 2 * L;
+        lb.base = (int64_t)nx * ((int64_t)ny * iz + row);
+        lb.gstride = nx;
+        lb.estride = 1;
+        lb.nvalid = min(2 * L, ny - row);
+    } else {
+        lb = line_block<AXIS>(grp, 2 * L, nx, ny, nz);
+    }
+    const int tid = threadIdx.x;
+    cplx *tw = ab_lds;  // twiddles, then the exchange buffers
+    TwoStep W = two_step_of(A, B, L, FIXED ? fastdiv_magic(FIXED) : ax.mg_M, tid, tw, ab_lds + n);
+    double *lam = reinterpret_cast<double *>(ab_lds + n + L * two_step_row(A, B));  // 2 L
+    double *lz = lam + 2 * L;                                                       // n
+    W.lam = lam;
+    W.lz = lz;
+
+    // twiddles and z denominators on their way before the lines
+    constexpr int TQ = 256 / kAbThreads;
+    d2v wq[TQ];
+    double zq[TQ];
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+        const int i = min(tid + q * kAbThreads, n - 1);
+        wq[q] = gload(reinterpret_cast<const d2v *>(ax.tw), i);
+        if (KIND == kFftPoisson) zq[q] = gload(J.lam[2], i);
+    }
+    auto stage = [&]() __attribute__((always_inline))
+    {
+#pragma unroll
+        for (int q = 0; q < TQ; ++q) {
+            const int i = tid + q * kAbThreads;
+            if (i < n) {
+                tw[i] = cplx{wq[q].x, wq[q].y};
+                if (KIND == kFftPoisson) lz[i] = zq[q];
+            }
+        }
+        if (KIND == kFftPoisson && tid < 2 * L) {
+            // lam_x + lam_y of real line tid; -1 marks the DC line (ix = iy = 0);
+            // lines past the grid's end get 1 (they hold zeros; no 0/0)
+            double v = 1.0;
+            if (tid < lb.nvalid) {
+                const int l = (int)lb.base + tid;  // < nx ny <= 2^20
+                const int iy = l / nx, ix = l - iy * nx;
+                v = (l == 0) ? -1.0 : gload(J.lam[0], ix) + gload(J.lam[1], iy);
+            }
+            lam[tid] = v;
+        }
+    };
+    const LineAccess<AXIS> acc(lb, W);
+    cplx a[16];
+    auto load = [&](auto count, int step) __attribute__((always_inline))
+    {
+        acc.template load<decltype(count)::value>(a, (FROM_SRC ? J.src : J.data) + lb.base, step);
+    };
+    auto store = [&](auto count, int step) __attribute__((always_inline))
+    {
+        constexpr int P = decltype(count)::value;
+        if (SCALE) {
+            const double scale = J.inv_n;
+#pragma unroll
+            for (int m = 0; m < P; ++m) a[m] = cplx{a[m].re * scale, a[m].im * scale};
+        }
+        acc.template store<P>(a, J.data + lb.base, step);
+    };
+    two_step_lines<KIND, FIXED>(W, a, load, stage, store);
+}
+
+// ------------------------------------------------ x and y passes by planes
+// Where the x and y lengths of every job take the two steps, a z plane fits in
+// LDS with at most kPlaneWaves wavefronts of lines (fft_plan_planes) and there
+// are few planes (fft_by_planes), one launch does both passes, a workgroup per
+// plane: x then y (FWD) or y then x, the plane in LDS in between.  At such
+// sizes a pass is latency; this saves the second one's launch, its trip through
+// memory and the gap between the two: at 32^3 7.8 and 7.0 us against 4.5 + 4.6
+// and 4.7 + 4.3 and the gaps.  STEP: at the start of a step rho comes from the
+// charge grid on the way, and a wavefront of its own does the rest of
+// launch_begin_step_b (9.7 us; k_begin_step_b and its gap took 4).  Steps:
+// 32^3 92.1 -> 85.7 us, 45x50x63 147.0 -> 140.6, eight small instances 945 ->
+// 895 per 8 steps.
+// The limits: with 1280 planes (a group of 32 members of 16 to 64 cells) the
+// pair took 25 us each way for the members that could, 21 to 24 by axis for all
+// of them, since 200 registers and the planes' LDS leave few wavefronts per CU;
+// 40x40x500 and 48x48x512 solve in 71 and 82 us against 77 and 89.
+template <bool FWD, bool STEP>
+__global__ void __launch_bounds__((kPlaneWaves + 1) * 64)
+    k_fft_planes(const FftJob *__restrict__ jobs, FftStep step0)
+{
+    extern __shared__ cplx ab_lds[];
+    const FftJob &J = jobs[blockIdx.y];
+    const int nx = J.n[0], ny = J.n[1], nz = J.n[2];
+    const int waves = J.plane;  // wavefronts at work
+    if ((int)blockIdx.x >= nz) return;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const InstDev *I = STEP ? step0.insts + blockIdx.y : nullptr;
+    const int par = STEP ? step0.parity[blockIdx.y] : 0;
+    const FftAxisDev &ax = J.ax[0], &ay = J.ax[1];
+    const int ps = nx | 1;  // row of the plane: odd, so columns and rows spread over the banks
+    cplx *twx = ab_lds, *twy = twx + nx, *xbuf = twy + ny;
+    const int row = max(ax.ab_lines * two_step_row(ax.A, ax.B), ay.ab_lines * two_step_row(ay.A, ay.B));
+    double *plane = reinterpret_cast<double *>(xbuf + waves * row);
+    xbuf += min(wave, waves - 1) * row;
+    const int64_t base = (int64_t)nx * ny * blockIdx.x;
+    auto stage = [&]() __attribute__((always_inline))
+    {
+        for (int i = tid; i < nx; i += (int)blockDim.x) {
+            const d2v w = gload(reinterpret_cast<const d2v *>(ax.tw), i);
+            twx[i] = cplx{w.x, w.y};
+        }
+        for (int i = tid; i < ny; i += (int)blockDim.x) {
+            const d2v w = gload(reinterpret_cast<const d2v *>(ay.tw), i);
+            twy[i] = cplx{w.x, w.y};
+        }
+        __syncthreads();
+    };
+    auto staged = []() {};
+    cplx a[16];
+    constexpr int KIND = FWD ? kFftR2HC : kFftHC2R;
+    auto x_lines = [&](int g, auto &stage) __attribute__((always_inline))
+    {
+        const TwoStep W = two_step_of(ax.A, ax.B, ax.ab_lines, ax.mg_M, lane, twx, xbuf);
+        LineBlock lb;
+        lb.base = base + (int64_t)(g * 2 * W.L) * nx;
+        lb.gstride = nx;
+        lb.estride = 1;
+        lb.nvalid = min(2 * W.L, ny - g * 2 * W.L);
+        const LineAccess<0> acc(lb, W);
+        double *p0 = plane + (g * 2 * W.L + 2 * W.c) * ps + W.t;
+        auto load = [&](auto count, int step) __attribute__((always_inline))
+        {
+            constexpr int P = decltype(count)::value;
+            if (FWD && STEP) {
+                acc.template load<P>(a, (const double *)I->rho_acc[par] + lb.base, step);
+                const double scale = I->fix_inv;
+                cplx z[16];
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    a[m].re = (double)__double_as_longlong(a[m].re) * scale;
+                    a[m].im = (double)__double_as_longlong(a[m].im) * scale;
+                    z[m] = cplx{0.0, 0.0};
+                }
+                acc.template store<P>(a, I->rho + lb.base, step);
+                acc.template store<P>(z, (double *)I->rho_acc[par ^ 1] + lb.base, step);
+            } else if (FWD) {
+                acc.template load<P>(a, J.src + lb.base, step);
+            } else {
+#pragma unroll
+                for (int m = 0; m < P; ++m)
+                    a[m] = cplx{acc.va ? p0[m * step] : 0.0, acc.vb ? p0[m * step + ps] : 0.0};
+            }
+        };
+        auto store = [&](auto count, int step) __attribute__((always_inline))
+        {
+            constexpr int P = decltype(count)::value;
+            if (FWD) {
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    if (acc.va) p0[m * step] = a[m].re;
+                    if (acc.vb) p0[m * step + ps] = a[m].im;
+                }
+            } else {
+                const double scale = J.inv_n;
+#pragma unroll
+                for (int m = 0; m < P; ++m) a[m] = cplx{a[m].re * scale, a[m].im * scale};
+                acc.template store<P>(a, J.data + lb.base, step);
+            }
+        };
+        two_step_lines<KIND, 0>(W, a, load, stage, store);
+    };
+    auto y_lines = [&](int g, auto &stage) __attribute__((always_inline))
+    {
+        const TwoStep W = two_step_of(ay.A, ay.B, ay.ab_lines, ay.mg_M, lane, twy, xbuf);
+        LineBlock lb;
+        lb.base = base + g * 2 * W.L;
+        lb.gstride = 1;
+        lb.estride = nx;
+        lb.nvalid = min(2 * W.L, nx - g * 2 * W.L);
+        const LineAccess<1> acc(lb, W);
+        double *p0 = plane + W.t * ps + g * 2 * W.L + 2 * W.c;
+        auto load = [&](auto count, int step) __attribute__((always_inline))
+        {
+            constexpr int P = decltype(count)::value;
+            if (!FWD) {
+                acc.template load<P>(a, J.data + lb.base, step);
+            } else {
+#pragma unroll
+                for (int m = 0; m < P; ++m)
+                    a[m] = cplx{acc.va ? p0[m * step * ps] : 0.0,
+                                acc.vb ? p0[m * step * ps + 1] : 0.0};
+            }
+        };
+        auto store = [&](auto count, int step) __attribute__((always_inline))
+        {
+            constexpr int P = decltype(count)::value;
+            if (!FWD) {
+#pragma unroll
+                for (int m = 0; m < P; ++m) {
+                    if (acc.va) p0[m * step * ps] = a[m].re;
+                    if (acc.vb) p0[m * step * ps + 1] = a[m].im;
+                }
+            } else {
+                acc.template store<P>(a, J.data + lb.base, step);
+            }
+        };
+        two_step_lines<KIND, 0>(W, a, load, stage, store);
+    };
+    const int gx = (ny + 2 * ax.ab_lines - 1) / (2 * ax.ab_lines);
+    const int gy = (nx + 2 * ay.ab_lines - 1) / (2 * ay.ab_lines);
+    // one group of lines per wavefront and axis (waves is the larger number of
+    // groups); every wavefront passes the barrier of stage() once
+    if (FWD) {
+        if (wave < gx)
+            x_lines(wave, stage);
+        else
+            stage();
+        if (STEP && wave == waves) {
+            // the wavefront beyond those of the lines
+            if (step0.queue && blockIdx.x == 0 && blockIdx.y == 0 && lane == 0) *step0.queue = 0u;
+            if (blockIdx.x == 0 && lane < kFlagWords) I->flags[lane] = 0ull;
+            reserve_next(I, par, (int64_t)blockIdx.x * 64 + lane, (int64_t)nz * 64);
+        }
+        __syncthreads();
+        if (wave < gy) y_lines(wave, staged);
+    } else {
+        if (wave < gy)
+            y_lines(wave, stage);
+        else
+            stage();
+        __syncthreads();
+        if (wave < gx) x_lines(wave, staged);
+    }
+}
+
 }  // namespace
 
 void fft_plan_divisors(FftAxisDev &ax)
@@ -826,19 +1080,58 @@ void fft_two_step(int n, int *A, int *B)
 int64_t fft_two_step_lds(int A, int B)
 {
     const int L = kAbThreads / (A > B ? A : B);
-    const int ra = B * (A | 1), rb = A * (B | 1);
-    return (int64_t)(A * B + L * (ra > rb ? ra : rb)) * (int64_t)sizeof(double2) +
+    return (int64_t)(A * B + L * two_step_row(A, B)) * (int64_t)sizeof(double2) +
            (2 * L + A * B) * (int64_t)sizeof(double);
 }
 
-void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz)
+// LDS bytes of k_fft_planes with `waves` wavefronts
+static int64_t plane_lds(const FftJob &J, int waves)
+{
+    const FftAxisDev &ax = J.ax[0], &ay = J.ax[1];
+    const int row = std::max(ax.ab_lines * two_step_row(ax.A, ax.B),
+                             ay.ab_lines * two_step_row(ay.A, ay.B));
+    return (int64_t)(ax.n + ay.n + waves * row) * (int64_t)sizeof(double2) +
+           (int64_t)(ax.n | 1) * ay.n * (int64_t)sizeof(double);
+}
+
+void fft_plan_planes(FftJob &J)
+{
+    J.plane = 0;
+    const FftAxisDev &ax = J.ax[0], &ay = J.ax[1];
+    if (ax.A == 0 || ay.A == 0) return;
+    const int gx = (ay.n + 2 * ax.ab_lines - 1) / (2 * ax.ab_lines);
+    const int gy = (ax.n + 2 * ay.ab_lines - 1) / (2 * ay.ab_lines);
+    const int waves = std::max(gx, gy);
+    if (waves > kPlaneWaves || plane_lds(J, waves) > kPlaneLds) return;
+    J.plane = waves;
+}
+
+void fft_solve_add(FftSolve &l, const FftJob &J)
+{
+    for (int a = 0; a < 3; ++a) fft_add(l.ax[a], J.ax[a], a, J.n[0], J.n[1], J.n[2], J.plane);
+    if (J.plane == 0) {
+        l.all_planes = false;
+        return;
+    }
+    l.planes = std::max(l.planes, J.n[2]);
+    l.total_planes += J.n[2];
+    l.plane_waves = std::max(l.plane_waves, J.plane);
+    l.lds = std::max(l.lds, plane_lds(J, J.plane));
+}
+
+bool fft_by_planes(const FftSolve &l)
+{
+    return l.all_planes && l.total_planes > 0 && l.total_planes <= kMaxPlanes;
+}
+
+void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz, int plane)
 {
     if (ax.A == 0) {
         l.groups = std::max(l.groups, fft_groups(axis, fft_group_lines(ax.n), nx, ny, nz));
         l.rs = std::max(l.rs, fft_radix_set(ax));
         return;
     }
-    const int64_t g = fft_groups(axis, 2 * ax.ab_lines, nx, ny, nz);
+    const int64_t g = two_step_groups(axis, 2 * ax.ab_lines, nx, ny, nz, plane);
     if (ax.A == 16 && ax.B == 16) {
         l.groups16 = std::max(l.groups16, g);
     } else {
@@ -881,6 +1174,32 @@ static hipError_t launch_pass(const FftJob *jobs, int njobs, const FftLaunch &l,
                            (unsigned)l.lds_ab, st, jobs);
     }
     return hipGetLastError();
+}
+
+hipError_t fft_poisson(const FftJob *jobs, int njobs, const FftSolve &l, const FftStep *step,
+                       hipStream_t st)
+{
+    if (njobs <= 0) return hipSuccess;
+    const bool planes = fft_by_planes(l);
+    const dim3 g((unsigned)l.planes, (unsigned)njobs), b((unsigned)(64 * l.plane_waves)),
+        b1((unsigned)(64 * (l.plane_waves + 1)));
+    hipError_t e = hipSuccess;
+    if (planes && step)
+        hipLaunchKernelGGL((k_fft_planes<true, true>), g, b1, (unsigned)l.lds, st, jobs, *step);
+    else if (planes)
+        hipLaunchKernelGGL((k_fft_planes<true, false>), g, b, (unsigned)l.lds, st, jobs, FftStep{});
+    else {
+        e = fft_pass(kPassR2hcXFromSrc, jobs, njobs, l.ax[0], st);
+        if (e == hipSuccess) e = fft_pass(kPassR2hcY, jobs, njobs, l.ax[1], st);
+    }
+    if (e == hipSuccess) e = fft_pass(kPassPoissonZ, jobs, njobs, l.ax[2], st);
+    if (e == hipSuccess && planes)
+        hipLaunchKernelGGL((k_fft_planes<false, false>), g, b, (unsigned)l.lds, st, jobs, FftStep{});
+    else {
+        if (e == hipSuccess) e = fft_pass(kPassHc2rY, jobs, njobs, l.ax[1], st);
+        if (e == hipSuccess) e = fft_pass(kPassHc2rXScaled, jobs, njobs, l.ax[0], st);
+    }
+    return e == hipSuccess ? hipGetLastError() : e;
 }
 
 hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, const FftLaunch &l,

@@ -35,6 +35,8 @@ __host__ __device__ inline uint32_t fastdiv_magic(uint32_t d)
     return d <= 1 ? 0u : (uint32_t)((0x100000000ull + d - 1) / d);
 }
 
+struct InstDev;
+
 struct FftAxisDev {
     int n;
     int nfac;
@@ -105,6 +107,26 @@ struct FftJob {
     FftAxisDev ax[3];
     const double *lam[3];  // (2 sin(pi k/n))^2 per axis
     double inv_n;          // 1 / (nx ny nz)
+    int plane;             // wavefronts per plane when the x and y passes can go
+                           // by planes (fft_plan_planes), or 0
+};
+
+// Launches of a Poisson solve over a table of jobs.
+struct FftSolve {
+    FftLaunch ax[3];          // the axis passes
+    bool all_planes = true;   // every job's x and y passes can go by planes:
+    int planes = 0;           // most planes of a job,
+    int64_t total_planes = 0; // planes of all jobs,
+    int plane_waves = 0;      // most wavefronts and LDS bytes
+    int64_t lds = 0;
+};
+
+// Start of a step whose x and y passes go by planes: rho comes from the charge
+// grids of insts[job], and what launch_begin_step_b does is done on the way.
+struct FftStep {
+    const InstDev *insts;
+    const int *parity;
+    unsigned int *queue;
 };
 
 enum FftPass : int {
@@ -121,11 +143,25 @@ enum FftPass : int {
 int fft_radix_set(const FftAxisDev &ax);
 
 // Adds a job's axis to the launch of that axis' passes.
-void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz);
+void fft_add(FftLaunch &l, const FftAxisDev &ax, int axis, int nx, int ny, int nz, int plane = 0);
 
 // One axis pass for every job of the device table `jobs`.  Each job's form
 // depends on its axis length alone, so it computes the same in every table.
 hipError_t fft_pass(FftPass pass, const FftJob *jobs, int njobs, const FftLaunch &l,
                     hipStream_t st);
+
+// Sets J.plane from J.n and J.ax.
+void fft_plan_planes(FftJob &J);
+
+// Adds a job to a solve's launches.
+void fft_solve_add(FftSolve &l, const FftJob &J);
+
+// The solve's x and y passes go by planes.
+bool fft_by_planes(const FftSolve &l);
+
+// Forward x and y from src to data, the fused Poisson z pass, inverse y and x.
+// step (only when fft_by_planes): start the step too and take rho from there.
+hipError_t fft_poisson(const FftJob *jobs, int njobs, const FftSolve &l, const FftStep *step,
+                       hipStream_t st);
 
 }  // namespace ohpic

@@ -230,4 +230,20 @@ __device__ __forceinline__ int wrap_index(int i, int n)
     return i;
 }
 
+// Reserves each bin's whole current count as the front run of the next buffer:
+// the stayers always fit, and arrivals from neighbours are placed behind them
+// from the start.  (Done here, a tile's workgroup starts without waiting for a
+// reservation of its own, and a tile may be split among several workgroups.)
+__device__ __forceinline__ void reserve_next(const InstDev *I, int par, int64_t t0, int64_t stride)
+{
+    for (int s = 0; s < I->nspecies; ++s) {
+        const SpecDev &S = I->sp[s];
+        for (int64_t t = t0; t < I->ntiles; t += stride) {
+            const unsigned long long c = S.count[par][t];
+            const int cap = S.bin_cap[t], F = min(bin_front(c), cap);
+            S.count[par ^ 1][t] = (unsigned long long)(F + min(bin_back(c), cap - F));
+        }
+    }
+}
+
 }  // namespace ohpic

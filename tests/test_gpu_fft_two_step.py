@@ -94,3 +94,36 @@ def test_members_of_every_form_equal_alone(ohp):
     finally:
         for s in sims:
             s.close()
+
+
+# x and y lengths whose passes go by planes (up to 512 of them, up to four
+# wavefronts of lines, up to 64 KiB of LDS) and their nearest neighbours
+PLANES = ((4, 4, 1), (4, 4, 512), (4, 4, 520), (6, 45, 5), (45, 6, 5), (39, 26, 3), (55, 50, 3),
+          (64, 48, 4), (64, 64, 2), (32, 32, 32))
+
+
+@pytest.mark.parametrize("n", PLANES)
+def test_planes_equal_axis_passes(ohp, orc, n):
+    rho = np.random.default_rng(n[2]).standard_normal(n[0] * n[1] * n[2])
+    with poisson(ohp, n, rho) as sim:
+        sim.field_solve()
+        assert rel_l2(sim.grid(ohp.FIELD_PHI), orc.poisson(n, rho)) <= 1e-12
+
+    def make():
+        rng = np.random.default_rng(n[0])
+        cfg = ohp.SimConfig(n=n, qm=[-1.0, 1.0], q_macro=[-0.01, 0.01], capacity=[700, 300], dt=0.1)
+        sim = ohp.Simulation(cfg)
+        for s, m in enumerate((700, 300)):
+            sim.load_particles(s, *[rng.uniform(0, k, m) for k in n], *rng.normal(0, 0.3, (3, m)))
+        return sim
+
+    # alone, and beside a member with a 2-point axis, for which no launch of the
+    # group goes by planes: the same bit for bit
+    with make() as a, make() as b, poisson(ohp, (2, 2, 2), np.zeros(8)) as other:
+        a.step(3)
+        with ohp.Group() as grp:
+            grp.attach(b)
+            grp.attach(other)
+            grp.step(3)
+            for w in (ohp.FIELD_RHO, ohp.FIELD_PHI, ohp.FIELD_EX, ohp.FIELD_EY, ohp.FIELD_EZ):
+                assert np.array_equal(a.grid(w), b.grid(w))
