@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(kFftBlock)
 // inverse runs the same steps backwards.
 //
 // What bounds it: at 256^3 (16 x 16) a pass moves 16 B per node in 44 to 46 us,
-// 5.9 TB/s (52 to 63 us with radix-4 stages in LDS; the fused z pass takes 68,
+// 5.9 TB/s (52 to 63 us with radix-4 stages in LDS; the fused z pass takes 56,
 // its division included).  The passes of a small grid are one wavefront's
 // chain of a load, two or three exchanges and a store: at 32^3 4.2 to 6.9 us
 // each, where the LDS stages (2 to 5 round trips, twice the barriers) took 6.3
@@ -545,6 +545,15 @@ __host__ __device__ inline int two_step_row(int A, int B)  // complex values per
     return ra > rb ? ra : rb;
 }
 
+// The 16 x 16 z pass exchanges real and imaginary parts one after the other,
+// in half the LDS: with more registers and work per line than the other passes
+// it is short of wavefronts in flight (6 per CU, with the split 10):
+// 68 -> 56 us at 256^3.
+__host__ __device__ constexpr bool two_step_split(int kind, int fixed)
+{
+    return kind == kFftPoisson && fixed == 16;
+}
+
 __device__ __forceinline__ TwoStep two_step_of(int A, int B, int L, uint32_t mg_M, int lane,
                                                const cplx *tw, cplx *xbuf)
 {
@@ -591,6 +600,28 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
             a[k] = cmul(a[k], cplx{w.re, decltype(sign)::value < 0 ? w.im : -w.im});
         }
     };
+    // SPLIT: a[k] goes to place put(k) of the line's buffer and b[k] is read from
+    // place get(k), real parts first and then the imaginary ones, so the buffer
+    // holds doubles
+    constexpr bool SPLIT = two_step_split(KIND, FIXED);
+    auto exchange = [&](cplx (&b)[16], auto put, auto get) __attribute__((always_inline))
+    {
+        double *x = reinterpret_cast<double *>(xl), re[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[put(k)] = a[k].re;
+        wave_exchange();
+#pragma unroll
+        for (int k = 0; k < 16; ++k) re[k] = x[get(k)];
+        wave_exchange();
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[put(k)] = a[k].im;
+        wave_exchange();
+#pragma unroll
+        for (int k = 0; k < 16; ++k) b[k] = cplx{re[k], x[get(k)]};
+        wave_exchange();
+    };
+    auto by_row = [&](int k) __attribute__((always_inline)) { return t * 17 + k; };
+    auto by_column = [&](int k) __attribute__((always_inline)) { return k * 17 + t; };
     // step 1 (thread j = t), twiddles, transpose
     auto first = [&](auto count) __attribute__((always_inline))
     {
@@ -631,6 +662,10 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
         if (one) {
             Dft<SIGN, P>::run(a);
             twiddles(Sign(), count);
+            if (SPLIT) {
+                exchange(a, by_row, by_column);
+                return;
+            }
 #pragma unroll
             for (int k1 = 0; k1 < P; ++k1) xl[t * RP + k1] = a[k1];
         }
@@ -642,8 +677,9 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
         constexpr int P = decltype(count)::value;  // B
         constexpr int RP = P | 1;
         if (two) {
+            if (!SPLIT)
 #pragma unroll
-            for (int j = 0; j < P; ++j) a[j] = xl[j * RA + t];
+                for (int j = 0; j < P; ++j) a[j] = xl[j * RA + t];
             Dft<SIGN, P>::run(a);
         }
         if (KIND == kFftHC2R) {
@@ -651,12 +687,19 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
             return;
         }
         // each mode meets its partner n - k
-        wave_exchange();  // transpose reads done
-        if (two) {
+        cplx z[16];
+        if (SPLIT) {
+            exchange(z, by_column, [&](int k2) __attribute__((always_inline)) {
+                return t == 0 ? (k2 == 0 ? 0 : (16 - k2) * 17) : (15 - k2) * 17 + 16 - t;
+            });
+        } else {
+            wave_exchange();  // transpose reads done
+            if (two) {
 #pragma unroll
-            for (int k2 = 0; k2 < P; ++k2) xl[k2 * RA + t] = a[k2];
+                for (int k2 = 0; k2 < P; ++k2) xl[k2 * RA + t] = a[k2];
+            }
+            wave_exchange();
         }
-        wave_exchange();
         if (two) {
             // mode n - k: row P - 1 - k2, or P - k2 (mod P) for t = 0
             const cplx *x = t == 0 ? xl + RA : xl + A - t;
@@ -667,7 +710,7 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
             for (int k2 = 0; k2 < P; ++k2) {
                 const int k = t + A * k2;
                 const cplx zk = a[k2];
-                const cplx zm = k2 == 0 && t == 0 ? xl[0] : x[(P - 1 - k2) * RA];
+                const cplx zm = SPLIT ? z[k2] : k2 == 0 && t == 0 ? xl[0] : x[(P - 1 - k2) * RA];
                 if (KIND == kFftR2HC) {
                     // position k of the halfcomplex lines: of A_k = (Z_k +
                     // conj Z_{n-k}) / 2 and B_k = (Z_k - conj Z_{n-k}) / 2i the
@@ -695,10 +738,14 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
             return;
         }
         // inverse: DFT over k2 (thread k1 = t), twiddles, transpose
-        wave_exchange();  // partner reads done before the buffer is reused
+        if (!SPLIT) wave_exchange();  // partner reads done before the buffer is reused
         if (two) {
             Dft<+1, P>::run(a);
             twiddles(Back(), count);
+            if (SPLIT) {
+                exchange(a, by_row, by_column);
+                return;
+            }
 #pragma unroll
             for (int j = 0; j < P; ++j) xl[t * RP + j] = a[j];
         }
@@ -710,7 +757,8 @@ __device__ __forceinline__ void two_step_lines(const TwoStep &W, cplx (&a)[16], 
         constexpr int P = decltype(count)::value;  // A
         if (one) {
 #pragma unroll
-            for (int k1 = 0; k1 < P; ++k1) a[k1] = xl[k1 * RB + t];
+            for (int k1 = 0; k1 < P; ++k1)
+                if (!SPLIT) a[k1] = xl[k1 * RB + t];
             Dft<+1, P>::run(a);
             store(count, B);
         }
@@ -826,7 +874,11 @@ __global__ void __launch_bounds__(kAbThreads) k_fft_two_step(const FftJob *__res
     const int tid = threadIdx.x;
     cplx *tw = ab_lds;  // twiddles, then the exchange buffers
     TwoStep W = two_step_of(A, B, L, FIXED ? fastdiv_magic(FIXED) : ax.mg_M, tid, tw, ab_lds + n);
-    double *lam = reinterpret_cast<double *>(ab_lds + n + L * two_step_row(A, B));  // 2 L
+    constexpr bool SPLIT = two_step_split(KIND, FIXED);
+    if (SPLIT) W.xl = reinterpret_cast<cplx *>(reinterpret_cast<double *>(ab_lds + n) +
+                                               W.c * two_step_row(A, B));
+    double *lam = reinterpret_cast<double *>(ab_lds + n) +
+                  (SPLIT ? 1 : 2) * L * two_step_row(A, B);  // 2 L
     double *lz = lam + 2 * L;                                                       // n
     W.lam = lam;
     W.lz = lz;
@@ -1084,6 +1136,11 @@ int64_t fft_two_step_lds(int A, int B)
            (2 * L + A * B) * (int64_t)sizeof(double);
 }
 
+static int64_t two_step_split_lds()
+{
+    return fft_two_step_lds(16, 16) - 4 * two_step_row(16, 16) * (int64_t)sizeof(double);
+}
+
 // LDS bytes of k_fft_planes with `waves` wavefronts
 static int64_t plane_lds(const FftJob &J, int waves)
 {
@@ -1166,7 +1223,9 @@ static hipError_t launch_pass(const FftJob *jobs, int njobs, const FftLaunch &l,
     if (l.groups16 > 0) {
         const dim3 g((unsigned)round_up_xcds(l.groups16), (unsigned)njobs), b(kAbThreads);
         hipLaunchKernelGGL((k_fft_two_step<KIND, AXIS, FROM_SRC, SCALE, 16>), g, b,
-                           (unsigned)fft_two_step_lds(16, 16), st, jobs);
+                           (unsigned)(two_step_split(KIND, 16) ? two_step_split_lds()
+                                                               : fft_two_step_lds(16, 16)),
+                           st, jobs);
     }
     if (l.groups_ab > 0) {
         const dim3 g((unsigned)round_up_xcds(l.groups_ab), (unsigned)njobs), b(kAbThreads);
