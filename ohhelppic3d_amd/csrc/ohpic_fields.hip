@@ -32,7 +32,7 @@ __device__ __forceinline__ double wave_sum(double v)
 // difference of poisson_field_solver.f90:139-144 averaged onto nodes as at
 // :165-170, periodic.  blockIdx.y = instance; each block walks whole x rows
 // (32-bit row indexing) and writes its partial sums of rho*phi, |E|^2 and
-// rho to e_partial[3*block]; k_reduce_e_b adds them in block order.  With an
+// rho to e_partial[3*block]; k_energy_sums_b or k_end_step_b adds them.  With an
 // even nx every thread takes V = 2 neighbouring x points: 16-byte loads of
 // the centre, y and z neighbour pairs and of rho, 8-byte loads of the two x
 // neighbours outside the pair, 16-byte stores.

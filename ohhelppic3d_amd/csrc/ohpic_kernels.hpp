@@ -60,7 +60,7 @@ hipError_t launch_cell_counts(const InstDev *insts, int inst, int s, int par, in
 
 // The fused step as one resident grid of `blocks` workgroups that claim the
 // nitems work items in list order from *queue (which must be 0 at launch:
-// launch_begin_step_b zeroes it).  particles_queue_blocks: workgroups of that kernel
+// the start of a step zeroes it).  particles_queue_blocks: workgroups of that kernel
 // resident on the whole device.
 hipError_t launch_particles_queue(int precision, int weight_order, const int T[3], bool ids,
                                   const InstDev *insts, const WorkItem *items, int nitems,

@@ -225,7 +225,7 @@ __device__ __forceinline__ void load_meta(SpecMeta *meta, const InstDev *__restr
 }
 
 // The m particles of a chunk's front run are written.  The step started with
-// the whole count reserved (k_begin_step_b, k_reserve_next_b): a tile of one
+// the whole count reserved (k_begin_step_b, k_fft_planes or k_reserve_next_b): a tile of one
 // chunk releases what its leavers left unused; a chunk of several leaves its
 // count for k_close_chunks.
 __device__ __forceinline__ void publish_front(const InstDev *__restrict__ I, const SpecDev &S,
