@@ -37,18 +37,21 @@ inline int64_t bin_capacity(int64_t c, double slack)
 // one, 0.173 ms).  A real gradient is steeper than that and does not count.
 inline std::vector<int64_t> expected_counts(const std::vector<int64_t> &counts, const int nt[3])
 {
-    const int nx = nt[0], ny = nt[1], nz = nt[2];
     // one periodic 3-point sum per axis
     std::vector<int64_t> a(counts), b(counts.size());
-    const int n[3] = {nx, ny, nz};
-    const int64_t stride[3] = {1, nx, (int64_t)nx * ny};
+    const int64_t total = (int64_t)counts.size();
+    int64_t stride = 1;
     for (int ax = 0; ax < 3; ++ax) {
-        for (int64_t t = 0; t < (int64_t)a.size(); ++t) {
-            const int i = (int)(t / stride[ax] % n[ax]);
-            const int64_t lo = i > 0 ? t - stride[ax] : t + (n[ax] - 1) * stride[ax];
-            const int64_t hi = i + 1 < n[ax] ? t + stride[ax] : t - (n[ax] - 1) * stride[ax];
-            b[t] = a[lo] + a[t] + a[hi];
-        }
+        const int n = nt[ax];
+        for (int64_t t0 = 0; t0 < total; t0 += n * stride)
+            for (int i = 0; i < n; ++i) {
+                const int64_t *lo = &a[t0 + (i > 0 ? i - 1 : n - 1) * stride];
+                const int64_t *at = &a[t0 + i * stride];
+                const int64_t *hi = &a[t0 + (i + 1 < n ? i + 1 : 0) * stride];
+                int64_t *out = &b[t0 + i * stride];
+                for (int64_t k = 0; k < stride; ++k) out[k] = lo[k] + at[k] + hi[k];
+            }
+        stride *= n;
         a.swap(b);
     }
     for (size_t t = 0; t < a.size(); ++t) {
