@@ -22,22 +22,25 @@ SOURCES = ["ohpic_particles.hip", "ohpic_particles_mixed.hip", "ohpic_fields.hip
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("OHPIC_ARCH", "gfx950")
 
-# -packed-fp32-ops keeps the compiler from emitting packed FP32 VALU ops.  The
-# atomic optimizer is off: it turns one lane's LDS counter add into a wave-wide
-# reduction that waits for its result at once, while the particle kernels need
-# it only after the charge deposit (they combine lanes themselves).
+# -packed-fp32-ops keeps the compiler from emitting packed FP32 VALU ops.
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17", "-Wall",
     "-Wno-unused-result", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-mllvm", "-amdgpu-atomic-optimizer-strategy=None",
     "-I" + os.path.join(ROOT, "include"),
 ]
+
+# The particle kernels without the atomic optimizer: it turns one lane's LDS
+# counter add into a wave-wide reduction that waits for its result at once,
+# while they need it only after the charge deposit.  Their counters that many
+# lanes add to are combined in the source (count_lanes, wave_counter_add).
+SOURCE_FLAGS = {src: ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]
+                for src in ("ohpic_particles.hip", "ohpic_particles_mixed.hip")}
 
 
 def _compile(src: str) -> str:
     out = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
     lang = ["-x", "hip"]
-    cmd = [HIPCC, *FLAGS, *lang, "-c", os.path.join(CSRC, src), "-o", out]
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *lang, "-c", os.path.join(CSRC, src), "-o", out]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr[-6000:]}")

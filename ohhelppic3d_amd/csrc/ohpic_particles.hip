@@ -133,7 +133,7 @@ __device__ __forceinline__ void route_back(const SpecDev &S, int nbuf, int t, co
     if (b + f < cap)
         store_p64(S, nbuf, base + (cap - 1 - b), q, ids);
     else
-        gatomic_add(&flags[kFlagOverflow], 1ull);
+        count_lanes(&flags[kFlagOverflow]);
 }
 
 template <bool IDS, int CAP>
@@ -395,7 +395,7 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                         q.z = apply_periodic(apply_periodic(q.z, nz), nz);
                         if (!(q.x >= 0.0 && q.x < nx && q.y >= 0.0 && q.y < ny && q.z >= 0.0 &&
                               q.z < nz)) {
-                            gatomic_add(&I->flags[kFlagRange], 1ull);
+                            count_lanes(&I->flags[kFlagRange]);
                             q.x = fmin(fmax(q.x - floor(q.x / nx) * nx, 0.0), nx - 1e-9);
                             q.y = fmin(fmax(q.y - floor(q.y / ny) * ny, 0.0), ny - 1e-9);
                             q.z = fmin(fmax(q.z - floor(q.z / nz) * nz, 0.0), nz - 1e-9);
@@ -461,7 +461,7 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                                 }
                     } else {
                         unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
-                        gatomic_add(&I->flags[kFlagFast], 1ull);
+                        count_lanes(&I->flags[kFlagFast]);
 #pragma unroll
                         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -570,7 +570,7 @@ __global__ void k_bin_count(const InstDev *__restrict__ insts, int inst, int s, 
         }
     }
     const bool inb = live && in_box(I, x, y, z);
-    if (live && !inb) gatomic_add(&I->flags[kFlagRange], 1ull);
+    if (live && !inb) count_lanes(&I->flags[kFlagRange]);
     const int t =
         inb ? ((int)x) / tx_ + I->nt[0] * (((int)y) / ty_ + I->nt[1] * (((int)z) / tz_)) : 0;
     (void)wave_counter_add(S.count[lbuf ^ 1], t, inb);
@@ -604,7 +604,7 @@ __global__ void k_bin_scatter(const InstDev *__restrict__ insts, int inst, int s
     if (slot < gload(S.bin_cap, t))
         store_p64(S, lbuf ^ 1, gload(S.bin_base, t) + slot, q, ids);
     else
-        gatomic_add(&I->flags[kFlagOverflow], 1ull);
+        count_lanes(&I->flags[kFlagOverflow]);
 }
 
 // Compact both runs of bins tiles[i] (tiles null: t0 + i) of buffer src into

@@ -190,7 +190,7 @@ __device__ __forceinline__ void route_back_mx(const SpecDev &S, int nbuf, int t,
     if (b + f < cap)
         store_pmx(S, nbuf, base + (cap - 1 - b), q, ids);
     else
-        gatomic_add(&flags[kFlagOverflow], 1ull);
+        count_lanes(&flags[kFlagOverflow]);
 }
 
 template <bool IDS, int CAP>
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                     const bool ok =
                         fabsf(sx) < kMaxShift && fabsf(sy) < kMaxShift && fabsf(sz) < kMaxShift;
                     if (!ok) {
-                        gatomic_add(&I->flags[kFlagRange], 1ull);
+                        count_lanes(&I->flags[kFlagRange]);
                     } else {
                         q.w[0] = (uint32_t)((int32_t)q.w[0] + (int32_t)rintf(sx));
                         q.w[1] = (uint32_t)((int32_t)q.w[1] + (int32_t)rintf(sy));
@@ -585,7 +585,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                             }
                     } else {
                         unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
-                        gatomic_add(&I->flags[kFlagFast], 1ull);
+                        count_lanes(&I->flags[kFlagFast]);
                         const int gx = wrap_cell(lox + rx, nx), gy = wrap_cell(loy + ry, ny),
                                   gz = wrap_cell(loz + rz, nz);
 #pragma unroll
@@ -705,7 +705,7 @@ __global__ void k_bin_count_mx(const InstDev *__restrict__ insts, int inst, int 
         t = gload((const int32_t *)S.buf[lbuf][0], i);
     }
     const bool ok = live && list_valid(I, t, q, tx_, ty_, tz_);
-    if (live && !ok) gatomic_add(&I->flags[kFlagRange], 1ull);
+    if (live && !ok) count_lanes(&I->flags[kFlagRange]);
     (void)wave_counter_add(S.count[lbuf ^ 1], ok ? t : 0, ok);
 }
 
@@ -730,7 +730,7 @@ __global__ void k_bin_scatter_mx(const InstDev *__restrict__ insts, int inst, in
     if (slot < gload(S.bin_cap, t))
         store_pmx(S, lbuf ^ 1, gload(S.bin_base, t) + slot, q, ids);
     else
-        gatomic_add(&I->flags[kFlagOverflow], 1ull);
+        count_lanes(&I->flags[kFlagOverflow]);
 }
 
 __global__ void k_bins_to_list_mx(const InstDev *__restrict__ insts, int inst, int s, int src,
@@ -854,7 +854,7 @@ __global__ void k_load_hump_mx(const InstDev *__restrict__ insts, int inst, int 
             break;
         }
     }
-    if (!ok) atomicAdd(fail, 1ull);
+    if (!ok) count_lanes(fail);
     double vx, vy, vz;
     maxwell3(r, vth, vx, vy, vz);
     store_loaded_mx(I, S, b, i, x, y, z, vx, vy, vz, i, I->track_ids != 0, tx_, ty_, tz_);
