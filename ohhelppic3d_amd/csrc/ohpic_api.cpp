@@ -119,8 +119,6 @@ struct ohpic_ctx {
     WorkItem *d_items = nullptr;
     int nitems = 0;
     int nitems_alloc = 0;
-    CloseItem *d_close = nullptr;  // split tiles (capacity ntiles)
-    int nclose = 0;
     int slots = 1;               // workgroups of the fused particle kernel resident at once
     int64_t *d_tmp64 = nullptr;  // [ntiles] scratch for repack / store
     int32_t *d_tmp32a = nullptr; // [ntiles]
@@ -261,8 +259,8 @@ struct TileLoad {
 };
 
 // No chunk is made smaller than this many slots: it costs an E tile, a charge
-// flush and a part in the closing launch (tiles of 9.4K slots in 2 chunks: 32^3
-// x 64 ppc mixed 124 us per launch, whole 88 us).
+// flush (tiles of 9.4K slots in 2 chunks: 32^3 x 64 ppc mixed 124 us per launch,
+// whole 88 us).
 constexpr int64_t kMinChunkLoad = 8192;
 
 // Chunks per tile (nch[i] of tiles[i]) and the order the tiles are dispatched
@@ -323,7 +321,6 @@ int64_t estimate_bytes(const ohpic_config &c, int num_cus)
     b += (int64_t)(c.nx + c.ny + c.nz) * (16 + 8);  // twiddles, Green's-function tables
     b += max_work_items(c, nt, num_cus) *
          ((int64_t)sizeof(WorkItem) + kKeSlots * 8 + kMaxSpecies * (int64_t)sizeof(int32_t));
-    b += nt * (int64_t)sizeof(CloseItem);
     return b;
 }
 
@@ -390,16 +387,14 @@ void tile_loads(const ohpic_ctx *ctx, int inst, std::vector<TileLoad> &out)
     }
 }
 
-// The work items of the planned tiles in dispatch order, and the list of split
-// tiles.  Slots count per instance (next_slot), chunks of a tile in a row.
+// The work items of the planned tiles in dispatch order.  Slots count per
+// instance (next_slot), chunks of a tile in a row.
 void emit_items(const std::vector<TileLoad> &tiles, const std::vector<int> &nch,
-                std::vector<int> &next_slot, std::vector<WorkItem> &items,
-                std::vector<CloseItem> &close)
+                std::vector<int> &next_slot, std::vector<WorkItem> &items)
 {
     for (size_t i = 0; i < tiles.size(); ++i) {
         const TileLoad &t = tiles[i];
         int &slot = next_slot[t.inst];
-        if (nch[i] > 1) close.push_back(CloseItem{t.inst, t.tile, nch[i], slot});
         for (int c = 0; c < nch[i]; ++c)
             items.push_back(WorkItem{t.inst, t.tile, (int16_t)c, (int16_t)nch[i], slot++});
     }
@@ -413,11 +408,10 @@ int build_work_items(ohpic_ctx *ctx)
     plan_chunks(tiles, ctx->slots, ctx->cfg.chunks > 0 ? 0 : (int64_t)ctx->num_cus * 8, nch);
     if (ctx->cfg.chunks > 0) nch.assign(tiles.size(), ctx->cfg.chunks);
     std::vector<WorkItem> items;
-    std::vector<CloseItem> close;
-    emit_items(tiles, nch, next_slot, items, close);
+    emit_items(tiles, nch, next_slot, items);
     if ((int)items.size() > ctx->nitems_alloc) {
         for (void *old : {(void *)ctx->d_items, (void *)ctx->h.ke_partial,
-                          (void *)ctx->h.chunk_front}) {
+                          (void *)ctx->h.claims}) {
             if (!old) continue;
             HIPCHK(ctx, hipStreamSynchronize(ctx->st));
             (void)hipFree(old);
@@ -428,13 +422,13 @@ int build_work_items(ohpic_ctx *ctx)
         }
         ctx->d_items = nullptr;
         ctx->h.ke_partial = nullptr;
-        ctx->h.chunk_front = nullptr;
+        ctx->h.claims = nullptr;
         ctx->nitems_alloc = 0;
         int rc = dalloc(ctx, &ctx->d_items, (int64_t)items.size());
         if (rc) return rc;
         rc = dalloc(ctx, &ctx->h.ke_partial, (int64_t)items.size() * kKeSlots);
         if (rc) return rc;
-        rc = dalloc(ctx, &ctx->h.chunk_front, (int64_t)items.size() * kMaxSpecies);
+        rc = dalloc(ctx, &ctx->h.claims, (int64_t)items.size() * kMaxSpecies);
         if (rc) return rc;
         HIPCHK(ctx, launch_fill_f64(ctx->h.ke_partial, (int64_t)items.size() * kKeSlots, 0.0,
                                     ctx->st));
@@ -442,12 +436,9 @@ int build_work_items(ohpic_ctx *ctx)
     }
     ctx->nitems = (int)items.size();
     ctx->h.nitems = ctx->nitems;
-    ctx->nclose = (int)close.size();
+    ctx->h.split = items.size() > tiles.size();
     HIPCHK(ctx, hipMemcpyAsync(ctx->d_items, items.data(), items.size() * sizeof(WorkItem),
                                hipMemcpyHostToDevice, ctx->st));
-    if (!close.empty())
-        HIPCHK(ctx, hipMemcpyAsync(ctx->d_close, close.data(), close.size() * sizeof(CloseItem),
-                                   hipMemcpyHostToDevice, ctx->st));
     ctx->items = std::move(items);
     ctx->items_ver += 1;
     return sync_upload_inst(ctx);
@@ -456,13 +447,9 @@ int build_work_items(ohpic_ctx *ctx)
 // The particle kernel over this context's work items.
 hipError_t run_particles(ohpic_ctx *ctx, int mode)
 {
-    hipError_t e = launch_particles(mode, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
-                                    ctx->cfg.track_ids != 0, ctx->d_inst, ctx->d_items,
-                                    ctx->nitems, parity_of(ctx), ctx->st);
-    if (e == hipSuccess && (mode == kModeFused || mode == kModeBoundary))
-        e = launch_close_chunks(ctx->cfg.precision, ctx->d_inst, ctx->d_close, ctx->nclose,
-                                ctx->cfg.nspecies, parity_of(ctx), ctx->st);
-    return e;
+    return launch_particles(mode, ctx->cfg.precision, ctx->cfg.weight_order, ctx->T,
+                            ctx->cfg.track_ids != 0, ctx->d_inst, ctx->d_items, ctx->nitems,
+                            parity_of(ctx), ctx->st);
 }
 
 // Assign capacities/bases from per-bin counts and upload them.
@@ -1032,9 +1019,6 @@ struct ohpic_group {
     WorkItem *d_items = nullptr;
     int64_t cap_items = 0;
     int nitems = 0;
-    CloseItem *d_close = nullptr;      // split tiles
-    int64_t cap_close = 0;
-    int nclose = 0, max_ns = 0;
     bool ids = false;                  // some member keeps particle ids
     bool dirty = true;
     int64_t max_ng = 0;
@@ -1098,7 +1082,7 @@ void gfree(T *&p)
     p = nullptr;
 }
 
-int group_reserve(ohpic_group *g, int ninst, int64_t nitems, int64_t nclose)
+int group_reserve(ohpic_group *g, int ninst, int64_t nitems)
 {
     if (ninst > g->cap_insts) {
         const int cap = std::max(ninst, std::max(16, 2 * g->cap_insts));
@@ -1128,15 +1112,6 @@ int group_reserve(ohpic_group *g, int ninst, int64_t nitems, int64_t nclose)
         GHIP(g, hipMalloc((void **)&g->d_items, cap * sizeof(WorkItem)));
         g->cap_items = cap;
     }
-    if (nclose > g->cap_close) {
-        const int64_t cap = std::max<int64_t>(nclose, std::max<int64_t>(1024, 2 * g->cap_close));
-        GHIP(g, hipStreamSynchronize(g->st));
-        drop_graph(g);
-        gfree(g->d_close);
-        g->cap_close = 0;
-        GHIP(g, hipMalloc((void **)&g->d_close, cap * sizeof(CloseItem)));
-        g->cap_close = cap;
-    }
     return OHPIC_OK;
 }
 
@@ -1145,8 +1120,7 @@ int group_reserve(ohpic_group *g, int ninst, int64_t nitems, int64_t nclose)
 // share of the device is not split as if it ran alone.  A member with a given
 // chunk count, or whose planned items would not fit the rows it holds, keeps
 // its own split.  rows[i]: items of member i.
-void group_items(ohpic_group *g, std::vector<WorkItem> &items, std::vector<CloseItem> &close,
-                 std::vector<int> &rows)
+void group_items(ohpic_group *g, std::vector<WorkItem> &items, std::vector<int> &rows)
 {
     const int n = (int)g->members.size();
     std::vector<TileLoad> tiles;
@@ -1165,7 +1139,7 @@ void group_items(ohpic_group *g, std::vector<WorkItem> &items, std::vector<Close
     for (size_t k = 0; k < tiles.size(); ++k)
         if (!own[tiles[k].inst].empty()) nch[k] = own[tiles[k].inst][tiles[k].tile];
     std::vector<int> next(n, 0);
-    emit_items(tiles, nch, next, items, close);
+    emit_items(tiles, nch, next, items);
     rows = next;
 }
 
@@ -1180,22 +1154,17 @@ int group_refresh(ohpic_group *g)
                  g->members[i]->items_ver != g->seen_items[i];
     if (tables) {
         g->ids = false;
-        g->max_ns = 0;
-        for (ohpic_ctx *m : g->members) {
-            g->ids = g->ids || m->cfg.track_ids != 0;
-            g->max_ns = std::max(g->max_ns, m->cfg.nspecies);
-        }
+        for (ohpic_ctx *m : g->members) g->ids = g->ids || m->cfg.track_ids != 0;
         if (n > 0)
             g->queue_blocks =
                 particles_queue_blocks(g->precision, g->weight_order, g->T, g->ids, g->device);
         std::vector<InstDev> insts(n);
         std::vector<FftJob> jobs(n);
         std::vector<WorkItem> items;
-        std::vector<CloseItem> close;
         std::vector<int> rows;
-        group_items(g, items, close, rows);
+        group_items(g, items, rows);
         if (items.size() > (size_t)INT32_MAX) return gfail(g, OHPIC_EINVAL, "more than 2^31 work items");
-        int rc = group_reserve(g, n, (int64_t)items.size(), (int64_t)close.size());
+        int rc = group_reserve(g, n, (int64_t)items.size());
         if (rc) return rc;
         g->max_ng = 0;
         g->max_ntiles = g->max_rows = 0;
@@ -1204,6 +1173,7 @@ int group_refresh(ohpic_group *g)
             ohpic_ctx *m = g->members[i];
             insts[i] = m->h;
             insts[i].nitems = rows[i];
+            insts[i].split = rows[i] > m->ntiles;
             jobs[i] = m->job;
             g->max_ng = std::max(g->max_ng, m->ng);
             g->max_ntiles = std::max(g->max_ntiles, m->ntiles);
@@ -1213,7 +1183,6 @@ int group_refresh(ohpic_group *g)
             g->seen_items[i] = m->items_ver;
         }
         g->nitems = (int)items.size();
-        g->nclose = (int)close.size();
         if (n > 0) {
             GHIP(g, hipMemcpyAsync(g->d_insts, insts.data(), n * sizeof(InstDev),
                                    hipMemcpyHostToDevice, g->st));
@@ -1222,9 +1191,6 @@ int group_refresh(ohpic_group *g)
         }
         if (!items.empty())
             GHIP(g, hipMemcpyAsync(g->d_items, items.data(), items.size() * sizeof(WorkItem),
-                                   hipMemcpyHostToDevice, g->st));
-        if (!close.empty())
-            GHIP(g, hipMemcpyAsync(g->d_close, close.data(), close.size() * sizeof(CloseItem),
                                    hipMemcpyHostToDevice, g->st));
         GHIP(g, hipStreamSynchronize(g->st));
         drop_graph(g);
@@ -1268,9 +1234,6 @@ hipError_t group_enqueue(ohpic_group *g, int k)
                 e = launch_particles(kModeFused, g->precision, g->weight_order, g->T, g->ids,
                                      g->d_insts, g->d_items, g->nitems, g->d_parity, g->st);
         }
-        if (e == hipSuccess)
-            e = launch_close_chunks(g->precision, g->d_insts, g->d_close, g->nclose, g->max_ns,
-                                    g->d_parity, g->st);
         if (e == hipSuccess)
             e = launch_end_step_b(g->d_insts, g->d_parity, n, true,
                                   g->d_flags + (size_t)s * n * kFlagSlots, g->st);
@@ -1390,10 +1353,8 @@ int group_step(ohpic_group *g, int nsteps)
                         ++r;
                     }
                 }
-                // an overflow followed by a step that went through (bin
-                // arrivals race with the front reservation near a full bin)
-                // leaves E one step behind: the rest run alone, each with its
-                // own field solve
+                // an overflow before the last step leaves E one step behind:
+                // the rest run alone, each with its own field solve
                 for (; r < k && rc == OHPIC_OK; ++r) rc = one_step(m);
                 // every step of the sequence went through and one left a bin
                 // tight: move the bins the last step listed (a member that
@@ -1686,7 +1647,6 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
     CREATE_HIP(hipHostGetDevicePointer((void **)&ctx->dh_flags, ctx->h_flags, 0));
     CREATE_HIP(hipHostMalloc((void **)&ctx->h_diag, kDiagSlots * sizeof(double),
                              hipHostMallocDefault));
-    CREATE_CHK(dalloc(ctx, &ctx->d_close, nt));
     ctx->slots = particles_queue_blocks(c.precision, c.weight_order, ctx->T, c.track_ids != 0,
                                         ctx->device);
     CREATE_CHK(sync_upload_inst(ctx));
@@ -2047,7 +2007,7 @@ int ohpic_boundary(ohpic_ctx *ctx)
     GateShared gate;
     if (!ctx) return fail(nullptr, OHPIC_EINVAL, "ctx is NULL");
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    HIPCHK(ctx, launch_reserve_next_b(ctx->d_inst, parity_of(ctx), 1, ctx->ntiles, ctx->st));
+    HIPCHK(ctx, launch_clear_next_b(ctx->d_inst, parity_of(ctx), 1, ctx->ntiles, ctx->st));
     HIPCHK(ctx, run_particles(ctx, kModeBoundary));
     int rc = read_flags(ctx);
     if (rc) return rc;
@@ -2498,7 +2458,6 @@ int ohpic_group_destroy(ohpic_group *g)
     gfree(g->d_parity);
     gfree(g->d_flags);
     gfree(g->d_items);
-    gfree(g->d_close);
     gfree(g->d_queue);
     if (g->h_flags) (void)hipHostFree(g->h_flags);
     (void)hipStreamDestroy(g->st);

@@ -1085,7 +1085,7 @@ __global__ void __launch_bounds__((kPlaneWaves + 1) * 64)
             // the wavefront beyond those of the lines
             if (step0.queue && blockIdx.x == 0 && blockIdx.y == 0 && lane == 0) *step0.queue = 0u;
             if (blockIdx.x == 0 && lane < kFlagWords) I->flags[lane] = 0ull;
-            reserve_next(I, par, (int64_t)blockIdx.x * 64 + lane, (int64_t)nz * 64);
+            clear_next(I, par, (int64_t)blockIdx.x * 64 + lane, (int64_t)nz * 64);
         }
         __syncthreads();
         if (wave < gy) y_lines(wave, staged);

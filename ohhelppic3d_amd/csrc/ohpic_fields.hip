@@ -264,17 +264,17 @@ __global__ void k_prepare_next_b(const InstDev *__restrict__ insts, const int *_
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
-__global__ void k_reserve_next_b(const InstDev *__restrict__ insts, const int *__restrict__ parity)
+__global__ void k_clear_next_b(const InstDev *__restrict__ insts, const int *__restrict__ parity)
 {
     const InstDev *I = insts + blockIdx.y;
     const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    reserve_next(I, parity[blockIdx.y], t0, (int64_t)gridDim.x * blockDim.x);
+    clear_next(I, parity[blockIdx.y], t0, (int64_t)gridDim.x * blockDim.x);
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
 // Start of a step: rho := the current charge grid * 2^-charge_bits, the next
-// charge grid, the flags and the queue counter zeroed and the next bin words
-// reserved, in the same sweep.
+// charge grid, the next bin words, the flags and the queue counter zeroed, in
+// the same sweep.
 __global__ void k_begin_step_b(const InstDev *__restrict__ insts, const int *__restrict__ parity,
                                unsigned int *__restrict__ queue)
 {
@@ -292,15 +292,16 @@ __global__ void k_begin_step_b(const InstDev *__restrict__ insts, const int *__r
         rho[i] = (double)(long long)acc[i] * scale;
         next[i] = 0ull;
     }
-    reserve_next(I, par, t0, stride);
+    clear_next(I, par, t0, stride);
     if (t0 < kFlagWords) I->flags[t0] = 0ull;
 }
 
 // End of a step: block x reduces energy sum x (k_energy_sums_b); unless a bin
 // overflowed, all blocks then scan a share of
-// the step's new bins (buffer parity ^ 1): listed bins go to tight_list (their
-// number to kFlagListed) and a tight one raises kFlagTight (the host then
-// moves them before the next step).  The last block to finish reports the
+// the step's new bins (buffer parity ^ 1): one whose runs meet raises
+// kFlagOverflow, listed bins go to tight_list (their number to kFlagListed) and
+// a tight one raises kFlagTight (the host then moves them before the next
+// step).  The last block to finish reports the
 // flags: out[i*kFlagSlots + k] := flags[k] of instance i.  Of a group (flip)
 // it completes the instance's step too: parity[i] flips unless a bin
 // overflowed (the host then redoes that step in list mode from the unchanged
@@ -326,6 +327,7 @@ __global__ void __launch_bounds__(kSumBlock) k_end_step_b(const InstDev *__restr
                 const unsigned long long c = S.count[nb][t];
                 const int cap = S.bin_cap[t], used = bin_front(c) + bin_back(c);
                 if (!bin_listed(cap, used, I->tight_frac)) continue;
+                if (used > cap) atomicAdd(&flags[kFlagOverflow], 1ull);
                 const unsigned long long k = atomicAdd(&flags[kFlagListed], 1ull);
                 if (k < (unsigned long long)kTightListCap) I->tight_list[k] = tight_entry(s, t, used);
                 if (bin_tight(cap, used, I->tight_frac)) atomicOr(&flags[kFlagTight], 1ull);
@@ -514,11 +516,11 @@ hipError_t launch_prepare_next_b(const InstDev *insts, const int *parity, int ni
     return hipGetLastError();
 }
 
-hipError_t launch_reserve_next_b(const InstDev *insts, const int *parity, int ninst,
+hipError_t launch_clear_next_b(const InstDev *insts, const int *parity, int ninst,
                                  int max_ntiles, hipStream_t st)
 {
     if (ninst <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reserve_next_b, dim3(grid_blocks(max_ntiles, ninst), ninst), dim3(256), 0,
+    hipLaunchKernelGGL(k_clear_next_b, dim3(grid_blocks(max_ntiles, ninst), ninst), dim3(256), 0,
                        st, insts, parity);
     return hipGetLastError();
 }

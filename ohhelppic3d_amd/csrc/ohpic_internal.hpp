@@ -97,7 +97,9 @@ struct InstDev {
     double *ke_partial;           // [kKeSlots][nitems], each row reduced by one block
     double *e_partial;            // [kEfieldMaxBlocks][3] field-energy partial sums
     int nitems;                   // work items of this instance (row length of ke_partial)
-    int32_t *chunk_front;         // [nitems][kMaxSpecies] front-run counts of split tiles' chunks
+    int32_t *claims;              // [nitems][kMaxSpecies] slots of the new front run that a split
+                                  // tile's items have taken, at its first item
+    int split;                    // some tile is split
     unsigned long long *flags;    // kFlagSlots
 };
 
@@ -107,11 +109,6 @@ struct WorkItem {
     int16_t chunk;     // this item's slice of every bin of the tile
     int16_t nchunks;   // slices per bin
     int32_t slot;      // row of the per-item partial-sum table
-};
-// A tile split into several work items (slots slot0 ... slot0 + nchunks - 1):
-// k_close_chunks joins their parts of the new front run.
-struct CloseItem {
-    int32_t inst, tile, nchunks, slot0;
 };
 // largest chunks per tile a configuration may ask for (WorkItem::nchunks)
 constexpr int kMaxChunks = 32767;
@@ -230,20 +227,15 @@ __device__ __forceinline__ int wrap_index(int i, int n)
     return i;
 }
 
-// Reserves each bin's whole current count as the front run of the next buffer:
-// the stayers always fit, and arrivals from neighbours are placed behind them
-// from the start.  (Done here, a tile's workgroup starts without waiting for a
-// reservation of its own, and a tile may be split among several workgroups.)
-__device__ __forceinline__ void reserve_next(const InstDev *I, int par, int64_t t0, int64_t stride)
+// Empties the next buffer's bin words and the claims of split tiles.
+__device__ __forceinline__ void clear_next(const InstDev *I, int par, int64_t t0, int64_t stride)
 {
     for (int s = 0; s < I->nspecies; ++s) {
-        const SpecDev &S = I->sp[s];
-        for (int64_t t = t0; t < I->ntiles; t += stride) {
-            const unsigned long long c = S.count[par][t];
-            const int cap = S.bin_cap[t], F = min(bin_front(c), cap);
-            S.count[par ^ 1][t] = (unsigned long long)(F + min(bin_back(c), cap - F));
-        }
+        unsigned long long *__restrict__ w = I->sp[s].count[par ^ 1];
+        for (int64_t t = t0; t < I->ntiles; t += stride) w[t] = 0ull;
     }
+    if (I->split)
+        for (int64_t t = t0; t < (int64_t)I->nitems * kMaxSpecies; t += stride) I->claims[t] = 0;
 }
 
 }  // namespace ohpic

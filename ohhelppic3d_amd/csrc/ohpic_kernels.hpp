@@ -35,11 +35,6 @@ bool tile_supported(int tx, int ty, int tz);
 hipError_t launch_particles(int mode, int precision, int weight_order, const int T[3], bool ids,
                             const InstDev *insts, const WorkItem *items, int nitems,
                             const int *parity, hipStream_t st);
-// After a fused or boundary launch with split tiles: joins the chunks' parts
-// of each listed tile's new front runs (ns: species of the instance that has
-// most).
-hipError_t launch_close_chunks(int precision, const InstDev *insts, const CloseItem *list, int n,
-                               int ns, const int *parity, hipStream_t st);
 // Bin a contiguous list [0, n) of buffer lbuf into the front runs of buffer
 // lbuf^1 (count first, then scatter once capacities are set); wrap != 0
 // applies the periodic wrap twice to each position first.
@@ -103,9 +98,8 @@ hipError_t launch_rho_from_acc_b(const InstDev *insts, const int *parity, int ni
 // max_blocks: the largest efield_blocks_of() over the instances
 hipError_t launch_efield_b(const InstDev *insts, int ninst, int max_blocks, bool reduce,
                            hipStream_t st);
-// rho from the current charge grid, the next charge grid, flags and queue
-// counter zeroed, and the next bin words reserved (launch_reserve_next_b), in
-// one launch at the start of a step
+// rho from the current charge grid, and the next charge grid and bin words, the
+// flags and the queue counter zeroed, in one launch at the start of a step
 hipError_t launch_begin_step_b(const InstDev *insts, const int *parity, int ninst,
                                int64_t max_ng, int max_ntiles, unsigned int *queue,
                                hipStream_t st);
@@ -118,9 +112,8 @@ hipError_t launch_end_step_b(const InstDev *insts, int *parity, int ninst, bool 
 // zero the next buffer's bin words and charge grid and the flags (list mode)
 hipError_t launch_prepare_next_b(const InstDev *insts, const int *parity, int ninst,
                                  int64_t max_ng, int max_ntiles, hipStream_t st);
-// next bin words := each bin's whole current count as front run (what the
-// particle kernels' stayers fill; arrivals go behind it), flags := 0
-hipError_t launch_reserve_next_b(const InstDev *insts, const int *parity, int ninst,
+// next bin words and flags := 0
+hipError_t launch_clear_next_b(const InstDev *insts, const int *parity, int ninst,
                                  int max_ntiles, hipStream_t st);
 // diag[kDiagKeOld..] := sums of ke_partial over the instance's items
 hipError_t launch_reduce_ke_b(const InstDev *insts, int ninst, hipStream_t st);

@@ -27,7 +27,8 @@ constexpr int kStash = 64;     // per-wave stash of particles that stayed (below
 // left takes one from the wavefront's stash instead; a wavefront whose stash
 // is too small for its holes puts its stayers there and stores nothing, which
 // happens once per kStash leavers or so.  The stashes that are left at the end
-// follow the last block as one run, so the front run has no gap.
+// follow the last block as one run, or, of a tile split among several work
+// items, go to the back run, so the front run has no gap.
 
 // Rank of this lane among the set lanes below it.
 __device__ __forceinline__ int lane_rank(unsigned long long m)
@@ -234,18 +235,38 @@ __device__ __forceinline__ void load_meta(SpecMeta *meta, const InstDev *__restr
     meta[tid] = m;
 }
 
-// The m particles of a chunk's front run are written.  The step started with
-// the whole count reserved (k_begin_step_b, k_fft_planes or k_reserve_next_b): a tile of one
-// chunk releases what its leavers left unused; a chunk of several leaves its
-// count for k_close_chunks.
-__device__ __forceinline__ void publish_front(const InstDev *__restrict__ I, const SpecDev &S,
-                                              const WorkItem &it, int s, int nbuf, int tile,
-                                              int cnt, int m, bool excl)
+// The front run of a split tile's bin is shared by its items: a wavefront takes
+// each of its blocks from a counter of the tile's own, and adds them to the
+// bin's word when the species is done.  (Taken from the word itself, which all
+// arrivals add to, with the words of 15 other tiles in its cache line: 16^3 x
+// 1000 ppc, 12 items per tile, 1285 us per step FP64 and 1465 mixed, against
+// 1035 and 1147.  Items with parts of the front run of their own and a launch
+// to join them: 1077 and 1186.)  The answer is waited for here: pending in the
+// register that a whole tile's answer from LDS takes, it made every tile wait
+// for its loads ahead too (96^3 x 32 ppc FP64 1105 -> 1120 us per launch).
+__device__ __forceinline__ int claim_block(const InstDev *__restrict__ I, const WorkItem &it, int s)
 {
-    if (!excl)
-        gstore(I->chunk_front, (int64_t)it.slot * kMaxSpecies + s, m);
-    else if (m < cnt)
-        gatomic_add(&S.count[nbuf][tile], (unsigned long long)(-(long long)(cnt - m)));
+    int32_t *p = &I->claims[(int64_t)(it.slot - it.chunk) * kMaxSpecies + s];
+    return uniform(
+        __hip_atomic_fetch_add(as_global(p), 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// Adds the m stayers of a tile that is one item.  Arrivals look at the word as
+// they add to it (route_back); the runs of a bin that is too full also meet
+// where its stayers come last, which the end of the step (k_end_step_b), or
+// here the CHECKing item itself, sees: a step is redone only if stayers and
+// arrivals together exceed a bin.  (With the whole old count reserved at the
+// start of the step, 32^3 x 16 ppc at a thermal speed of 0.3 cells per step
+// overflowed every step: 540 us against 121, FP64.)
+template <bool CHECK>
+__device__ __forceinline__ bool add_front(unsigned long long *word, int m, int cap)
+{
+    if (CHECK) {
+        const unsigned long long old = gatomic_add(word, (unsigned long long)m);
+        return (int64_t)bin_front(old) + m + bin_back(old) > cap;
+    }
+    if (m > 0) gatomic_add(word, (unsigned long long)m);
+    return false;
 }
 
 // The item's kinetic-energy partials, summed over its W wavefronts in order.

@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
     __shared__ Buf64<IDS, kStash> sStash[BINS ? kWaves : 1];
     __shared__ double sKe[PUSH ? kKeSlots : 1][kWaves];
     __shared__ SpecMeta sMeta[kMaxSpecies];
-    __shared__ int sBlk[BINS ? kMaxSpecies : 1];          // full blocks written
+    __shared__ int sBlk[BINS ? kMaxSpecies : 1];           // slots of the blocks written
     __shared__ int sLeft[BINS ? kMaxSpecies : 1][kWaves];  // stayers left in each stash
     __shared__ int sItem;
 
@@ -320,11 +320,11 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
             const double s0 = uniform(2 * t0 / (1 + tt)), s1 = uniform(2 * t1 / (1 + tt)),
                          s2 = uniform(2 * t2 / (1 + tt));
             double keo = 0.0, ken = 0.0;
+            int taken = 0;       // slots of this wavefront's blocks
             int lc = 0, sc = 0;  // particles in this wavefront's leaver buffer and stash
 
             const BinView64 cur = bin_view64(S, par, base, ids);
-            // this chunk's part of the new front run starts at its slot `start`
-            const BinView64 nxt = bin_view64(S, nbuf, base + start, ids);
+            const BinView64 nxt = bin_view64(S, nbuf, base, ids);
             P64 nextq{0, 0, 0, 0, 0, 0, 0};
             if (start + tid < end)
                 nextq = load_bin64(cur, (uint32_t)bin_slot(start + tid, F, B, cap), ids);
@@ -404,7 +404,7 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                     }
                 }
                 bool block = false;  // this wavefront stores a full block
-                int blk;             // its number (lane 0)
+                int blk;             // its first slot (lane 0)
                 int nst = 0;
                 unsigned long long sm = 0ull;
                 if (BINS) {
@@ -430,8 +430,10 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                     block = holes <= sc;
                     if (block) {
                         // (arrives while the charge is deposited)
-                        if (lane == 0) blk = atomicAdd(&sBlk[s], 1);
+                        if (lane == 0)
+                            blk = excl ? atomicAdd(&sBlk[s], 64) : claim_block(I, it, s);
                         sc -= holes;
+                        taken += 64;
                     }
                 }
                 if (DEP && active) {
@@ -487,7 +489,7 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                 } else if (block) {
                     wave_sync();
                     if (!stay) sStash[wv].get(sc + lane_rank(~sm), q, ids);
-                    store_bin64<true>(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                    store_bin64<true>(nxt, (uint32_t)(lane_bcast(blk, 0) + lane), q, ids);
                 } else if (nst > 0) {
                     wave_sync();
                     if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
@@ -495,24 +497,39 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
                 }
             }
             if (BINS) {
+                // the stayers left in the stashes: behind the blocks, or in the
+                // back run of a split tile
+                unsigned long long word = 0ull;
+                if (!excl && taken + sc > 0 && lane == 0)
+                    word = gatomic_add(&S.count[nbuf][tile],
+                                       (unsigned long long)taken | (unsigned long long)sc << 32);
                 flush_leavers<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids);
-                if (lane == 0) sLeft[s][wv] = sc;
-                __syncthreads();
-                // the stayers left in the stashes follow the blocks
-                int o = 64 * sBlk[s], m = o;
+                if (excl) {
+                    if (lane == 0) sLeft[s][wv] = sc;
+                    __syncthreads();
+                    int o = sBlk[s];
 #pragma unroll
-                for (int w = 0; w < kWaves; ++w) {
-                    const int r = sLeft[s][w];
-                    if (w < wv) o += r;
-                    m += r;
-                }
-                if (lane < sc) {
-                    P64 q;
-                    sStash[wv].get(lane, q, ids);
-                    store_bin64<false>(nxt, (uint32_t)(o + lane), q, ids);
+                    for (int w = 0; w + 1 < kWaves; ++w) {
+                        const int r = sLeft[s][w];
+                        if (w < wv) o += r;
+                    }
+                    if (lane < sc) {
+                        P64 q;
+                        sStash[wv].get(lane, q, ids);
+                        store_bin64<false>(nxt, (uint32_t)(o + lane), q, ids);
+                    }
+                } else if (taken + sc > 0) {
+                    const unsigned long long old = lane_bcast(word, 0);
+                    const int front = bin_front(old) + taken, back = bin_back(old);
+                    if (front + back + sc > cap) {
+                        if (lane == 0) gatomic_add(&I->flags[kFlagOverflow], 1ull);
+                    } else if (lane < sc) {
+                        P64 q;
+                        sStash[wv].get(lane, q, ids);
+                        store_bin64<false>(nxt, (uint32_t)(cap - 1 - back - lane), q, ids);
+                    }
                 }
                 wave_sync();
-                if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
             }
             if (PUSH) {
                 keo = wave_total(keo);
@@ -525,6 +542,13 @@ __global__ void __launch_bounds__(fp_block(TX *TY *TZ))
         }
 
         __syncthreads();
+        if (BINS && excl && tid < ns) {
+            int m = sBlk[tid];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) m += sLeft[tid][w];
+            if (add_front<MODE == kModeBoundary>(&I->sp[tid].count[nbuf][tile], m, sMeta[tid].cap))
+                count_lanes(&I->flags[kFlagOverflow]);
+        }
         if (PUSH) write_ke<kWaves>(I, it, tid, ns, sKe);
         if (DEP) {
             unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
@@ -801,83 +825,6 @@ int particles_queue_blocks(int precision, int weight_order, const int T[3], bool
 #undef OHPIC_TILE
     }
     return per * cus;
-}
-
-// Joins the chunks' parts of a split tile's new front runs (blockIdx.x = list
-// entry, blockIdx.y = species).  Chunk c wrote chunk_front[slot0 + c] particles
-// from slot c * per on; the tile's front run is their sum M, so the gaps below
-// M (as many as the tile's leavers, a few per cent) take the particles at and
-// above M.  A step that overflowed a bin is redone from the other buffer.
-template <typename T, int C0>
-__global__ void __launch_bounds__(256) k_close_chunks(const InstDev *__restrict__ insts,
-                                                      const CloseItem *__restrict__ list,
-                                                      const int *__restrict__ parity)
-{
-    constexpr int kCached = 64;
-    __shared__ int sFront[kCached];
-    __shared__ int sSum;
-    const CloseItem c = list[blockIdx.x];
-    const InstDev *I = insts + c.inst;
-    const int s = blockIdx.y;
-    if (s >= I->nspecies || I->flags[kFlagOverflow] != 0ull) return;
-    const SpecDev &S = I->sp[s];
-    const int par = parity[c.inst], nbuf = par ^ 1;
-    const unsigned long long word = S.count[par][c.tile];
-    const int cap = S.bin_cap[c.tile], F = min(bin_front(word), cap);
-    const int cnt = F + min(bin_back(word), cap - F);
-    const int per = chunk_size(cnt, c.nchunks);
-    const int32_t *fr = I->chunk_front + (int64_t)c.slot0 * kMaxSpecies + s;
-    if (threadIdx.x == 0) sSum = 0;
-    __syncthreads();
-    int sum = 0;
-    for (int k = threadIdx.x; k < c.nchunks; k += blockDim.x) {
-        const int m = fr[(int64_t)k * kMaxSpecies];
-        if (k < kCached) sFront[k] = m;
-        sum += m;
-    }
-    if (sum) atomicAdd(&sSum, sum);
-    __syncthreads();
-    const int M = sSum;
-    auto front = [&](int k) { return k < kCached ? sFront[k] : fr[(int64_t)k * kMaxSpecies]; };
-    const int64_t base = S.bin_base[c.tile];
-    for (int j = threadIdx.x; j < cnt - M; j += blockDim.x) {
-        int hole = -1, from = -1, hj = j, fj = j;
-        for (int k = 0; k < c.nchunks; ++k) {
-            const int lo = k * per, end = lo + front(k);
-            if (hole < 0) {
-                const int h = max(0, min(min(cnt, lo + per), M) - end);
-                if (hj < h) hole = end + hj;
-                hj -= h;
-            }
-            if (from < 0) {
-                const int v = max(0, end - max(lo, M));
-                if (fj < v) from = max(lo, M) + fj;
-                fj -= v;
-            }
-            if (lo + per >= cnt) break;
-        }
-        if (hole < 0 || from < 0) break;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            T *p = (T *)S.buf[nbuf][C0 + k];
-            gstore(p, base + hole, gload(p, base + from));
-        }
-        if (I->track_ids) gstore(S.pid[nbuf], base + hole, gload(S.pid[nbuf], base + from));
-    }
-    if (threadIdx.x == 0)
-        S.count[nbuf][c.tile] = (S.count[nbuf][c.tile] & ~0xffffffffull) | (unsigned long long)M;
-}
-
-hipError_t launch_close_chunks(int precision, const InstDev *insts, const CloseItem *list, int n,
-                               int ns, const int *parity, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    const dim3 g(n, ns);
-    if (precision == 1)
-        hipLaunchKernelGGL((k_close_chunks<uint32_t, 1>), g, dim3(256), 0, st, insts, list, parity);
-    else
-        hipLaunchKernelGGL((k_close_chunks<double, 0>), g, dim3(256), 0, st, insts, list, parity);
-    return hipGetLastError();
 }
 
 hipError_t launch_bin_count(const InstDev *insts, int inst, int s, int lbuf, int64_t n,

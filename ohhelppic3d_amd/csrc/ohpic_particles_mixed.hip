@@ -40,8 +40,10 @@ namespace {
 #ifndef OHPIC_MX_PREFETCH
 #define OHPIC_MX_PREFETCH 1
 #endif
-// Minimum waves per SIMD of the fused mixed kernel: 5 (96 VGPRs) measured
-// faster than the 4 the compiler picks on its own at 256^3 x 64 ppc.
+// Waves per SIMD the mixed kernel's registers are limited for: 5 (96 VGPRs)
+// measured faster than the 4 the compiler picks on its own at 256^3 x 64 ppc
+// with workgroups of 256 threads.  (Two workgroups of 512 are resident per CU,
+// 4 waves per SIMD.)
 #ifndef OHPIC_MX_MIN_WAVES
 #define OHPIC_MX_MIN_WAVES 5
 #endif
@@ -265,12 +267,18 @@ __device__ __forceinline__ void flush_leavers_mx(const BufMx<IDS, kLeaveCap> &lb
 // 256^3 x 32 10.91 -> 10.78 ms); a small tile has too little work for them
 // (8x8x4 tiles of a group of 32: 12.5 ms per 8 steps with 256, 15.6 with 512).
 constexpr int mx_block(int cells) { return cells >= 512 ? 512 : 256; }
+// With ids, the workgroups of 512 and the resident grid take the registers that
+// 4 waves per SIMD leave them: 5 would need scratch.
+constexpr int mx_min_waves(int cells, int mode, bool ids)
+{
+    return ids && (cells >= 512 || mode == kModeFusedQueue) ? 4 : OHPIC_MX_MIN_WAVES;
+}
 
 // IDS: instances may keep particle ids (each instance's track_ids says whether
 // it does); without it no register, LDS or branch is spent on them.
 template <int TX, int TY, int TZ, int WO, int MODE_, bool IDS>
 __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
-    __attribute__((amdgpu_waves_per_eu((MODE_ == kModeFusedQueue && IDS) ? 4 : OHPIC_MX_MIN_WAVES, 8)))
+    __attribute__((amdgpu_waves_per_eu(mx_min_waves(TX *TY *TZ, MODE_, IDS), 8)))
     k_particles_mixed(const InstDev *__restrict__ insts, const WorkItem *__restrict__ items,
                       const int *__restrict__ parity, unsigned int *__restrict__ queue,
                       int nitems)
@@ -299,7 +307,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
     __shared__ BufMx<IDS, kStash> sStash[BINS ? kWaves : 1];
     __shared__ double sKe[PUSH ? kKeSlots : 1][kWaves];
     __shared__ SpecMeta sMeta[kMaxSpecies];
-    __shared__ int sBlk[BINS ? kMaxSpecies : 1];          // full blocks written
+    __shared__ int sBlk[BINS ? kMaxSpecies : 1];           // slots of the blocks written
     __shared__ int sLeft[BINS ? kMaxSpecies : 1][kWaves];  // stayers left in each stash
     __shared__ int sItem;
 
@@ -398,13 +406,13 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
             const float s0 = uniform(2.0f * t0 / (1.0f + tt)), s1 = uniform(2.0f * t1 / (1.0f + tt)),
                         s2 = uniform(2.0f * t2 / (1.0f + tt));
             double keo = 0.0, ken = 0.0;
+            int taken = 0;       // slots of this wavefront's blocks
             int lc = 0, sc = 0;  // particles in this wavefront's leaver buffer and stash
 
             // the next kMxPrefetch particles of this lane are loaded ahead, so each
             // lane keeps that many particle reads in flight
             const BinView cur = bin_view(S, par, base, ids);
-            // this chunk's part of the new front run starts at its slot `start`
-            const BinView nxt = bin_view(S, nbuf, base + start, ids);
+            const BinView nxt = bin_view(S, nbuf, base, ids);
             PMx ahead[kMxPrefetch];
 #pragma unroll
             for (int k = 0; k < kMxPrefetch; ++k) {
@@ -507,7 +515,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                 if (MODE == kModeGatherPush) continue;
 
                 bool block = false;  // this wavefront stores a full block
-                int blk;             // its number (lane 0)
+                int blk;             // its first slot (lane 0)
                 bool stay = false;
                 int nst = 0;
                 unsigned long long sm = 0ull;
@@ -547,8 +555,10 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                     block = holes <= sc;
                     if (block) {
                         // both arrive while the charge is deposited
-                        if (lane == 0) blk = atomicAdd(&sBlk[s], 1);
+                        if (lane == 0)
+                            blk = excl ? atomicAdd(&sBlk[s], 64) : claim_block(I, it, s);
                         sc -= holes;
+                        taken += 64;
                         wave_sync();
                         if (!stay) sStash[wv].get(sc + lane_rank(~sm), fill, ids);
                     }
@@ -618,7 +628,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                     }
                 } else if (block) {
                     if (!stay) q = fill;
-                    store_bin<true>(nxt, (uint32_t)(lane_bcast(blk, 0) * 64 + lane), q, ids);
+                    store_bin<true>(nxt, (uint32_t)(lane_bcast(blk, 0) + lane), q, ids);
                 } else if (nst > 0) {
                     wave_sync();
                     if (stay) sStash[wv].put(sc + lane_rank(sm), q, ids);
@@ -626,24 +636,39 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                 }
             }
             if (BINS) {
+                // the stayers left in the stashes: behind the blocks, or in the
+                // back run of a split tile
+                unsigned long long word = 0ull;
+                if (!excl && taken + sc > 0 && lane == 0)
+                    word = gatomic_add(&S.count[nbuf][tile],
+                                       (unsigned long long)taken | (unsigned long long)sc << 32);
                 flush_leavers_mx<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids, lox, loy, loz);
-                if (lane == 0) sLeft[s][wv] = sc;
-                __syncthreads();
-                // the stayers left in the stashes follow the blocks
-                int o = 64 * sBlk[s], m = o;
+                if (excl) {
+                    if (lane == 0) sLeft[s][wv] = sc;
+                    __syncthreads();
+                    int o = sBlk[s];
 #pragma unroll
-                for (int w = 0; w < kWaves; ++w) {
-                    const int r = sLeft[s][w];
-                    if (w < wv) o += r;
-                    m += r;
-                }
-                if (lane < sc) {
-                    PMx q;
-                    sStash[wv].get(lane, q, ids);
-                    store_bin<false>(nxt, (uint32_t)(o + lane), q, ids);
+                    for (int w = 0; w + 1 < kWaves; ++w) {
+                        const int r = sLeft[s][w];
+                        if (w < wv) o += r;
+                    }
+                    if (lane < sc) {
+                        PMx q;
+                        sStash[wv].get(lane, q, ids);
+                        store_bin<false>(nxt, (uint32_t)(o + lane), q, ids);
+                    }
+                } else if (taken + sc > 0) {
+                    const unsigned long long old = lane_bcast(word, 0);
+                    const int front = bin_front(old) + taken, back = bin_back(old);
+                    if (front + back + sc > cap) {
+                        if (lane == 0) gatomic_add(&I->flags[kFlagOverflow], 1ull);
+                    } else if (lane < sc) {
+                        PMx q;
+                        sStash[wv].get(lane, q, ids);
+                        store_bin<false>(nxt, (uint32_t)(cap - 1 - back - lane), q, ids);
+                    }
                 }
                 wave_sync();
-                if (tid == 0) publish_front(I, S, it, s, nbuf, tile, cnt, m, excl);
             }
             if (PUSH) {
                 keo = wave_total(keo);
@@ -656,6 +681,13 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
         }
 
         __syncthreads();
+        if (BINS && excl && tid < ns) {
+            int m = sBlk[tid];
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) m += sLeft[tid][w];
+            if (add_front<MODE == kModeBoundary>(&I->sp[tid].count[nbuf][tile], m, sMeta[tid].cap))
+                count_lanes(&I->flags[kFlagOverflow]);
+        }
         if (PUSH) write_ke<kWaves>(I, it, tid, ns, sKe);
         if (DEP) {
             unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
