@@ -27,6 +27,7 @@
 #include "ohpic_fft.hpp"
 #include "ohpic_internal.hpp"
 #include "ohpic_kernels.hpp"
+#include "ohpic_plan.hpp"
 
 using namespace ohpic;
 
@@ -250,52 +251,6 @@ int64_t max_work_items(const ohpic_config &c, int64_t ntiles, int num_cus)
 {
     if (c.chunks > 0) return ntiles * c.chunks;
     return ntiles + (int64_t)num_cus * 8;
-}
-
-// One tile of one instance as plan_chunks sees it.
-struct TileLoad {
-    int inst, tile;
-    int64_t load;  // bin slots over all species
-};
-
-// No chunk is made smaller than this many slots: it costs an E tile, a charge
-// flush (tiles of 9.4K slots in 2 chunks: 32^3 x 64 ppc mixed 124 us per launch,
-// whole 88 us).
-constexpr int64_t kMinChunkLoad = 8192;
-
-// Chunks per tile (nch[i] of tiles[i]) and the order the tiles are dispatched
-// in, for `slots` workgroups resident at once: heaviest first (in steps of an
-// eighth of an octave, tiles of one step in grid order).  A tile stays whole
-// unless it would outlast the launch: split are the tiles of a grid with less
-// than a quarter as many tiles as workgroups, so that they fill the device
-// (16^3 x 200 ppc: 169 -> 149 us mixed, 189 -> 158 us FP64; with half as many,
-// 32^3 x 300 ppc mixed, whole tiles are faster, 317 against 363 us), and tiles
-// at least twice as heavy as the mean that hold at least a workgroup's
-// fair share of the work (a density peak).  Splitting further, so that the
-// last tiles of a launch end together, costs more than it gives (80x72x88 x 20
-// ppc mixed: 317 us per launch against 280).  At most max_extra items beyond
-// one per tile.  A group is planned as one: 32 members of 16^3-64^3, each
-// split as if it ran alone (62936 items), took 3.01 ms per particle launch,
-// planned together (5472 items) 1.4 ms.
-void plan_chunks(std::vector<TileLoad> &tiles, int64_t slots, int64_t max_extra,
-                 std::vector<int> &nch)
-{
-    auto level = [](int64_t l) { return l <= 0 ? -1 : (int)std::floor(8.0 * std::log2((double)l)); };
-    std::stable_sort(tiles.begin(), tiles.end(), [&](const TileLoad &a, const TileLoad &b) {
-        return level(a.load) > level(b.load);
-    });
-    nch.assign(tiles.size(), 1);
-    if (tiles.empty()) return;
-    int64_t work = 0, extra = 0;
-    for (const TileLoad &t : tiles) work += t.load;
-    const int64_t share = work / slots, nt = (int64_t)tiles.size();
-    const int64_t unit = std::max(
-        kMinChunkLoad, 4 * nt <= slots ? share : std::max(share / 2, work / nt));
-    for (size_t i = 0; i < tiles.size(); ++i) {
-        const int64_t want = tiles[i].load / unit;
-        nch[i] = (int)std::max<int64_t>(1, std::min<int64_t>({want, 1 + max_extra - extra, 256}));
-        extra += nch[i] - 1;
-    }
 }
 
 // Device bytes ohpic_create allocates for c (plus the lazily allocated
@@ -1155,9 +1110,9 @@ int group_refresh(ohpic_group *g)
     if (tables) {
         g->ids = false;
         for (ohpic_ctx *m : g->members) g->ids = g->ids || m->cfg.track_ids != 0;
-        if (n > 0)
-            g->queue_blocks =
-                particles_queue_blocks(g->precision, g->weight_order, g->T, g->ids, g->device);
+        // (members share precision, weights and tile)
+        for (ohpic_ctx *m : g->members)
+            if ((m->cfg.track_ids != 0) == g->ids) g->queue_blocks = m->slots;
         std::vector<InstDev> insts(n);
         std::vector<FftJob> jobs(n);
         std::vector<WorkItem> items;
@@ -1648,7 +1603,7 @@ int ohpic_create(const ohpic_config *cfg, ohpic_ctx **out)
     CREATE_HIP(hipHostMalloc((void **)&ctx->h_diag, kDiagSlots * sizeof(double),
                              hipHostMallocDefault));
     ctx->slots = particles_queue_blocks(c.precision, c.weight_order, ctx->T, c.track_ids != 0,
-                                        ctx->device);
+                                        ctx->num_cus);
     CREATE_CHK(sync_upload_inst(ctx));
     CREATE_CHK(build_work_items(ctx));
     CREATE_HIP(hipStreamSynchronize(ctx->st));

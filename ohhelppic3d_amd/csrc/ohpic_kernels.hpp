@@ -56,12 +56,12 @@ hipError_t launch_cell_counts(const InstDev *insts, int inst, int s, int par, in
 // The fused step as one resident grid of `blocks` workgroups that claim the
 // nitems work items in list order from *queue (which must be 0 at launch:
 // the start of a step zeroes it).  particles_queue_blocks: workgroups of that kernel
-// resident on the whole device.
+// resident on a device of `cus` compute units.
 hipError_t launch_particles_queue(int precision, int weight_order, const int T[3], bool ids,
                                   const InstDev *insts, const WorkItem *items, int nitems,
                                   const int *parity, unsigned int *queue, int blocks,
                                   hipStream_t st);
-int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int device);
+int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int cus);
 
 // mixed-precision particles (ohpic_particles_mixed.hip)
 hipError_t launch_particles_mixed(int mode, int weight_order, const int T[3], bool ids,

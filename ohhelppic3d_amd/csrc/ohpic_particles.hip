@@ -802,14 +802,8 @@ hipError_t launch_particles_queue(int precision, int weight_order, const int T[3
     return hipErrorInvalidValue;
 }
 
-int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int device)
+int particles_queue_blocks(int precision, int weight_order, const int T[3], bool ids, int cus)
 {
-    int cus = 256;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess)
-        cus = prop.multiProcessorCount;
-    else
-        (void)hipGetLastError();
     int per = 1;
     if (precision == 1) {
         per = particles_mixed_queue_blocks(weight_order, T, ids);
