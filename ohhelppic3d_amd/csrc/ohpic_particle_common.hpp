@@ -240,10 +240,11 @@ __device__ __forceinline__ void load_meta(SpecMeta *meta, const InstDev *__restr
 // bin's word when the species is done.  (Taken from the word itself, which all
 // arrivals add to, with the words of 15 other tiles in its cache line: 16^3 x
 // 1000 ppc, 12 items per tile, 1285 us per step FP64 and 1465 mixed, against
-// 1035 and 1147.  Items with parts of the front run of their own and a launch
-// to join them: 1077 and 1186.)  The answer is waited for here: pending in the
-// register that a whole tile's answer from LDS takes, it made every tile wait
-// for its loads ahead too (96^3 x 32 ppc FP64 1105 -> 1120 us per launch).
+// 1017 and 1086.  Items with parts of the front run of their own and a launch
+// to join them: 1080 and 1188.)  It is called, and its answer waited for, where
+// only split tiles come: an answer pending in a register that whole tiles share
+// makes them wait for their loads ahead and their stores as well (96^3 x 32 ppc
+// FP64 1105 -> 1120 us per launch, 128^3 x 8 mixed in 4^3 tiles 546 -> 582).
 __device__ __forceinline__ int claim_block(const InstDev *__restrict__ I, const WorkItem &it, int s)
 {
     int32_t *p = &I->claims[(int64_t)(it.slot - it.chunk) * kMaxSpecies + s];

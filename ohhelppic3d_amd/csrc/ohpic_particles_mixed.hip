@@ -555,8 +555,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                     block = holes <= sc;
                     if (block) {
                         // both arrive while the charge is deposited
-                        if (lane == 0)
-                            blk = excl ? atomicAdd(&sBlk[s], 64) : claim_block(I, it, s);
+                        if (excl && lane == 0) blk = atomicAdd(&sBlk[s], 64);
                         sc -= holes;
                         taken += 64;
                         wave_sync();
@@ -628,6 +627,7 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                     }
                 } else if (block) {
                     if (!stay) q = fill;
+                    if (!excl && lane == 0) blk = claim_block(I, it, s);
                     store_bin<true>(nxt, (uint32_t)(lane_bcast(blk, 0) + lane), q, ids);
                 } else if (nst > 0) {
                     wave_sync();
@@ -636,29 +636,32 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
                 }
             }
             if (BINS) {
+                flush_leavers_mx<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids, lox, loy, loz);
                 // the stayers left in the stashes: behind the blocks, or in the
                 // back run of a split tile
-                unsigned long long word = 0ull;
-                if (!excl && taken + sc > 0 && lane == 0)
-                    word = gatomic_add(&S.count[nbuf][tile],
-                                       (unsigned long long)taken | (unsigned long long)sc << 32);
-                flush_leavers_mx<TX, TY, TZ, IDS>(sLeave[wv], lc, I, S, nbuf, ids, lox, loy, loz);
                 if (excl) {
                     if (lane == 0) sLeft[s][wv] = sc;
                     __syncthreads();
-                    int o = sBlk[s];
+                    int o = sBlk[s], m = o;
 #pragma unroll
-                    for (int w = 0; w + 1 < kWaves; ++w) {
+                    for (int w = 0; w < kWaves; ++w) {
                         const int r = sLeft[s][w];
                         if (w < wv) o += r;
+                        m += r;
                     }
                     if (lane < sc) {
                         PMx q;
                         sStash[wv].get(lane, q, ids);
                         store_bin<false>(nxt, (uint32_t)(o + lane), q, ids);
                     }
+                    if (tid == 0 && add_front<MODE == kModeBoundary>(&S.count[nbuf][tile], m, cap))
+                        count_lanes(&I->flags[kFlagOverflow]);
                 } else if (taken + sc > 0) {
-                    const unsigned long long old = lane_bcast(word, 0);
+                    unsigned long long old = 0ull;
+                    if (lane == 0)
+                        old = gatomic_add(&S.count[nbuf][tile],
+                                          (unsigned long long)taken | (unsigned long long)sc << 32);
+                    old = lane_bcast(old, 0);
                     const int front = bin_front(old) + taken, back = bin_back(old);
                     if (front + back + sc > cap) {
                         if (lane == 0) gatomic_add(&I->flags[kFlagOverflow], 1ull);
@@ -681,13 +684,6 @@ __global__ void __launch_bounds__(mx_block(TX *TY *TZ))
         }
 
         __syncthreads();
-        if (BINS && excl && tid < ns) {
-            int m = sBlk[tid];
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) m += sLeft[tid][w];
-            if (add_front<MODE == kModeBoundary>(&I->sp[tid].count[nbuf][tile], m, sMeta[tid].cap))
-                count_lanes(&I->flags[kFlagOverflow]);
-        }
         if (PUSH) write_ke<kWaves>(I, it, tid, ns, sKe);
         if (DEP) {
             unsigned long long *__restrict__ racc = I->rho_acc[acc_buf];
