@@ -131,7 +131,7 @@ __device__ __forceinline__ unsigned long long lane_bcast(unsigned long long v, i
 
 // Particle state streams through each step once, so its full-line accesses
 // carry the non-temporal hint: 256^3 x 32 ppc mixed 11.82 -> 10.91 ms per
-// launch, 256^3 x 16 FP64 11.14 -> 10.85 ms, and the field kernels of smaller
+// launch, 256^3 x 16 FP64 11.14 -> 10.42 ms, and the field kernels of smaller
 // grids find their arrays in the last-level cache (the 32^3 x 16 push loses
 // 1 us, its field solve gains 1.5 us).  Partial lines (leavers, the ends of
 // runs) are stored without it: they are merged in L2.

@@ -17,15 +17,16 @@
 // The LDS charge block is flushed with one global 64-bit atomic per node.
 // Integer accumulation makes rho independent of particle order and timing.
 //
-// What bounds it: large grids stream 96 B per particle, at 4.75 TB/s of the 5.2
-// TB/s a bare copy of the same shape reaches; the rest is per tile (E tile,
-// charge flush, the leavers' atomics).  Small grids wait: so every load of an
-// item's start is issued before the first is used, nothing in the particle
-// loop waits for a store, a block's number or the stash, and a species ends
-// with one barrier.  Against slots from an LDS counter at any alignment, a
-// store wait per iteration and the wrap and tile index of every particle:
-// 256^3 x 16 ppc 12.16 -> 11.14 ms, 96^3 x 32 1.35 -> 1.19 ms, 32^3 x 16 51 ->
-// 40 us per launch (HIP events, one box).
+// What bounds it: large grids stream 96 B per particle, at 6.1 TB/s or 0.76 of
+// the 8 TB/s peak (256^3 x 64 ppc, 33.9 ms per launch); the rest is per tile (E
+// tile, charge flush, the leavers' atomics).  Small grids wait: so every load
+// of an item's start is issued before the first is used, nothing in a whole
+// tile's particle loop waits for a store, a block's number or the stash, and a
+// species ends with one barrier.  Against slots from an LDS counter at any
+// alignment, a store wait per iteration and the wrap and tile index of every
+// particle: 256^3 x 16 ppc 12.16 -> 9.3-10.4 ms (the same build differs that
+// much between runs), 96^3 x 32 1.35 -> 1.11 ms, 32^3 x 16 51 -> 38 us per
+// launch.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

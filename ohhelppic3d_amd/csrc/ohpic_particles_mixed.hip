@@ -20,9 +20,9 @@
 // 22 LDS per particle) with their latencies.  So the wrap and the new tile are
 // found only for particles that leave, when their buffer is routed; the E
 // gather reads its eight nodes before it uses one; and no iteration waits for
-// its own stores.  With the aligned blocks of the front run: 256^3 x 32 ppc
-// 12.62 -> 11.82 ms, 128^3 x 64 with a density peak 3.93 -> 3.21 ms, 64^3 x 32
-// 313 -> 249 us per launch (HIP events, one box).
+// its own stores.  With that, the aligned blocks of the front run and the
+// larger workgroups below: 256^3 x 32 ppc 12.62 -> 10.4 ms, 128^3 x 64 with a
+// density peak 3.93 -> 2.75 ms, 64^3 x 32 313 -> 219 us per launch.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
