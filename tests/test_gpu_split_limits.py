@@ -89,3 +89,22 @@ def test_most_particles_leave(ohp, precision, tile, chunks):
         b.step(3)
         assert a.diagnostics()["repacks"] == 0
         same(ohp, a, b)
+
+
+@pytest.mark.parametrize("precision", PREC)
+@pytest.mark.parametrize("chunks", [1, 3])
+def test_boundary_operator_overflow(ohp, precision, chunks):
+    sp = free(60000, 8, speed=0.5, wave=12.0)
+    with make(ohp, sp, precision, tile=(4, 4, 4), chunks=chunks, slack=0.01) as a, \
+            make(ohp, sp, precision, tile=(4, 4, 4), chunks=1, slack=12.0) as b:
+        for _ in range(6):
+            a.deposit()
+            a.field_solve()
+            a.gather_push()
+            a.boundary()
+        assert a.diagnostics()["repacks"] > 0
+        b.step(6)
+        for s in range(2):
+            p, q = (by_pid(m.store_particles(s, True)) for m in (a, b))
+            assert all(np.array_equal(p[k], q[k]) for k in q), s
+        assert np.array_equal(a.cell_counts(), b.cell_counts())
